@@ -46,6 +46,37 @@ constexpr int kChunkGrain = 64;    // source chunks of the ordered kernel: multi
 
 void launch_pair(const PairArgs& a, hipStream_t s);
 
+struct SymSys;
+// Small systems (wide_kernels.hip): kWideTargets targets per unit of work, a
+// wave (split 1) or a workgroup (split 4) per unit, sources across the lanes.
+constexpr int kWideTargets = 4;
+struct WideItem {
+  int32_t sys;
+  int32_t tgt;  // first target within the system
+};
+struct WideArgs {
+  int kind;     // 0 open RPY, 1 bottom wall, 2 per system
+  int fp32;     // 1: FP32 pair terms and per-lane sums, FP64 across lanes
+  int blocks;   // BlockBits mask
+  int split;    // 1 or 4
+  const void* pos;  // float4 / double4 records
+  const double* F;  // 3N AoS (nullptr when absent)
+  const double* T;
+  double* U;  // 3N, overwritten
+  double* W;  // 3N (nullptr without angular velocities)
+  // units: items[0 .. nunits) into the table `sys`, or (items nullptr) equal
+  // systems of ns particles with per_sys units each
+  const WideItem* items;
+  const SymSys* sys;
+  int nunits;
+  int per_sys;
+  int64_t ns;
+  const int* active;  // per-system flags; units of systems with 0 are skipped (nullptr: all)
+  const int* stop;    // as PairArgs::stop
+  double t0, rt0, r0;
+};
+void launch_pair_wide(const WideArgs& a, hipStream_t s);
+
 // Translational product with several force vectors in one pass over the pairs:
 // U_r = t0 * M F_r, r < nrhs.  F holds nrhs consecutive 3N vectors; the
 // partial of vector r and chunk c goes to U + (r * nch + c) * n3.

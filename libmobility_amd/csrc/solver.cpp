@@ -364,12 +364,14 @@ void NBodySolver::sym_shape(bool special, int tpl_req, int nch_req, int& tpl, in
   if (hmax > 0) nch = std::max(nch, 1);
 }
 
-bool NBodySolver::use_sym(int blocks) const {
+bool NBodySolver::use_sym(int blocks) {
   if (sym_mode_ == 0 || N_ <= 0) return false;
   if (blocks != kUF && blocks != (kUF | kWF) && blocks != (kUT | kWT) &&
       blocks != (kUF | kUT | kWT | kWF))
     return false;
-  return sym_mode_ == 1 || N_ >= kSymAutoN;
+  if (sym_mode_ == 1) return true;
+  return N_ >= kSymAutoN &&
+         (keep_order_ || numSystems() == 1 || mean_system_size() > kSymAutoMean);
 }
 
 // Items: per pass, for every system and tile, the system's chunks of the
@@ -620,6 +622,99 @@ void NBodySolver::launch_sym(int blocks, bool fp32, const void* rec, const doubl
   run_sym(tpl, nch, h, blocks, fp32, rec, F, T, U, W);
 }
 
+double NBodySolver::mean_system_size() {
+  if (mean_size_struct_ != struct_id_ || mean_size_N_ != N_) {
+    double s2 = 0.0;
+    for (size_t s = 0; s + 1 < sys_off_host_.size(); ++s) {
+      const double n = (double)(sys_off_host_[s + 1] - sys_off_host_[s]);
+      s2 += n * n;
+    }
+    mean_size_ = N_ > 0 ? s2 / (double)N_ : 0.0;
+    mean_size_struct_ = struct_id_;
+    mean_size_N_ = N_;
+  }
+  return mean_size_;
+}
+
+// Not where the caller chose a decomposition (tiling, algorithm, launch mode).
+bool NBodySolver::use_wide() {
+  return !keep_order_ && tile_tpl_ == 0 && tile_nch_ == 0 && algorithm_ != kNaive && algorithm_ != kBlock &&
+         persistent_mode_ == -1 && mean_system_size() <= kWideMaxSize;
+}
+
+// Units of kWideTargets targets of one system.  Equal systems of one kind need
+// no list; else the systems with the most work per unit come first.
+void NBodySolver::ensure_wide_plan() {
+  if (wide_.N == N_ && wide_.structure == struct_id_) return;
+  constexpr int targets = kWideTargets;
+  const int nsys = (int)sys_off_host_.size() - 1;
+  const int64_t n0 = sys_off_host_[1] - sys_off_host_[0];
+  bool equal = kind_code() != 2;
+  for (int s = 1; s < nsys && equal; ++s)
+    equal = sys_off_host_[s + 1] - sys_off_host_[s] == n0;
+  wide_.N = -1;
+  if (equal) {
+    wide_.per_sys = (int)((n0 + targets - 1) / targets);
+    wide_.nunits = wide_.per_sys * nsys;
+    wide_.ns = n0;
+  } else {
+    std::vector<SymSys> systems(nsys);
+    std::vector<int> order(nsys);
+    for (int s = 0; s < nsys; ++s) {
+      SymSys& S = systems[s];
+      S.off = sys_off_host_[s];
+      S.n = (int32_t)(sys_off_host_[s + 1] - sys_off_host_[s]);
+      S.ntiles = S.hmax = 0;
+      S.wall = s < (int)sys_kind_host_.size() ? sys_kind_host_[s] : (wall_ ? 1 : 0);
+      order[s] = s;
+    }
+    std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
+      return (double)systems[x].n * (systems[x].wall ? 5.0 : 1.0) >
+             (double)systems[y].n * (systems[y].wall ? 5.0 : 1.0);
+    });
+    std::vector<WideItem> items;
+    for (int s : order)
+      for (int32_t t = 0; t < systems[s].n; t += targets) items.push_back(WideItem{s, t});
+    wide_.items.reserve(sizeof(WideItem) * std::max<size_t>(items.size(), 1));
+    wide_.sys.reserve(sizeof(SymSys) * systems.size());
+    LM_HIP(hipMemcpyAsync(wide_.items.as<void>(), items.data(), sizeof(WideItem) * items.size(),
+                          hipMemcpyHostToDevice, stream_));
+    LM_HIP(hipMemcpyAsync(wide_.sys.as<void>(), systems.data(), sizeof(SymSys) * systems.size(),
+                          hipMemcpyHostToDevice, stream_));
+    LM_HIP(hipStreamSynchronize(stream_));  // the host vectors go out of scope
+    wide_.nunits = (int)items.size();
+  }
+  wide_.listed = !equal;
+  wide_.structure = struct_id_;
+  wide_.N = N_;
+}
+
+void NBodySolver::launch_wide(int blocks, bool fp32, const void* rec, const double* F,
+                              const double* T, double* U, double* W) {
+  ensure_wide_plan();
+  WideArgs a{};
+  a.kind = kind_code();
+  a.fp32 = fp32 ? 1 : 0;
+  a.blocks = blocks;
+  a.split = wide_.nunits >= kWideWaveUnits && mean_system_size() <= kWideWaveMean ? 1 : 4;
+  a.pos = rec;
+  a.F = F;
+  a.T = (blocks & (kUT | kWT)) ? T : nullptr;
+  a.U = U;
+  a.W = (blocks & (kWT | kWF)) ? W : nullptr;
+  a.items = wide_.listed ? wide_.items.as<WideItem>() : nullptr;
+  a.sys = wide_.listed ? wide_.sys.as<SymSys>() : nullptr;
+  a.nunits = wide_.nunits;
+  a.per_sys = wide_.per_sys;
+  a.ns = wide_.ns;
+  a.active = pair_active_;
+  a.stop = pair_stop_;
+  a.t0 = t0_;
+  a.rt0 = rt0_;
+  a.r0 = r0_;
+  launch_pair_wide(a, stream_);
+}
+
 void NBodySolver::setPairTiling(int tpl, int nch) {
   if (tpl != 0 && tpl != 1 && tpl != 2 && tpl != 4)
     throw Error("[libmobility_amd] targets per lane must be 0 (auto), 1, 2 or 4");
@@ -833,10 +928,14 @@ void NBodySolver::pair_product(const void* rec64, const void* rec32, const doubl
   const bool fp32 = (prec < 0 ? pair_prec_ : prec) == kPairFP32;
   const void* rec = fp32 ? rec32 : rec64;
   last_sym_ = false;
+  last_wide_ = false;
   deferred_nch_ = 0;
   if (use_sym(blocks)) {
     launch_sym(blocks, fp32, rec, F, T, U, W);
     last_sym_ = true;
+  } else if (use_wide()) {
+    launch_wide(blocks, fp32, rec, F, T, U, W);
+    last_wide_ = true;
   } else if (seg_items_.count > 0) {
     // per-system Lanczos after some systems converged: their work is dropped
     launch_pair_items(seg_items_.buf.as<PairItem>(), seg_items_.count, seg_items_.tpl,
@@ -1188,6 +1287,11 @@ void NBodySolver::lanczos_product(const double* v, double* w) {
                  angular_ ? u + N3 : nullptr);
     pre_back(u, w, n);
   } else {
+    struct OrderGuard {
+      bool& f;
+      ~OrderGuard() { f = false; }
+    } guard{keep_order_};
+    keep_order_ = any_open_;
     pair_product(rec64_.as<void>(), rec32_.as<void>(), v, angular_ ? v + N3 : nullptr, w,
                  angular_ ? w + N3 : nullptr);
   }

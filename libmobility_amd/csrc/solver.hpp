@@ -99,10 +99,11 @@ class NBodySolver {
   // Pair-kernel tiling: targets per lane (1, 2, 4) and source chunks; 0 = auto.
   void setPairTiling(int tpl, int nch);
   void setAutotune(bool on) { autotune_ = on; }
-  // The symmetric path reports its targets per lane and offset chunks.
+  // The symmetric path reports its targets per lane and offset chunks, the
+  // wide kernel its targets per unit of work and one chunk.
   void lastPairTiling(int* tpl, int* nch) const {
-    *tpl = last_sym_ ? sym_.tpl : items_tpl_;
-    *nch = last_sym_ ? sym_.nchunks : items_nch_;
+    *tpl = last_sym_ ? sym_.tpl : (last_wide_ ? kWideTargets : items_tpl_);
+    *nch = last_sym_ ? sym_.nchunks : (last_wide_ ? 1 : items_nch_);
   }
   // Symmetric evaluation of one open or single-wall system, any block set
   // (-1 auto: from N = kSymAutoN; 0 off; 1 on).
@@ -110,7 +111,24 @@ class NBodySolver {
   // Particles (in total) from which the automatic mode evaluates each
   // unordered pair once: from 16384 it was 1.10-1.37x faster than the ordered
   // evaluation (open UF and wall 6x6, FP32 and FP64); at 8192 equal or slower.
+  // Ensembles also need a mean system size (of the system that the average
+  // particle is in) above kSymAutoMean: 60000 particles in systems of 1500
+  // take 58-555 us with sources across the lanes and 60-590 us symmetric; in
+  // systems of 800, 36-304 us and 60-580 us; of 3000, 106-1100 us and 100-1070 us.
   static constexpr int64_t kSymAutoN = 16384;
+  static constexpr double kSymAutoMean = 2048;
+  // Mean system size up to which the ordered evaluation puts sources across
+  // the lanes (wide_kernels.hip has both sides' times; equal from about 8000).
+  static constexpr double kWideMaxSize = 8192;
+  // Units of work from which each is one wave instead of a workgroup of four
+  // (which then only adds the waves' sums and a barrier): 20000 particles in
+  // systems of 256, open UF FP64, take 11.1 us with one wave per unit and 14.8
+  // with four, wall 6x6 38.7 and 47.9.  Below, four waves per unit fill the
+  // chip: 2000 particles in systems of 256 take 4.5 and 3.5 us, 10.7 and 7.1.
+  // From a mean size of kWideWaveMean a unit's wave is too long a tail (60000
+  // in systems of 3000, wall 6x6 FP32: 635 and 598 us).
+  static constexpr int kWideWaveUnits = 2048;
+  static constexpr double kWideWaveMean = 2048;
   // Memory for the symmetric path's partial sums (0: the default, 4 GiB);
   // ring offsets are split into passes that fit it.
   void setPairSymmetricMemory(int64_t bytes);
@@ -354,13 +372,42 @@ class NBodySolver {
   std::map<std::tuple<int64_t, int, int, int>, std::pair<int, int>> sym_tuned_;
   void sym_shape(bool special, int tpl_req, int nch_req, int& tpl, int& nch, int& ntiles,
                  int& hmax) const;
-  bool use_sym(int blocks) const;
+  bool use_sym(int blocks);
   void ensure_sym_plan(int tpl, int nch, int h, bool ang);
   void build_sym_active(const int* act);
   void run_sym(int tpl, int nch, int h, int blocks, bool fp32, const void* rec, const double* F,
                const double* T, double* U, double* W);
   void launch_sym(int blocks, bool fp32, const void* rec, const double* F, const double* T,
                   double* U, double* W);
+  // sources across the lanes (wide_kernels.hip), for small systems
+  struct WidePlan {
+    DevBuf items, sys;  // only for systems of different sizes or kinds
+    int nunits = 0, per_sys = 0;
+    int64_t ns = 0, N = -1;
+    uint64_t structure = 0;
+    bool listed = false;
+  };
+  WidePlan wide_;
+  bool last_wide_ = false;
+  // size of the system that the average particle is in, of the current structure
+  double mean_system_size();
+  double mean_size_ = 0.0;
+  uint64_t mean_size_struct_ = 0;
+  int64_t mean_size_N_ = -1;
+  bool use_wide();
+  // Products of a plain Lanczos recurrence over open systems: the summation
+  // order stays that of k_pair's chunks (k_pair_sym from kSymAutoN).  There the
+  // largest Ritz values converge to rounding within about 15 iterations, the
+  // recurrence loses its orthogonality, and from then on a change in the last
+  // bit grows some 200 times per iteration: at a tolerance of 1e-4 another
+  // order moved the results of a seed by 1e-6 to 9e-4 (1000-6000 particles,
+  // volume fractions 0.05-0.25) and the stop by up to 5 iterations, without
+  // being nearer to M^{1/2} W.  Above a wall and with the preconditioner the
+  // same comparison gives 1e-15 to 1e-13 (FP64) and 1e-7 to 1e-6 (FP32).
+  bool keep_order_ = false;
+  void ensure_wide_plan();
+  void launch_wide(int blocks, bool fp32, const void* rec, const double* F, const double* T,
+                   double* U, double* W);
   std::map<std::tuple<int, int, int>, std::vector<PairItem>> host_items_;
   uint64_t host_items_struct_ = 0;
   int64_t host_items_N_ = -1;

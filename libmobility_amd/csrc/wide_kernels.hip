@@ -1,0 +1,295 @@
+// The product of small systems: sources across the lanes.
+//
+// k_pair (nbody_kernels.hip) puts 256 targets into a workgroup's lanes, so a
+// system of 1000 particles fills 4 workgroups, has to be cut into source
+// chunks whose partial sums a second kernel adds, and each chunk is a serial
+// chain of 64 to 256 pairs behind one LDS tile.  Here a wave holds 64 sources
+// in its lanes and meets T targets, whose records it reads through the scalar
+// cache; each lane sums its own sources' contributions to the T targets, and
+// the wave adds its lanes at the end (lane swaps, then rotations inside the
+// rows of 16, a fixed order).  With SPLIT waves per group of T targets (SPLIT
+// 4: the whole workgroup) the waves take every SPLIT-th group of 64 sources
+// and meet in LDS, added in wave order.  There are N / T units of work instead
+// of N / 256, no partial sums in memory and no second launch.
+//
+// Bound by latency below about 500 particles (2.8-3.5 us: launch, one load of
+// the sources, the lane sums) and by VALU issue above.  T = 4: the fold costs
+// about 100 instructions per wave against 100 (open) to 770 (wall 6x6) per
+// group of 64 sources; T = 8 was 1.2-1.8x slower for 6x6 blocks (196-227
+// VGPRs, 2 waves per SIMD) and within 7 % for the translational block.
+// Microseconds per product, k_pair + k_chunk_reduce against this kernel:
+//   particles          96           512          1024         2000        4096        8192
+//   open UF FP64   11.0 / 3.0   13.0 / 3.5   15.0 / 4.6   19.7 / 8.5   33 / 22.5    81 / 74
+//   open UF FP32    9.3 / 2.8   11.3 / 3.3   13.2 / 4.2   17.7 / 6.5   25 / 15.3    55 / 44
+//   wall 6x6 FP64  40.8 / 4.8   44.4 / 7.1   48.5 / 11.4  61.3 / 31.3  126 / 105   411 / 406
+//   wall 6x6 FP32  36.4 / 4.5   39.9 / 6.4   43.8 / 9.9   54.2 / 22.2   95 / 66    242 / 229
+#include <type_traits>
+
+#include "kernels.hpp"
+#include "lm_common.hpp"
+#include "pair_device.hpp"
+#include "pair_math.hpp"
+
+namespace lm {
+
+namespace {
+
+constexpr int kWideWaves = kPairThreads / 64;
+
+// a' = {a's lanes 0-31, b's lanes 0-31}, b' = {a's lanes 32-63, b's 32-63};
+// returns a' + b': lane l < 32 holds a(l) + a(l + 32), lane l >= 32 the same of b.
+__device__ inline double fold32(double a, double b) {
+  const uint64_t x = __builtin_bit_cast(uint64_t, a), y = __builtin_bit_cast(uint64_t, b);
+  const auto lo = __builtin_amdgcn_permlane32_swap((uint32_t)x, (uint32_t)y, false, false);
+  const auto hi =
+      __builtin_amdgcn_permlane32_swap((uint32_t)(x >> 32), (uint32_t)(y >> 32), false, false);
+  return __builtin_bit_cast(double, ((uint64_t)hi[0] << 32) | lo[0]) +
+         __builtin_bit_cast(double, ((uint64_t)hi[1] << 32) | lo[1]);
+}
+// The same between the even and the odd rows of 16 lanes: even rows hold a's
+// sums, odd rows b's.
+__device__ inline double fold16(double a, double b) {
+  const uint64_t x = __builtin_bit_cast(uint64_t, a), y = __builtin_bit_cast(uint64_t, b);
+  const auto lo = __builtin_amdgcn_permlane16_swap((uint32_t)x, (uint32_t)y, false, false);
+  const auto hi =
+      __builtin_amdgcn_permlane16_swap((uint32_t)(x >> 32), (uint32_t)(y >> 32), false, false);
+  return __builtin_bit_cast(double, ((uint64_t)hi[0] << 32) | lo[0]) +
+         __builtin_bit_cast(double, ((uint64_t)hi[1] << 32) | lo[1]);
+}
+// Every lane gets v of the lane N places on in its row of 16 (cyclic).
+template <int N>
+__device__ inline double row_ror(double v) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, 0x120 + N, 0xf,
+                                                            0xf, true);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32),
+                                                            0x120 + N, 0xf, 0xf, true);
+  return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+__device__ inline double row_sum(double v) {
+  v += row_ror<8>(v);
+  v += row_ror<4>(v);
+  v += row_ror<2>(v);
+  return v + row_ror<1>(v);
+}
+
+// Sums NV values over the 64 lanes: v[q], q < NV / 4, of row r (lanes 16r ..
+// 16r + 15) becomes the sum of value (r / 2) NV/2 + (r mod 2) NV/4 + q.
+template <int NV>
+__device__ inline void wave_fold(double* v) {
+#pragma unroll
+  for (int q = 0; q < NV / 2; ++q) v[q] = fold32(v[q], v[q + NV / 2]);
+#pragma unroll
+  for (int q = 0; q < NV / 4; ++q) v[q] = row_sum(fold16(v[q], v[q + NV / 4]));
+}
+
+// The sums of T targets over the sources base, base + 64 * stride, ... < src1
+// (64 at a time, one per lane), left in v (T times U, then T times W) per lane.
+template <class R, bool WALL, int BLK, int T>
+__device__ inline void wide_sources(const typename Rec<R>::T* __restrict__ pos,
+                                    const double* __restrict__ F, const double* __restrict__ Tq,
+                                    int64_t tgt0, int ntgt, int64_t base, int64_t src1, int stride,
+                                    double t0, double rt0, double r0, double* v) {
+  using R4 = typename Rec<R>::T;
+  constexpr bool kNeedF = (BLK & (kUF | kWF)) != 0;
+  constexpr bool kNeedT = (BLK & (kUT | kWT)) != 0;
+  constexpr bool kAngular = (BLK & (kWT | kWF)) != 0;
+  constexpr bool kUF34 = !WALL && BLK == kUF;  // coefficients times 4/3 (rpy_far_uf34)
+  constexpr int G = T < 4 ? T : 4;             // pairs per overlap test
+  const int lane = threadIdx.x & 63;
+  R4 pi[T];  // uniform: scalar loads
+#pragma unroll
+  for (int t = 0; t < T; ++t) pi[t] = pos[tgt0 + (t < ntgt ? t : ntgt - 1)];
+  PairAcc<R> acc[T];
+#pragma unroll
+  for (int t = 0; t < T; ++t) acc_zero(acc[t]);
+  for (; base < src1; base += 64 * (int64_t)stride) {
+    const int64_t j = base + lane;
+    R4 pj = far_record<R4>();
+    Vec3<R> fj = {R(0), R(0), R(0)}, tj = {R(0), R(0), R(0)};
+    if (j < src1) {
+      pj = pos[j];
+      if (kNeedF) fj = {R(F[3 * j]), R(F[3 * j + 1]), R(F[3 * j + 2])};
+      if (kNeedT) tj = {R(Tq[3 * j]), R(Tq[3 * j + 1]), R(Tq[3 * j + 2])};
+    }
+    if constexpr (WALL) {
+#pragma unroll
+      for (int t = 0; t < T; ++t)
+        wall_pair<R, BLK>(pi[t].x, pi[t].y, pi[t].z, pi[t].w, pj.x, pj.y, pj.z, pj.w, fj.x, fj.y,
+                          fj.z, tj.x, tj.y, tj.z, acc[t]);
+    } else {
+#pragma unroll
+      for (int g = 0; g < T; g += G) {
+        R dx[G], dy[G], dz[G], r2[G], ir[G];
+        RpyCoef<R> cf[G];
+        NearTestCmp<R> near;
+#pragma unroll
+        for (int t = 0; t < G; ++t) {
+          dx[t] = pi[g + t].x - pj.x;
+          dy[t] = pi[g + t].y - pj.y;
+          dz[t] = pi[g + t].z - pj.z;
+          r2[t] = dx[t] * dx[t] + dy[t] * dy[t] + dz[t] * dz[t];
+          ir[t] = lm_rsqrt(r2[t]);
+          cf[t] = RpyCoef<R>{};
+          if constexpr (kUF34)
+            rpy_far_uf34<R>(ir[t], cf[t]);
+          else
+            rpy_far<R, BLK>(ir[t], cf[t]);
+          near.add(r2[t]);
+        }
+        if (__builtin_expect(near.hit(), 0)) {
+          lm_rare_path();
+#pragma unroll
+          for (int t = 0; t < G; ++t) {
+            if constexpr (kUF34)
+              rpy_near_select_uf34<R>(r2[t], ir[t], cf[t]);
+            else
+              rpy_near_select<R, BLK>(r2[t], ir[t], cf[t]);
+          }
+        }
+#pragma unroll
+        for (int t = 0; t < G; ++t)
+          open_accumulate<R, BLK>(dx[t], dy[t], dz[t], fj.x, fj.y, fj.z, tj.x, tj.y, tj.z, cf[t],
+                                  acc[g + t]);
+      }
+    }
+  }
+  const double tuf = kUF34 ? 0.75 * t0 : t0;
+#pragma unroll
+  for (int t = 0; t < T; ++t) {
+    v[3 * t + 0] = tuf * (double)acc[t].uf.x + rt0 * (double)acc[t].ut.x;
+    v[3 * t + 1] = tuf * (double)acc[t].uf.y + rt0 * (double)acc[t].ut.y;
+    v[3 * t + 2] = tuf * (double)acc[t].uf.z + rt0 * (double)acc[t].ut.z;
+    if constexpr (kAngular) {
+      v[3 * T + 3 * t + 0] = r0 * (double)acc[t].wt.x + rt0 * (double)acc[t].wf.x;
+      v[3 * T + 3 * t + 1] = r0 * (double)acc[t].wt.y + rt0 * (double)acc[t].wf.y;
+      v[3 * T + 3 * t + 2] = r0 * (double)acc[t].wt.z + rt0 * (double)acc[t].wf.z;
+    }
+  }
+}
+
+}  // namespace
+
+// Unit of work u: T targets of one system, from the list `items` or, for
+// equal systems, by its number.  SPLIT 4: one unit per workgroup; SPLIT 1: one
+// per wave.
+template <class R, int KIND, int BLK, int T, int SPLIT>
+__global__ __launch_bounds__(kPairThreads) void k_pair_wide(WideArgs a) {
+  using R4 = typename Rec<R>::T;
+  constexpr bool kAngular = (BLK & (kWT | kWF)) != 0;
+  constexpr int NV = (kAngular ? 6 : 3) * T;
+  static_assert(NV % 4 == 0, "the lane fold needs a multiple of 4 values");
+  __shared__ double s_red[kWideWaves][NV];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (a.stop != nullptr) {
+    // one read per workgroup, so that all its threads take the same branch
+    __shared__ int s_stop;
+    if (threadIdx.x == 0) s_stop = *(volatile const int*)a.stop;
+    __syncthreads();
+    if (s_stop != 0) return;
+  }
+  const int unit = SPLIT == 1 ? (int)blockIdx.x * kWideWaves + wave : (int)blockIdx.x;
+  bool live = unit < a.nunits;
+  int64_t tgt0 = 0, src0 = 0, src1 = 0;
+  int ntgt = 1, kind = KIND;
+  if (live) {
+    int sys;
+    if (a.items != nullptr) {
+      const WideItem it = a.items[unit];
+      const SymSys S = a.sys[it.sys];
+      sys = it.sys;
+      src0 = S.off;
+      src1 = S.off + S.n;
+      tgt0 = S.off + it.tgt;
+      kind = S.wall;
+    } else {
+      sys = unit / a.per_sys;
+      src0 = (int64_t)sys * a.ns;
+      src1 = src0 + a.ns;
+      tgt0 = src0 + (int64_t)(unit - sys * a.per_sys) * T;
+    }
+    ntgt = (int)min((int64_t)T, src1 - tgt0);
+    if (a.active != nullptr && a.active[sys] == 0) live = false;  // system already converged
+  }
+  if (SPLIT != 1 && !live) return;  // the whole workgroup
+  double v[NV];
+  if (live) {
+    const R4* pos = static_cast<const R4*>(a.pos);
+    const int64_t base = src0 + (SPLIT == 1 ? 0 : 64 * wave);
+    if (KIND == 2 ? kind != 0 : KIND == 1)
+      wide_sources<R, KIND != 0, BLK, T>(pos, a.F, a.T, tgt0, ntgt, base, src1, SPLIT, a.t0, a.rt0,
+                                         a.r0, v);
+    else
+      wide_sources<R, KIND == 1, BLK, T>(pos, a.F, a.T, tgt0, ntgt, base, src1, SPLIT, a.t0, a.rt0,
+                                         a.r0, v);
+    wave_fold<NV>(v);
+    if ((lane & 15) == 0) {
+      const int row = lane >> 4;
+      double* red = &s_red[wave][(row >> 1) * (NV / 2) + (row & 1) * (NV / 4)];
+#pragma unroll
+      for (int q = 0; q < NV / 4; ++q) red[q] = v[q];
+    }
+  }
+  __syncthreads();
+  if (!live) return;
+  // value q of the unit: component q of its targets' U, then of their W
+  const int q = SPLIT == 1 ? lane : (int)threadIdx.x;
+  if (q < NV) {
+    double s;
+    if (SPLIT == 1) {
+      s = s_red[wave][q];
+    } else {
+      s = s_red[0][q];
+#pragma unroll
+      for (int w = 1; w < kWideWaves; ++w) s += s_red[w][q];
+    }
+    const int e = q < 3 * T ? q : q - 3 * T;
+    if (e < 3 * ntgt) (q < 3 * T ? a.U : a.W)[3 * tgt0 + e] = s;
+  }
+}
+
+template <class R, int KIND, int BLK>
+static void launch_wide_split(const WideArgs& a, hipStream_t s) {
+  if (a.split == 4)
+    hipLaunchKernelGGL((k_pair_wide<R, KIND, BLK, kWideTargets, 4>), dim3((unsigned)a.nunits),
+                       dim3(kPairThreads), 0, s, a);
+  else if (a.split == 1)
+    hipLaunchKernelGGL((k_pair_wide<R, KIND, BLK, kWideTargets, 1>),
+                       dim3((unsigned)((a.nunits + kWideWaves - 1) / kWideWaves)),
+                       dim3(kPairThreads), 0, s, a);
+  else
+    throw Error("[libmobility_amd] wide launch takes 1 or 4 waves per unit");
+  LM_HIP(hipGetLastError());
+}
+
+template <class R, int KIND>
+static void launch_wide_blk(const WideArgs& a, hipStream_t s) {
+  switch (a.blocks) {
+    case kUF: launch_wide_split<R, KIND, kUF>(a, s); break;
+    case kUF | kWF: launch_wide_split<R, KIND, kUF | kWF>(a, s); break;
+    case kUT | kWT: launch_wide_split<R, KIND, kUT | kWT>(a, s); break;
+    case kUF | kUT | kWT | kWF: launch_wide_split<R, KIND, kUF | kUT | kWT | kWF>(a, s); break;
+    default: throw Error("[libmobility_amd] unsupported block combination");
+  }
+}
+
+template <class R>
+static void launch_wide_r(const WideArgs& a, hipStream_t s) {
+  switch (a.kind) {
+    case 0: launch_wide_blk<R, 0>(a, s); break;
+    case 1: launch_wide_blk<R, 1>(a, s); break;
+    case 2: launch_wide_blk<R, 2>(a, s); break;
+    default: throw Error("[libmobility_amd] invalid kernel kind");
+  }
+}
+
+void launch_pair_wide(const WideArgs& a, hipStream_t s) {
+  if (a.nunits <= 0) return;
+  if (a.fp32)
+    launch_wide_r<float>(a, s);
+  else
+    launch_wide_r<double>(a, s);
+}
+
+}  // namespace lm
