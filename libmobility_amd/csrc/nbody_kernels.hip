@@ -252,7 +252,16 @@ __device__ inline void sym_item(const SymItem& it, const SymArgs& a, typename Re
                                 typename Rec<R>::T* s_f, R* s_red) {
   using R4 = typename Rec<R>::T;
   constexpr int kTile = kPairThreads * TPL;
-  constexpr int SG = TPL >= 4 ? 1 : 4 / TPL;  // steps per overlap test (4 pairs)
+  // FP32: one step per overlap test, and the step's reciprocal square roots and
+  // lane moves between two scheduling fences, next to each other.  Two waves of
+  // a SIMD issue simple FP32 together (1.5-1.7 instructions per CU cycle, other
+  // VALU instructions 0.9, v_rsq_f32 0.47), but every v_rsq or DPP move that
+  // stands alone in such a stream costs 3-5 issue slots, and a run of them
+  // hardly more than one.  FP64 has no such pairing and keeps groups of 4 pairs.
+  //   131072 particles, 4 targets per lane 5.94 -> 5.55 ms, 2 per lane 6.25 ->
+  //   5.75 ms; 32768, 2 per lane 449 -> 414 us; 20011, 1 per lane 195 -> 186 us.
+  constexpr bool kFence = std::is_same<R, float>::value;
+  constexpr int SG = kFence || TPL >= 4 ? 1 : 4 / TPL;  // steps per overlap test
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const R4* __restrict__ pos = static_cast<const R4*>(a.pos);
   const double* __restrict__ F = a.F;
@@ -327,12 +336,28 @@ __device__ inline void sym_item(const SymItem& it, const SymArgs& a, typename Re
               dy[g][t] = pi[t].y - pg[g].y;
               dz[g][t] = pi[t].z - pg[g].z;
               r2[g][t] = dx[g][t] * dx[g][t] + dy[g][t] * dy[g][t] + dz[g][t] * dz[g][t];
-              ir[g][t] = lm_rsqrt(r2[g][t]);
-              cf[g][t] = RpyCoef<R>{};
-              rpy_far_uf34<R>(ir[g][t], cf[g][t]);
               near.add(r2[g][t]);
             }
           }
+          if constexpr (kFence) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int g = 0; g < SG; ++g)
+#pragma unroll
+            for (int t = 0; t < TPL; ++t) ir[g][t] = lm_rsqrt(r2[g][t]);
+          if constexpr (kFence) {
+            // the running sum moves here, beside the reciprocal square roots
+            sa.x = lane_rol1(sa.x);
+            sa.y = lane_rol1(sa.y);
+            sa.z = lane_rol1(sa.z);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+#pragma unroll
+          for (int g = 0; g < SG; ++g)
+#pragma unroll
+            for (int t = 0; t < TPL; ++t) {
+              cf[g][t] = RpyCoef<R>{};
+              rpy_far_uf34<R>(ir[g][t], cf[g][t]);
+            }
           if (__builtin_expect(near.hit(), 0)) {
             __asm__ __volatile__("");  // keep this a branch
 #pragma unroll
@@ -344,9 +369,11 @@ __device__ inline void sym_item(const SymItem& it, const SymArgs& a, typename Re
           for (int g = 0; g < SG; ++g) {
             // the running sum moves first and the step's terms accumulate
             // into it: one move per component and step, no separate add
-            sa.x = lane_rol1(sa.x);
-            sa.y = lane_rol1(sa.y);
-            sa.z = lane_rol1(sa.z);
+            if constexpr (!kFence) {
+              sa.x = lane_rol1(sa.x);
+              sa.y = lane_rol1(sa.y);
+              sa.z = lane_rol1(sa.z);
+            }
 #pragma unroll
             for (int t = 0; t < TPL; ++t) {
               const R fuf = cf[g][t].fuf, guf = cf[g][t].guf;
