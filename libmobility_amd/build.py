@@ -13,7 +13,7 @@ OUT_DIR = os.path.join(HERE, "lib")
 LIB = os.path.join(OUT_DIR, "liblmamd.so")
 OBJ_DIR = os.path.join(HERE, "_build")
 
-SOURCES = ["nbody_kernels.hip", "wide_kernels.hip", "lanczos_kernels.hip", "precond_kernels.hip",
+SOURCES = ["nbody_kernels.hip", "wide_kernels.hip", "sym_kernels.hip", "lanczos_kernels.hip", "precond_kernels.hip",
            "coarse_kernels.hip", "noalloc.hip", "coarse.cpp", "precond.cpp", "solver.cpp", "self_solver.cpp", "capi.cpp"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -41,7 +41,7 @@ def _compile(src):
 def build(verbose=True):
     os.makedirs(OBJ_DIR, exist_ok=True)
     os.makedirs(OUT_DIR, exist_ok=True)
-    with ThreadPoolExecutor(max_workers=min(4, os.cpu_count() or 1)) as ex:
+    with ThreadPoolExecutor(max_workers=min(8, os.cpu_count() or 1)) as ex:
         objs = list(ex.map(_compile, SOURCES))
     tmp = LIB + ".tmp"
     cmd = [HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", tmp, *objs]

@@ -435,19 +435,13 @@ int lm_selftest_pair_block_host(int wall, int fp32, const double* pi, const doub
       for (int col = 0; col < 6; ++col) {
         R v[6] = {0, 0, 0, 0, 0, 0};
         v[col] = R(1);
-        lm::PairAcc<R> acc;
-        lm::acc_zero(acc);
-        constexpr int all = lm::kUF | lm::kUT | lm::kWT | lm::kWF;
+        const lm::Vec3<R> f = {v[0], v[1], v[2]}, t = {v[3], v[4], v[5]};
+        R u[6];
         if (wall)
-          lm::wall_pair<R, all>(ri[0], ri[1], ri[2], ri[3], rj[0], rj[1], rj[2], rj[3], v[0], v[1],
-                                v[2], v[3], v[4], v[5], acc);
+          lm::block_column<R, true, false>(ri, rj, f, t, u);
         else
-          lm::open_pair<R, all>(ri[0] - rj[0], ri[1] - rj[1], ri[2] - rj[2], v[0], v[1], v[2], v[3],
-                                v[4], v[5], acc);
-        const double u[6] = {double(acc.uf.x + acc.ut.x), double(acc.uf.y + acc.ut.y),
-                             double(acc.uf.z + acc.ut.z), double(acc.wt.x + acc.wf.x),
-                             double(acc.wt.y + acc.wf.y), double(acc.wt.z + acc.wf.z)};
-        for (int row = 0; row < 6; ++row) blk[row * 6 + col] = u[row];
+          lm::block_column<R, false, false>(ri, rj, f, t, u);
+        for (int row = 0; row < 6; ++row) blk[row * 6 + col] = (double)u[row];
       }
     };
     if (fp32)
@@ -471,34 +465,20 @@ int lm_selftest_pair_both_host(int wall, const double* pi, const double* pj, dou
       r[q][2] = wall ? (z > a ? z : a) / a : z / a;
       r[q][3] = wall ? (b < 0 ? 0 : (b > 1 ? 1 : b)) : 1.0;
     }
-    constexpr int all = lm::kUF | lm::kUT | lm::kWT | lm::kWF;
-    const lm::Vec3<double> zero = {0, 0, 0};
     for (int col = 0; col < 6; ++col) {
       double v[6] = {0, 0, 0, 0, 0, 0};
       v[col] = 1.0;
       const lm::Vec3<double> f = {v[0], v[1], v[2]}, t = {v[3], v[4], v[5]};
       // forward: unit force/torque on j, velocities of i; reverse: unit
       // force/torque on i, what the same pair gives j (transposed blocks)
-      lm::PairAcc<double> acc;
-      lm::acc_zero(acc);
-      lm::Vec3<double> su = zero, sw = zero, du = zero, dw = zero;
-      lm::PairAcc<double> dummy;
-      lm::acc_zero(dummy);
+      double u[6], s6[6];
       if (wall) {
-        lm::pair_both<double, true, all>(r[0][0], r[0][1], r[0][2], r[0][3], r[1][0], r[1][1],
-                                         r[1][2], r[1][3], f, t, zero, zero, 1.0, 1.0, acc, du, dw);
-        lm::pair_both<double, true, all>(r[0][0], r[0][1], r[0][2], r[0][3], r[1][0], r[1][1],
-                                         r[1][2], r[1][3], zero, zero, f, t, 1.0, 1.0, dummy, su, sw);
+        lm::block_column<double, true, false>(r[0], r[1], f, t, u);
+        lm::block_column<double, true, true>(r[0], r[1], f, t, s6);
       } else {
-        lm::pair_both<double, false, all>(r[0][0], r[0][1], r[0][2], r[0][3], r[1][0], r[1][1],
-                                          r[1][2], r[1][3], f, t, zero, zero, 1.0, 1.0, acc, du, dw);
-        lm::pair_both<double, false, all>(r[0][0], r[0][1], r[0][2], r[0][3], r[1][0], r[1][1],
-                                          r[1][2], r[1][3], zero, zero, f, t, 1.0, 1.0, dummy, su,
-                                          sw);
+        lm::block_column<double, false, false>(r[0], r[1], f, t, u);
+        lm::block_column<double, false, true>(r[0], r[1], f, t, s6);
       }
-      const double u[6] = {acc.uf.x + acc.ut.x, acc.uf.y + acc.ut.y, acc.uf.z + acc.ut.z,
-                           acc.wt.x + acc.wf.x, acc.wt.y + acc.wf.y, acc.wt.z + acc.wf.z};
-      const double s6[6] = {su.x, su.y, su.z, sw.x, sw.y, sw.z};
       for (int row = 0; row < 6; ++row) {
         fwd[row * 6 + col] = u[row];
         rev[row * 6 + col] = s6[row];

@@ -56,7 +56,17 @@ template <bool WALL, class R, class R4>
 __device__ inline void pair_block_sum(const R4 ri, const R4 rj, R s[9]) {
   if (WALL) {
     UFCoef<R> k;
-    uf_coef_wall<R>(ri.x, ri.y, ri.z, ri.w, rj.x, rj.y, rj.z, rj.w, k);
+    uf_coef_wall<R>(ri.x, ri.y, ri.z, rj.x, rj.y, rj.z, k);
+    // the damping, and back from 4/3 of the block
+    const R q = R(0.75) * ri.w * rj.w;
+    k.a0 *= q;
+    k.cd *= q;
+    k.ex *= q;
+    k.ey *= q;
+    k.ez *= q;
+    k.hx *= q;
+    k.hy *= q;
+    k.hz *= q;
     const R dv[3] = {k.dx, k.dy, k.dz};
     const R ev[3] = {k.ex, k.ey, k.ez};
     const R gv[3] = {k.gx, k.gy, k.gz};

@@ -98,7 +98,7 @@ constexpr int multi_tpl(int nrhs) { return nrhs >= 4 ? 1 : 2; }
 // Symmetric evaluation (any block set, open or bottom-wall systems, one system
 // or an ensemble): the grand mobility matrix is symmetric (M_ji = M_ij^T
 // blockwise), so each unordered pair is evaluated once and applied to both
-// particles.  Each system is cut into tiles of 256 * tpl particles; tile I
+// particles.  Each system is cut into tiles of 64 * waves * tpl particles; tile I
 // meets tiles I + o (mod ntiles) for o = 1 .. hmax, hmax = ntiles / 2 (offset
 // ntiles / 2 of an even count only from I < ntiles / 2), so every unordered
 // tile pair of the system is met once.  Target-side sums of an item go to
@@ -108,9 +108,11 @@ constexpr int multi_tpl(int nrhs) { return nrhs >= 4 ? 1 : 2; }
 struct SymSys {
   int64_t off;     // first particle
   int32_t n;       // particles
-  int32_t ntiles;  // tiles of 256 * tpl
+  int32_t ntiles;  // tiles of 64 * waves * tpl
   int32_t hmax;    // ring offsets, ntiles / 2
   int32_t wall;    // 0 open RPY, 1 bottom wall
+  int32_t per;     // offsets per item (0: the pass's chunks share them evenly)
+  int32_t pad;
 };
 struct SymItem {
   int32_t sys;     // system
@@ -118,7 +120,7 @@ struct SymItem {
   int32_t o0, o1;  // partner offsets [o0, o1); o0 = 0: the diagonal tile
   int32_t chunk;   // target slab
 };
-// At most 256 particles of one tile of one system, for the reduction.
+// At most 256 particles of one system, for the reduction.
 struct SymRows {
   int64_t p0;
   int32_t np;
@@ -127,6 +129,7 @@ struct SymRows {
 struct SymArgs {
   int fp32;
   int tpl;
+  int waves;         // waves per workgroup: 4, or 1
   int wall;          // 0 open RPY, 1 bottom wall, 2 per system
   int blocks;        // BlockBits mask
   const void* pos;   // float4 / double4 records
@@ -147,7 +150,11 @@ struct SymArgs {
   const int* stop;
   double t0, rt0, r0;
 };
+// The open translational block in FP32, and (open blocks) the order of
+// operations that plain Lanczos products keep; 4 waves per workgroup.
 void launch_pair_sym(const SymArgs& a, hipStream_t s);
+// Every form, in symmetric units.
+void launch_pair_sym_unit(const SymArgs& a, hipStream_t s);
 // Per row block: out (= or +=, accumulate) the system's target slabs of the
 // pass (its chunks of offsets [o0, o1), at most nch of them, then the
 // diagonal slab nch when `diag`), then its source slabs of offsets o0 ..
@@ -158,7 +165,8 @@ struct SymReduceArgs {
   const double* slab_t;
   const double* slab_s;
   int64_t n3;
-  int nch, o0, o1, diag, accumulate, tpl;
+  int nch, o0, o1, diag, accumulate;
+  int tile;  // particles per tile
   const SymSys* sys;
   const SymRows* rows;
   int nrows;

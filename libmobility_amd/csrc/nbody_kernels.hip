@@ -19,6 +19,7 @@
 #include "lm_common.hpp"
 #include "pair_device.hpp"
 #include "pair_math.hpp"
+#include "sym_item.hpp"
 
 namespace lm {
 
@@ -59,9 +60,12 @@ __device__ inline void pair_item(const PairItem& it, const typename Rec<R>::T* _
     const int cnt = (int)min((int64_t)kPairThreads, it.src1 - base);
     __syncthreads();
     if (j < it.src1) {
-      s_pos[tid] = pos[j];
-      if (kNeedF) s_f[tid] = R4{R(F[3 * j]), R(F[3 * j + 1]), R(F[3 * j + 2]), R(0)};
-      if (kNeedT) s_t[tid] = R4{R(T[3 * j]), R(T[3 * j + 1]), R(T[3 * j + 2]), R(0)};
+      const R4 pj = pos[j];
+      s_pos[tid] = pj;
+      // wall: symmetric units (pair_math.hpp), the damping with the force
+      const R bf = WALL ? pj.w : R(1), bt = WALL ? pj.w * R(r0 / rt0) : R(1);
+      if (kNeedF) s_f[tid] = R4{bf * R(F[3 * j]), bf * R(F[3 * j + 1]), bf * R(F[3 * j + 2]), R(0)};
+      if (kNeedT) s_t[tid] = R4{bt * R(T[3 * j]), bt * R(T[3 * j + 1]), bt * R(T[3 * j + 2]), R(0)};
     } else {
       s_pos[tid] = far_record<R4>();
       if (kNeedF) s_f[tid] = R4{R(0), R(0), R(0), R(0)};
@@ -71,13 +75,19 @@ __device__ inline void pair_item(const PairItem& it, const typename Rec<R>::T* _
     if constexpr (WALL) {
       for (int s = 0; s < cnt; ++s) {
         const R4 pj = s_pos[s];
-        R4 fj, tj;
-        if (kNeedF) fj = s_f[s]; else fj = R4{R(0), R(0), R(0), R(0)};
-        if (kNeedT) tj = s_t[s]; else tj = R4{R(0), R(0), R(0), R(0)};
+        const Vec3<R> zero = {R(0), R(0), R(0)};
+        Vec3<R> fj = zero, tj = zero, none = zero;
+        if (kNeedF) fj = {s_f[s].x, s_f[s].y, s_f[s].z};
+        if (kNeedT) tj = {s_t[s].x, s_t[s].y, s_t[s].z};
 #pragma unroll
-        for (int k = 0; k < TPL; ++k)
-          wall_pair<R, BLK>(pi[k].x, pi[k].y, pi[k].z, pi[k].w, pj.x, pj.y, pj.z, pj.w, fj.x,
-                            fj.y, fj.z, tj.x, tj.y, tj.z, acc[k]);
+        for (int k = 0; k < TPL; ++k) {
+          // U in acc.uf, W in acc.wf
+          PairGeo<R> g;
+          pair_distances<R, true>(pi[k].x, pi[k].y, pi[k].z, pj.x, pj.y, pj.z, g);
+          pair_inverses<R, true>(g);
+          pair_unit<R, true, BLK, false>(g, pj.z, fj, tj, zero, zero, acc[k].uf, acc[k].wf, none,
+                                         none);
+        }
       }
     } else {
       // Open boundaries: a group of SG sources x TPL targets (4 pairs) gets
@@ -156,6 +166,12 @@ __device__ inline void pair_item(const PairItem& it, const typename Rec<R>::T* _
     if (loc < it.ntgt) {
       const int64_t i = it.tgt0 + loc;
       const PairAcc<double>& a = acc64[k];
+      if constexpr (WALL) {
+        const double b = (double)pi[k].w;
+        put3(Uo + 3 * i, 0.75 * t0 * b, a.uf.x, a.uf.y, a.uf.z);
+        if (kAngular) put3(Wo + 3 * i, rt0 * b, a.wf.x, a.wf.y, a.wf.z);
+        continue;
+      }
       Uo[3 * i + 0] = tuf * a.uf.x + rt0 * a.ut.x;
       Uo[3 * i + 1] = tuf * a.uf.y + rt0 * a.ut.y;
       Uo[3 * i + 2] = tuf * a.uf.z + rt0 * a.ut.z;
@@ -228,24 +244,6 @@ __global__ __launch_bounds__(kPairThreads) void k_pair(
 // (DPP wave_rol:1), so after 64 steps every source has met all targets of the
 // wave and its sum sits back in lane (source index).  The four waves' sums are
 // added in a fixed order and written once per source to the offset's slab.
-
-// Lane l receives lane (l + 1) mod 64.
-template <class R>
-__device__ inline R lane_rol1(R v);
-template <>
-__device__ inline float lane_rol1<float>(float v) {
-  return __builtin_bit_cast(
-      float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x134, 0xf, 0xf, true));
-}
-template <>
-__device__ inline double lane_rol1<double>(double v) {
-  const uint64_t b = __builtin_bit_cast(uint64_t, v);
-  const uint32_t lo =
-      (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, 0x134, 0xf, 0xf, true);
-  const uint32_t hi =
-      (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), 0x134, 0xf, 0xf, true);
-  return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
-}
 
 template <class R, int TPL>
 __device__ inline void sym_item(const SymItem& it, const SymArgs& a, typename Rec<R>::T* s_pos,
@@ -433,11 +431,12 @@ __device__ inline void sym_item(const SymItem& it, const SymArgs& a, typename Re
   }
 }
 
-// General symmetric item (bottom wall, or open boundaries with angular
-// blocks): the same ring, lanes and rotation as sym_item, with pair_both
-// giving both directions of every block from one set of coefficients.  The
-// source sums carry U (units of t0) and, with angular blocks, W (units of r0).
-template <class R, bool WALL, int BLK, int TPL>
+// Open boundaries with angular blocks, in the order of operations that plain
+// Lanczos products keep: the same ring, lanes and rotation as sym_item, with
+// open_both giving both directions of every block from one set of
+// coefficients.  The source sums carry U (units of t0) and, with angular
+// blocks, W (units of r0).
+template <class R, int BLK, int TPL>
 __device__ inline void sym_item_gen(const SymItem& it, const SymArgs& a,
                                     typename Rec<R>::T* s_pos, typename Rec<R>::T* s_f,
                                     typename Rec<R>::T* s_t, R* s_red) {
@@ -516,8 +515,8 @@ __device__ inline void sym_item_gen(const SymItem& it, const SymArgs& a,
           Vec3<R> cu = zero, cw = zero;
 #pragma unroll
           for (int t = 0; t < TPL; ++t)
-            pair_both<R, WALL, BLK>(pi[t].x, pi[t].y, pi[t].z, pi[t].w, pj4.x, pj4.y, pj4.z, pj4.w,
-                                    fj, tj, fi[t], ti[t], kut, kwf, acc[t], cu, cw);
+            open_pair_both<R, BLK>(pi[t].x - pj4.x, pi[t].y - pj4.y, pi[t].z - pj4.z, fj, tj,
+                                   fi[t], ti[t], kut, kwf, acc[t], cu, cw);
           su.x = lane_rol1(su.x) + cu.x;
           su.y = lane_rol1(su.y) + cu.y;
           su.z = lane_rol1(su.z) + cu.z;
@@ -593,19 +592,28 @@ __device__ inline void sym_item_gen(const SymItem& it, const SymArgs& a,
   }
 }
 
+// LDS of one item of the order-keeping evaluation.
+template <class R, int BLK>
+struct SymKeepLds {
+  using R4 = typename Rec<R>::T;
+  R4 pos[4 * 128];
+  R4 f[(BLK & (kUF | kWF)) ? 4 * 128 : 1];
+  R4 t[(BLK & (kUT | kWT)) ? 4 * 128 : 1];
+  R red[4 * ((BLK & (kWT | kWF)) ? 6 : 3) * kPairThreads];
+};
+
 // One item per workgroup: a diagonal tile (all ordered pairs of tile I, the
-// self pairs included) or a range of partner offsets.  KIND: 0 open, 1 wall,
-// 2 per system (mixed ensembles).
+// self pairs included) or a range of partner offsets.  KIND: 0 open, 2 per
+// system (mixed ensembles; their wall systems run in symmetric units).
 template <class R, int KIND, int BLK, int TPL>
 __global__ __launch_bounds__(kPairThreads) void k_pair_sym(SymArgs a) {
   using R4 = typename Rec<R>::T;
-  constexpr bool kNeedF = (BLK & (kUF | kWF)) != 0;
-  constexpr bool kNeedT = (BLK & (kUT | kWT)) != 0;
-  constexpr int kComp = (BLK & (kWT | kWF)) ? 6 : 3;
-  __shared__ R4 s_pos[4 * 128];
-  __shared__ R4 s_f[kNeedF ? 4 * 128 : 1];
-  __shared__ R4 s_t[kNeedT ? 4 * 128 : 1];
-  __shared__ R s_red[4 * kComp * kPairThreads];
+  using Keep = SymKeepLds<R, BLK>;
+  using Unit = SymLds<R, BLK, 4>;
+  constexpr size_t kLds =
+      KIND == 2 && sizeof(Unit) > sizeof(Keep) ? sizeof(Unit) : sizeof(Keep);
+  __shared__ __align__(16) unsigned char s_mem[kLds];
+  Keep& lds = *reinterpret_cast<Keep*>(s_mem);
   if (a.stop != nullptr) {
     // one read per workgroup, so that all its threads take the same branch
     __shared__ int s_stop;
@@ -616,7 +624,12 @@ __global__ __launch_bounds__(kPairThreads) void k_pair_sym(SymArgs a) {
   const SymItem it = a.items[blockIdx.x];
   if (a.active != nullptr && a.active[it.sys] == 0) return;  // system already converged
   const SymSys S = a.sys[it.sys];
-  const bool wall = KIND == 2 ? S.wall != 0 : KIND == 1;
+  if constexpr (KIND == 2) {
+    if (S.wall != 0) {
+      sym_unit<R, true, BLK, TPL, 4>(it, S, a, *reinterpret_cast<Unit*>(s_mem));
+      return;
+    }
+  }
   if (it.o0 == 0) {
     constexpr int kTile = kPairThreads * TPL;
     PairItem p;
@@ -626,35 +639,16 @@ __global__ __launch_bounds__(kPairThreads) void k_pair_sym(SymArgs a) {
     p.src0 = p.tgt0;
     p.src1 = p.tgt0 + p.ntgt;
     p.chunk = it.chunk;
-    p.wall = wall ? 1 : 0;
+    p.wall = 0;
     p.sys = it.sys;
-    const R4* pos = static_cast<const R4*>(a.pos);
-    R4* sf = kNeedF ? s_f : s_pos;
-    R4* st = kNeedT ? s_t : s_pos;
-    if constexpr (KIND != 0) {
-      if (wall) {
-        pair_item<R, true, BLK, TPL>(p, pos, a.F, a.T, a.slab_t, a.slab_tw, a.n3, a.t0, a.rt0, a.r0,
-                                     s_pos, sf, st);
-        return;
-      }
-    }
-    if constexpr (KIND != 1)
-      pair_item<R, false, BLK, TPL>(p, pos, a.F, a.T, a.slab_t, a.slab_tw, a.n3, a.t0, a.rt0, a.r0,
-                                    s_pos, sf, st);
+    pair_item<R, false, BLK, TPL>(p, static_cast<const R4*>(a.pos), a.F, a.T, a.slab_t, a.slab_tw,
+                                  a.n3, a.t0, a.rt0, a.r0, lds.pos, lds.f, lds.t);
     return;
   }
-  if constexpr (KIND != 0) {
-    if (wall) {
-      sym_item_gen<R, true, BLK, TPL>(it, a, s_pos, s_f, s_t, s_red);
-      return;
-    }
-  }
-  if constexpr (KIND != 1) {
-    if constexpr (BLK == kUF)
-      sym_item<R, TPL>(it, a, s_pos, s_f, s_red);  // the open translational fast path
-    else
-      sym_item_gen<R, false, BLK, TPL>(it, a, s_pos, s_f, s_t, s_red);
-  }
+  if constexpr (BLK == kUF)
+    sym_item<R, TPL>(it, a, lds.pos, lds.f, lds.red);
+  else
+    sym_item_gen<R, BLK, TPL>(it, a, lds.pos, lds.f, lds.t, lds.red);
 }
 
 // ---- several force vectors per pass (translational block) ----------------------
@@ -686,11 +680,13 @@ __device__ inline void pair_item_multi(const PairItem& it, const typename Rec<R>
     const int64_t j = base + tid;
     __syncthreads();
     if (j < it.src1) {
-      s_pos[tid] = pos[j];
+      const R4 pj = pos[j];
+      s_pos[tid] = pj;
+      const R b = WALL ? pj.w : R(1);  // the wall's damping goes with the force
 #pragma unroll
       for (int r = 0; r < NR; ++r) {
         const double* f = F + (int64_t)r * n3 + 3 * j;
-        s_f[r * kPairThreads + tid] = R4{R(f[0]), R(f[1]), R(f[2]), R(0)};
+        s_f[r * kPairThreads + tid] = R4{b * R(f[0]), b * R(f[1]), b * R(f[2]), R(0)};
       }
     } else {
       s_pos[tid] = far_record<R4>();
@@ -707,7 +703,7 @@ __device__ inline void pair_item_multi(const PairItem& it, const typename Rec<R>
       for (int k = 0; k < TPL; ++k) {
         UFCoef<R> c;
         if constexpr (WALL) {
-          uf_coef_wall<R>(pi[k].x, pi[k].y, pi[k].z, pi[k].w, pj.x, pj.y, pj.z, pj.w, c);
+          uf_coef_wall<R>(pi[k].x, pi[k].y, pi[k].z, pj.x, pj.y, pj.z, c);
 #pragma unroll
           for (int r = 0; r < NR; ++r) uf_apply_wall<R>(c, fj[r].x, fj[r].y, fj[r].z, acc[k][r]);
         } else {
@@ -755,7 +751,7 @@ __device__ inline void pair_item_multi(const PairItem& it, const typename Rec<R>
 #pragma unroll
       for (int r = 0; r < NR; ++r) {
         double* o = U + ((int64_t)r * nch + it.chunk) * n3;
-        const double tuf = WALL ? t0 : 0.75 * t0;
+        const double tuf = 0.75 * t0 * (WALL ? (double)pi[k].w : 1.0);
         o[3 * i + 0] = tuf * acc64[k][r].x;
         o[3 * i + 1] = tuf * acc64[k][r].y;
         o[3 * i + 2] = tuf * acc64[k][r].z;
@@ -891,12 +887,11 @@ static void launch_pair_sym_tpl(const SymArgs& a, hipStream_t s) {
   LM_HIP(hipGetLastError());
 }
 
+// Lanczos products have forces, or forces and torques.
 template <class R, int KIND>
 static void launch_pair_sym_blk(const SymArgs& a, hipStream_t s) {
   switch (a.blocks) {
     case kUF: launch_pair_sym_tpl<R, KIND, kUF>(a, s); break;
-    case kUF | kWF: launch_pair_sym_tpl<R, KIND, kUF | kWF>(a, s); break;
-    case kUT | kWT: launch_pair_sym_tpl<R, KIND, kUT | kWT>(a, s); break;
     case kUF | kUT | kWT | kWF: launch_pair_sym_tpl<R, KIND, kUF | kUT | kWT | kWF>(a, s); break;
     default: throw Error("[libmobility_amd] unsupported block combination");
   }
@@ -906,7 +901,6 @@ template <class R>
 static void launch_pair_sym_r(const SymArgs& a, hipStream_t s) {
   switch (a.wall) {
     case 0: launch_pair_sym_blk<R, 0>(a, s); break;
-    case 1: launch_pair_sym_blk<R, 1>(a, s); break;
     case 2: launch_pair_sym_blk<R, 2>(a, s); break;
     default: throw Error("[libmobility_amd] invalid kernel kind");
   }
@@ -914,6 +908,7 @@ static void launch_pair_sym_r(const SymArgs& a, hipStream_t s) {
 
 void launch_pair_sym(const SymArgs& a, hipStream_t s) {
   if (a.nitems <= 0) return;
+  if (a.waves != 4) throw Error("[libmobility_amd] unsupported shape of the symmetric kernel");
   if (a.fp32)
     launch_pair_sym_r<float>(a, s);
   else
@@ -942,8 +937,8 @@ __device__ inline double add_slabs(double s, const double* __restrict__ p, int c
   return s;
 }
 
-// Three workgroups per row block (at most 256 particles of one tile of one
-// system), one thread per entry.  Bound by HBM for large systems (607 MB at
+// Three workgroups per row block (at most 256 particles of one system), one
+// thread per entry.  Bound by HBM for large systems (607 MB at
 // 131072 particles and 193 slabs: 116 -> 100 us, 6.0 TB/s) and by latency for
 // small ones (20011 particles, 79 slabs: 23.7 -> 8.4 us; 10007, 41 slabs: 6.7
 // -> 3.9 us, against one workgroup per row block and one load at a time).
@@ -953,11 +948,12 @@ __global__ __launch_bounds__(kPairThreads) void k_sym_reduce(SymReduceArgs r) {
   const int64_t e = 3 * rb.p0 + (int64_t)(blockIdx.x % 3) * kPairThreads + threadIdx.x;
   if (e >= 3 * (rb.p0 + rb.np)) return;
   const SymSys S = r.sys[rb.sys];
-  const int64_t kTile = (int64_t)kPairThreads * r.tpl;
-  const int tile = (int)((rb.p0 - S.off) / kTile);
+  const int tile = (int)((e / 3 - S.off) / r.tile);
   const int hi = min(r.o1, S.hmax + 1);  // this system's offsets in the pass: [o0, hi)
   const int width = hi - r.o0;
-  const int nchp = width > 0 ? min(r.nch, width) : 0;
+  // target slabs of this system in the pass
+  const int nchp =
+      width <= 0 ? 0 : (S.per > 0 ? (width + S.per - 1) / S.per : min(r.nch, width));
   // an even tile count meets offset ntiles/2 only from tiles I < ntiles/2, so
   // that slab (the ring's last) holds no rows of tiles J < ntiles/2
   const bool drop = S.ntiles % 2 == 0 && 2 * tile < S.ntiles && hi - 1 == S.ntiles / 2;

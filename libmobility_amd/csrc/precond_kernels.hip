@@ -232,7 +232,6 @@ __global__ __launch_bounds__(256) void k_local_targets(const double4* __restrict
                                                        float* __restrict__ target,
                                                        int* __restrict__ status) {
   constexpr int KD = D * KC, LD = KD + 1;
-  constexpr int BLK = D == 6 ? (kUF | kUT | kWT | kWF) : kUF;
   __shared__ double buf[4][KD * LD];
   __shared__ double4 P[KC];
   __shared__ double red[4];
@@ -256,33 +255,26 @@ __global__ __launch_bounds__(256) void k_local_targets(const double4* __restrict
     for (int col = 0; col < D; ++col) {
       double v[6] = {0, 0, 0, 0, 0, 0};
       v[col] = 1.0;
-      PairAcc<double> acc;
-      acc_zero(acc);
+      const double ra[4] = {pa.x, pa.y, pa.z, pa.w}, rb[4] = {pb.x, pb.y, pb.z, pb.w};
+      const Vec3<double> f = {v[0], v[1], v[2]}, t = {v[3], v[4], v[5]};
+      double q[6];
       if (wall)
-        wall_pair<double, BLK>(pa.x, pa.y, pa.z, pa.w, pb.x, pb.y, pb.z, pb.w, v[0], v[1], v[2],
-                               v[3], v[4], v[5], acc);
+        block_column<double, true, false>(ra, rb, f, t, q);
       else
-        open_pair<double, BLK>(pa.x - pb.x, pa.y - pb.y, pa.z - pb.z, v[0], v[1], v[2], v[3],
-                               v[4], v[5], acc);
+        block_column<double, false, false>(ra, rb, f, t, q);
       double* c = Y + (D * a) * LD + D * b + col;
       if (D == 3) {
-        c[0 * LD] = acc.uf.x;
-        c[1 * LD] = acc.uf.y;
-        c[2 * LD] = acc.uf.z;
-      } else if (col < 3) {  // a force: U from UF, W from WF
-        c[0 * LD] = acc.uf.x;
-        c[1 * LD] = acc.uf.y;
-        c[2 * LD] = acc.uf.z;
-        c[3 * LD] = s3 * acc.wf.x;
-        c[4 * LD] = s3 * acc.wf.y;
-        c[5 * LD] = s3 * acc.wf.z;
-      } else {  // a torque: U from UT, W from WT
-        c[0 * LD] = s3 * acc.ut.x;
-        c[1 * LD] = s3 * acc.ut.y;
-        c[2 * LD] = s3 * acc.ut.z;
-        c[3 * LD] = acc.wt.x;
-        c[4 * LD] = acc.wt.y;
-        c[5 * LD] = acc.wt.z;
+        c[0 * LD] = q[0];
+        c[1 * LD] = q[1];
+        c[2 * LD] = q[2];
+      } else {  // a force: U from UF, W from WF; a torque: U from UT, W from WT
+        const double su = col < 3 ? 1.0 : s3, sw = col < 3 ? s3 : 1.0;
+        c[0 * LD] = su * q[0];
+        c[1 * LD] = su * q[1];
+        c[2 * LD] = su * q[2];
+        c[3 * LD] = sw * q[3];
+        c[4 * LD] = sw * q[4];
+        c[5 * LD] = sw * q[5];
       }
     }
   }

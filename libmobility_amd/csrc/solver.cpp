@@ -342,36 +342,72 @@ void NBodySolver::setPairSymmetricMemory(int64_t bytes) {
   sym_budget_ = bytes == 0 ? kDefaultSymBudget : bytes;
 }
 
-// Shape of a symmetric tiling request (0 = default rule): targets per lane
-// (open translational block of one system: 2 from N = 65536, else 1; other
-// cases 1, at most 2) and offset chunks per tile (about 8192 items), at most
-// the longest ring.  ntiles is the total over systems, hmax the longest ring.
-void NBodySolver::sym_shape(bool special, int tpl_req, int nch_req, int& tpl, int& nch,
-                            int& ntiles, int& hmax) const {
+// Shape of a symmetric tiling request (0 = default rule): waves per workgroup,
+// targets per lane, and offset chunks per tile, at most the longest ring.  ntiles is the total over systems, hmax the longest ring.
+NBodySolver::SymShape NBodySolver::sym_shape(int blocks, bool fp32, int tpl_req, int nch_req) {
   const int nsys = (int)sys_off_host_.size() - 1;
-  tpl = tpl_req != 0 ? tpl_req : (special && nsys == 1 && N_ >= 65536 ? 2 : 1);
-  if (!(special && nsys == 1)) tpl = std::min(tpl, 2);  // 4 only for one open system
-  const int64_t bt = (int64_t)kPairThreads * tpl;
-  ntiles = 0;
-  hmax = 0;
+  const bool open_uf = kind_code() == 0 && blocks == kUF && nsys == 1;
+  SymShape sh;
+  const bool lanczos_blocks = blocks == kUF || blocks == (kUF | kUT | kWT | kWF);
+  sh.keep = (keep_order_ && kind_code() != 1 && lanczos_blocks) ||
+            (fp32 && kind_code() == 0 && blocks == kUF) || (open_uf && tpl_req == 4);
+  if (sh.keep) {
+    sh.tpl = tpl_req != 0 ? tpl_req : (open_uf && N_ >= 65536 ? 2 : 1);
+    if (!keep_order_ && tpl_req == 0 && open_uf) sh.tpl = N_ >= 98304 ? 4 : (N_ >= 32768 ? 2 : 1);
+    if (!open_uf) sh.tpl = std::min(sh.tpl, 2);  // 4 only for one open system
+  } else {
+    const double n = nsys == 1 ? (double)N_ : mean_system_size();
+    sh.waves = tpl_req == 0 && n < kSymWaveN ? 1 : 4;
+    sh.tpl = tpl_req != 0 ? std::min(tpl_req, 2) : (!any_wall_ && n >= kSymTwoN ? 2 : 1);
+  }
+  const int64_t bt = 64 * (int64_t)sh.waves * sh.tpl;
   for (int s = 0; s < nsys; ++s) {
     const int nt = (int)((sys_off_host_[s + 1] - sys_off_host_[s] + bt - 1) / bt);
-    ntiles += nt;
-    hmax = std::max(hmax, nt / 2);
+    sh.ntiles += nt;
+    sh.hmax = std::max(sh.hmax, nt / 2);
   }
-  nch = nch_req != 0 ? nch_req : (8192 + std::max(ntiles, 1) - 1) / std::max(ntiles, 1);
-  nch = std::min(nch, hmax);
-  if (hmax > 0) nch = std::max(nch, 1);
+  if (keep_order_ || nch_req != 0) {
+    sh.nch = nch_req != 0 ? nch_req : (8192 + std::max(sh.ntiles, 1) - 1) / std::max(sh.ntiles, 1);
+    sh.nch = std::min(sh.nch, sh.hmax);
+    if (sh.hmax > 0) sh.nch = std::max(sh.nch, 1);
+    return sh;
+  }
+  // Offsets per item: equally many in every item of a kind (48 offsets in 32
+  // chunks, every other one twice the work, took 1.3 times as long as in 16 or
+  // 48), so that there are about 16384 items: 8192 where they are single waves
+  // of one system and 4096 with two or four targets per lane, whose target
+  // slabs would cost more than the shorter tail gives (131072 particles, four
+  // targets: 5.66 ms with 32 chunks, 5.77 with 64).  A wall pair weighs three
+  // open ones; in a ragged ensemble (96 systems up to 8192, FP32) items of up
+  // to 32 offsets, 0.4 ms for one wave, made it 486 us instead of 455.
+  double work = 0.0;
+  for (int s = 0; s < nsys; ++s) {
+    const double nt = (double)((sys_off_host_[s + 1] - sys_off_host_[s] + bt - 1) / bt);
+    work += nt * std::floor(nt / 2) * (sys_kind_host_[s] ? 3.0 : 1.0);
+  }
+  const double unit = work / (sh.tpl > 1 ? 4096 : (nsys == 1 && sh.waves == 1 ? 8192 : 16384));
+  const double one = kind_code() == 1 ? 3.0 : 1.0;  // work of an offset of one kind
+  sh.per[0] = std::max(1, (int)std::lround(unit / (kind_code() == 2 ? 1.0 : one)));
+  sh.per[1] = kind_code() == 2 ? std::max(1, (int)std::lround(unit / 3.0)) : sh.per[0];
+  for (int s = 0; s < nsys; ++s) {
+    const int h = (int)((sys_off_host_[s + 1] - sys_off_host_[s] + bt - 1) / bt) / 2;
+    const int per = sh.per[sys_kind_host_[s] ? 1 : 0];
+    sh.nch = std::max(sh.nch, (h + per - 1) / per);
+  }
+  return sh;
 }
 
-bool NBodySolver::use_sym(int blocks) {
+bool NBodySolver::use_sym(int blocks, bool fp32) {
   if (sym_mode_ == 0 || N_ <= 0) return false;
   if (blocks != kUF && blocks != (kUF | kWF) && blocks != (kUT | kWT) &&
       blocks != (kUF | kUT | kWT | kWF))
     return false;
   if (sym_mode_ == 1) return true;
-  return N_ >= kSymAutoN &&
-         (keep_order_ || numSystems() == 1 || mean_system_size() > kSymAutoMean);
+  if (keep_order_) return N_ >= kSymKeepN;
+  const double n = mean_system_size();
+  if (N_ >= kSymKeepN && n >= kSymEnsembleMean) return true;
+  if (any_wall_) return n >= kSymWallN;
+  return n >= (fp32 ? kSymOpenFp32N : kSymOpenN);
 }
 
 // Items: per pass, for every system and tile, the system's chunks of the
@@ -381,12 +417,14 @@ bool NBodySolver::use_sym(int blocks) {
 // slabs (one per chunk, plus the diagonal in the first) and one source slab
 // per offset, reduced into the output in that order, the first pass
 // assigning and later ones adding.
-void NBodySolver::ensure_sym_plan(int tpl, int nch, int h, bool ang) {
-  if (sym_.N == N_ && sym_.structure == struct_id_ && sym_.tpl == tpl && sym_.nchunks == nch &&
-      sym_.ang == (ang ? 1 : 0) && sym_.budget == sym_budget_)
+void NBodySolver::ensure_sym_plan(const SymShape& sh, bool ang) {
+  SymPlan& plan = sym();
+  const int tpl = sh.tpl, nch = sh.nch, h = sh.hmax;
+  if (plan.N == N_ && plan.structure == struct_id_ && plan.tpl == tpl && plan.waves == sh.waves &&
+      plan.nchunks == nch && plan.per == sh.per[0] && plan.ang == (ang ? 1 : 0) && plan.budget == sym_budget_)
     return;
   const int nsys = (int)sys_off_host_.size() - 1;
-  const int64_t bt = (int64_t)kPairThreads * tpl;
+  const int64_t bt = 64 * (int64_t)sh.waves * tpl;
   std::vector<SymSys> systems(nsys);
   std::vector<SymRows> rows;
   for (int s = 0; s < nsys; ++s) {
@@ -397,6 +435,8 @@ void NBodySolver::ensure_sym_plan(int tpl, int nch, int h, bool ang) {
     S.ntiles = (int32_t)((e - b + bt - 1) / bt);
     S.hmax = S.ntiles / 2;
     S.wall = s < (int)sys_kind_host_.size() ? sys_kind_host_[s] : (wall_ ? 1 : 0);
+    S.per = sh.per[S.wall ? 1 : 0];
+    S.pad = 0;
     for (int64_t p0 = b; p0 < e; p0 += kPairThreads)
       rows.push_back(SymRows{p0, (int32_t)std::min<int64_t>(kPairThreads, e - p0), s});
   }
@@ -404,8 +444,8 @@ void NBodySolver::ensure_sym_plan(int tpl, int nch, int h, bool ang) {
   const double per_offset = 1.0 + (h > 0 ? (double)nch / h : 0.0);
   const int span = std::max(1, (int)(((double)sym_budget_ / unit - 2.0) / per_offset));
   std::vector<SymItem> items;
-  sym_.passes.clear();
-  sym_.max_slabs = 0;
+  plan.passes.clear();
+  plan.max_slabs = 0;
   int oa = 1;
   do {
     const int ob = std::min(h + 1, oa + span);
@@ -416,20 +456,24 @@ void NBodySolver::ensure_sym_plan(int tpl, int nch, int h, bool ang) {
     ps.oa = oa;
     ps.ob = ob;
     ps.nch = width > 0 ? std::max(1, std::min(width, (int)(((int64_t)nch * width + h - 1) / h))) : 0;
+    if (sh.per[0] > 0) {
+      const int least = std::min(sh.per[0], sh.per[1]);
+      ps.nch = (width + least - 1) / least;
+    }
     ps.diag = first ? 1 : 0;
     std::vector<std::pair<double, SymItem>> pass_items;
     for (int s = 0; s < nsys; ++s) {
       const SymSys& S = systems[s];
       const double wgt = S.wall ? 5.0 : 1.0;
       const int ws = std::min(ob, S.hmax + 1) - oa;  // this system's offsets in the pass
-      const int cs = ws > 0 ? std::min(ps.nch, ws) : 0;
+      const int cs = ws <= 0 ? 0 : (S.per > 0 ? (ws + S.per - 1) / S.per : std::min(ps.nch, ws));
       for (int I = 0; I < S.ntiles; ++I)
         for (int c = 0; c < cs; ++c) {
           SymItem it;
           it.sys = s;
           it.tile = I;
-          it.o0 = oa + (int)((int64_t)c * ws / cs);
-          it.o1 = oa + (int)((int64_t)(c + 1) * ws / cs);
+          it.o0 = oa + (S.per > 0 ? c * S.per : (int)((int64_t)c * ws / cs));
+          it.o1 = oa + (S.per > 0 ? std::min(ws, (c + 1) * S.per) : (int)((int64_t)(c + 1) * ws / cs));
           it.chunk = c;
           pass_items.emplace_back(wgt * (it.o1 - it.o0), it);
         }
@@ -446,68 +490,75 @@ void NBodySolver::ensure_sym_plan(int tpl, int nch, int h, bool ang) {
                        });
     for (const auto& pi : pass_items) items.push_back(pi.second);
     ps.nitems = (int)items.size() - ps.item0;
-    sym_.max_slabs = std::max(sym_.max_slabs, (size_t)(ps.nch + ps.diag + width));
-    sym_.passes.push_back(ps);
+    plan.max_slabs = std::max(plan.max_slabs, (size_t)(ps.nch + ps.diag + width));
+    plan.passes.push_back(ps);
     oa = ob;
   } while (oa <= h);
-  sym_.items.reserve(sizeof(SymItem) * std::max<size_t>(items.size(), 1));
-  sym_.sys.reserve(sizeof(SymSys) * systems.size());
-  sym_.rows.reserve(sizeof(SymRows) * rows.size());
-  LM_HIP(hipMemcpyAsync(sym_.items.as<void>(), items.data(), sizeof(SymItem) * items.size(),
+  plan.items.reserve(sizeof(SymItem) * std::max<size_t>(items.size(), 1));
+  plan.sys.reserve(sizeof(SymSys) * systems.size());
+  plan.rows.reserve(sizeof(SymRows) * rows.size());
+  LM_HIP(hipMemcpyAsync(plan.items.as<void>(), items.data(), sizeof(SymItem) * items.size(),
                         hipMemcpyHostToDevice, stream_));
-  LM_HIP(hipMemcpyAsync(sym_.sys.as<void>(), systems.data(), sizeof(SymSys) * systems.size(),
+  LM_HIP(hipMemcpyAsync(plan.sys.as<void>(), systems.data(), sizeof(SymSys) * systems.size(),
                         hipMemcpyHostToDevice, stream_));
-  LM_HIP(hipMemcpyAsync(sym_.rows.as<void>(), rows.data(), sizeof(SymRows) * rows.size(),
+  LM_HIP(hipMemcpyAsync(plan.rows.as<void>(), rows.data(), sizeof(SymRows) * rows.size(),
                         hipMemcpyHostToDevice, stream_));
   LM_HIP(hipStreamSynchronize(stream_));  // the host vectors go out of scope (items are kept)
-  sym_.host_items = std::move(items);
-  sym_.N = N_;
-  sym_.structure = struct_id_;
-  sym_.tpl = tpl;
-  sym_.nchunks = nch;
-  sym_.hmax = h;
-  sym_.ang = ang ? 1 : 0;
-  sym_.budget = sym_budget_;
-  sym_.nitems = (int)sym_.host_items.size();
-  sym_.nrows = (int)rows.size();
-  sym_.active_valid = false;
+  plan.host_items = std::move(items);
+  plan.N = N_;
+  plan.structure = struct_id_;
+  plan.tpl = tpl;
+  plan.waves = sh.waves;
+  plan.nchunks = nch;
+  plan.per = sh.per[0];
+  plan.hmax = h;
+  plan.ang = ang ? 1 : 0;
+  plan.budget = sym_budget_;
+  plan.nitems = (int)plan.host_items.size();
+  plan.nrows = (int)rows.size();
+  plan.active_valid = false;
 }
 
 // Per-system Lanczos: the items of the systems still iterating, pass by pass
 // (filtered from the plan's host list, already in launch order).
 void NBodySolver::build_sym_active(const int* act) {
-  sym_.active_valid = false;
-  if (sym_.N != N_ || sym_.structure != struct_id_ || sym_.host_items.empty()) return;
-  sym_.active_passes = sym_.passes;
-  sym_active_host_.reserve(sizeof(SymItem) * sym_.host_items.size());
+  // per-system recurrences: the plan their products use (any_open_: kept order)
+  SymPlan& plan = sym_plan_[any_open_ && !pre_on() ? 1 : 0];
+  plan.active_valid = false;
+  if (plan.N != N_ || plan.structure != struct_id_ || plan.host_items.empty()) return;
+  plan.active_passes = plan.passes;
+  sym_active_host_.reserve(sizeof(SymItem) * plan.host_items.size());
   SymItem* dst = sym_active_host_.as<SymItem>();
   int count = 0;
-  for (size_t p = 0; p < sym_.passes.size(); ++p) {
-    const SymPass& ps = sym_.passes[p];
-    sym_.active_passes[p].item0 = count;
+  for (size_t p = 0; p < plan.passes.size(); ++p) {
+    const SymPass& ps = plan.passes[p];
+    plan.active_passes[p].item0 = count;
     for (int k = ps.item0; k < ps.item0 + ps.nitems; ++k)
-      if (act[sym_.host_items[k].sys]) dst[count++] = sym_.host_items[k];
-    sym_.active_passes[p].nitems = count - sym_.active_passes[p].item0;
+      if (act[plan.host_items[k].sys]) dst[count++] = plan.host_items[k];
+    plan.active_passes[p].nitems = count - plan.active_passes[p].item0;
   }
   // the previous upload from the pinned buffer has completed: the caller
   // synchronised the stream after it
-  sym_.active_items.reserve(sizeof(SymItem) * std::max(count, 1));
+  plan.active_items.reserve(sizeof(SymItem) * std::max(count, 1));
   if (count > 0)
-    LM_HIP(hipMemcpyAsync(sym_.active_items.as<void>(), dst, sizeof(SymItem) * count,
+    LM_HIP(hipMemcpyAsync(plan.active_items.as<void>(), dst, sizeof(SymItem) * count,
                           hipMemcpyHostToDevice, stream_));
-  sym_.active_valid = true;
+  plan.active_valid = true;
 }
 
-void NBodySolver::run_sym(int tpl, int nch, int h, int blocks, bool fp32, const void* rec,
+void NBodySolver::run_sym(const SymShape& sh, int blocks, bool fp32, const void* rec,
                           const double* F, const double* T, double* U, double* W) {
   const bool ang = (blocks & (kWT | kWF)) != 0;
-  ensure_sym_plan(tpl, nch, h, ang);
-  const bool compact = pair_active_ != nullptr && sym_.active_valid;
-  const std::vector<SymPass>& passes = compact ? sym_.active_passes : sym_.passes;
-  const SymItem* items = compact ? sym_.active_items.as<SymItem>() : sym_.items.as<SymItem>();
+  ensure_sym_plan(sh, ang);
+  SymPlan& plan = sym();
+  last_sym_tpl_ = sh.tpl;
+  last_sym_chunks_ = sh.nch;
+  const bool compact = pair_active_ != nullptr && plan.active_valid;
+  const std::vector<SymPass>& passes = compact ? plan.active_passes : plan.passes;
+  const SymItem* items = compact ? plan.active_items.as<SymItem>() : plan.items.as<SymItem>();
   const int64_t n3 = 3 * N_;
-  part_u_.reserve(sizeof(double) * n3 * sym_.max_slabs);
-  if (ang) part_w_.reserve(sizeof(double) * n3 * sym_.max_slabs);
+  part_u_.reserve(sizeof(double) * n3 * plan.max_slabs);
+  if (ang) part_w_.reserve(sizeof(double) * n3 * plan.max_slabs);
   const int nsys = (int)sys_off_host_.size() - 1;
   for (size_t p = 0; p < passes.size(); ++p) {
     const SymPass& ps = passes[p];
@@ -518,8 +569,9 @@ void NBodySolver::run_sym(int tpl, int nch, int h, int blocks, bool fp32, const 
     double* slab_sw = ang ? slab_tw + (int64_t)nslab_t * n3 : nullptr;
     SymArgs a{};
     a.fp32 = fp32 ? 1 : 0;
-    a.tpl = tpl;
-    a.wall = nsys > 1 ? 2 : kind_code();
+    a.tpl = sh.tpl;
+    a.waves = sh.waves;
+    a.wall = sh.keep && nsys > 1 ? 2 : kind_code();
     a.blocks = blocks;
     a.pos = rec;
     a.F = F;
@@ -530,7 +582,7 @@ void NBodySolver::run_sym(int tpl, int nch, int h, int blocks, bool fp32, const 
     a.slab_sw = slab_sw;
     a.n3 = n3;
     a.obase = ps.oa;
-    a.sys = sym_.sys.as<SymSys>();
+    a.sys = plan.sys.as<SymSys>();
     a.items = items + ps.item0;
     a.nitems = ps.nitems;
     a.active = pair_active_;
@@ -538,7 +590,10 @@ void NBodySolver::run_sym(int tpl, int nch, int h, int blocks, bool fp32, const 
     a.t0 = t0_;
     a.rt0 = rt0_;
     a.r0 = r0_;
-    launch_pair_sym(a, stream_);
+    if (sh.keep)
+      launch_pair_sym(a, stream_);
+    else
+      launch_pair_sym_unit(a, stream_);
     SymReduceArgs r{};
     r.slab_t = slab_t;
     r.slab_s = slab_s;
@@ -548,10 +603,10 @@ void NBodySolver::run_sym(int tpl, int nch, int h, int blocks, bool fp32, const 
     r.o1 = ps.ob;
     r.diag = ps.diag;
     r.accumulate = p > 0 ? 1 : 0;
-    r.tpl = tpl;
-    r.sys = sym_.sys.as<SymSys>();
-    r.rows = sym_.rows.as<SymRows>();
-    r.nrows = sym_.nrows;
+    r.tile = 64 * sh.waves * sh.tpl;
+    r.sys = plan.sys.as<SymSys>();
+    r.rows = plan.rows.as<SymRows>();
+    r.nrows = plan.nrows;
     r.active = pair_active_;
     r.out = U;
     launch_sym_reduce(r, stream_);
@@ -567,7 +622,6 @@ void NBodySolver::run_sym(int tpl, int nch, int h, int blocks, bool fp32, const 
 void NBodySolver::launch_sym(int blocks, bool fp32, const void* rec, const double* F,
                              const double* T, double* U, double* W) {
   const int nsys = (int)sys_off_host_.size() - 1;
-  const bool special = kind_code() == 0 && blocks == kUF;
   const auto key = std::make_tuple(N_, fp32 ? 1 : 0, kind_code() + 4 * nsys, blocks);
   double pairs = 0.0;
   for (int s = 0; s < nsys; ++s) {
@@ -584,25 +638,24 @@ void NBodySolver::launch_sym(int blocks, bool fp32, const void* rec, const doubl
     float best = 1e30f;
     std::pair<int, int> pick{0, 0};
     std::vector<std::tuple<int, int, int>> seen;
-    for (int tr : {1, 2, 4})
+    for (int tr : {0, 1, 2, 4})
       for (int cr : {0, 16, 32, 64}) {
-        if (tr == 4 && !(special && nsys == 1)) continue;
-        int tpl, nch, nt, h;
-        sym_shape(special, tr, cr, tpl, nch, nt, h);
-        if (std::find(seen.begin(), seen.end(), std::make_tuple(tpl, nch, nt)) != seen.end())
-          continue;
-        seen.emplace_back(tpl, nch, nt);
-        run_sym(tpl, nch, h, blocks, fp32, rec, F, T, U, W);
+        const SymShape sh = sym_shape(blocks, fp32, tr, cr);
+        if (tr != 0 && sh.tpl != tr) continue;  // clamped
+        const auto id = std::make_tuple(sh.tpl, sh.nch, sh.ntiles);
+        if (std::find(seen.begin(), seen.end(), id) != seen.end()) continue;
+        seen.push_back(id);
+        run_sym(sh, blocks, fp32, rec, F, T, U, W);
         LM_HIP(hipEventRecord(e0, stream_));
-        run_sym(tpl, nch, h, blocks, fp32, rec, F, T, U, W);
-        run_sym(tpl, nch, h, blocks, fp32, rec, F, T, U, W);
+        run_sym(sh, blocks, fp32, rec, F, T, U, W);
+        run_sym(sh, blocks, fp32, rec, F, T, U, W);
         LM_HIP(hipEventRecord(e1, stream_));
         LM_HIP(hipEventSynchronize(e1));
         float ms = 0.f;
         LM_HIP(hipEventElapsedTime(&ms, e0, e1));
         if (ms < best) {
           best = ms;
-          pick = {tpl, nch};
+          pick = {tr, cr};
         }
       }
     (void)hipEventDestroy(e0);
@@ -617,9 +670,7 @@ void NBodySolver::launch_sym(int blocks, bool fp32, const void* rec, const doubl
       cr = it->second.second;
     }
   }
-  int tpl, nch, nt, h;
-  sym_shape(special, tr, cr, tpl, nch, nt, h);
-  run_sym(tpl, nch, h, blocks, fp32, rec, F, T, U, W);
+  run_sym(sym_shape(blocks, fp32, tr, cr), blocks, fp32, rec, F, T, U, W);
 }
 
 double NBodySolver::mean_system_size() {
@@ -930,7 +981,7 @@ void NBodySolver::pair_product(const void* rec64, const void* rec32, const doubl
   last_sym_ = false;
   last_wide_ = false;
   deferred_nch_ = 0;
-  if (use_sym(blocks)) {
+  if (use_sym(blocks, fp32)) {
     launch_sym(blocks, fp32, rec, F, T, U, W);
     last_sym_ = true;
   } else if (use_wide()) {
@@ -1287,10 +1338,7 @@ void NBodySolver::lanczos_product(const double* v, double* w) {
                  angular_ ? u + N3 : nullptr);
     pre_back(u, w, n);
   } else {
-    struct OrderGuard {
-      bool& f;
-      ~OrderGuard() { f = false; }
-    } guard{keep_order_};
+    OrderGuard guard{keep_order_};
     keep_order_ = any_open_;
     pair_product(rec64_.as<void>(), rec32_.as<void>(), v, angular_ ? v + N3 : nullptr, w,
                  angular_ ? w + N3 : nullptr);
@@ -1432,7 +1480,7 @@ int NBodySolver::lanczos_run_seg(SegSolve& S, const std::vector<int64_t>& off, b
       s.pair_active_ = nullptr;
       s.seg_blocks_ = nullptr;
       s.seg_items_.count = 0;
-      s.sym_.active_valid = false;
+      s.sym_plan_[0].active_valid = s.sym_plan_[1].active_valid = false;
     }
   } guard{*this};
   if (skip_converged_pairs) {
@@ -1665,6 +1713,8 @@ void NBodySolver::multi_product(const double* v, int nrhs, double* w) {
     mdot_multi_dev(t, nrhs, u);
     for (int r = 0; r < nrhs; ++r) pre_back(u + r * n3, w + r * n3, n3);
   } else {
+    OrderGuard guard{keep_order_};
+    keep_order_ = any_open_;
     mdot_multi_dev(v, nrhs, w);
   }
 }

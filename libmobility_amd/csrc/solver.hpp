@@ -102,24 +102,41 @@ class NBodySolver {
   // The symmetric path reports its targets per lane and offset chunks, the
   // wide kernel its targets per unit of work and one chunk.
   void lastPairTiling(int* tpl, int* nch) const {
-    *tpl = last_sym_ ? sym_.tpl : (last_wide_ ? kWideTargets : items_tpl_);
-    *nch = last_sym_ ? sym_.nchunks : (last_wide_ ? 1 : items_nch_);
+    *tpl = last_sym_ ? last_sym_tpl_ : (last_wide_ ? kWideTargets : items_tpl_);
+    *nch = last_sym_ ? last_sym_chunks_ : (last_wide_ ? 1 : items_nch_);
   }
   // Symmetric evaluation of one open or single-wall system, any block set
-  // (-1 auto: from N = kSymAutoN; 0 off; 1 on).
+  // (-1 auto; 0 off; 1 on).
   void setPairSymmetric(int mode);
-  // Particles (in total) from which the automatic mode evaluates each
-  // unordered pair once: from 16384 it was 1.10-1.37x faster than the ordered
-  // evaluation (open UF and wall 6x6, FP32 and FP64); at 8192 equal or slower.
-  // Ensembles also need a mean system size (of the system that the average
-  // particle is in) above kSymAutoMean: 60000 particles in systems of 1500
-  // take 58-555 us with sources across the lanes and 60-590 us symmetric; in
-  // systems of 800, 36-304 us and 60-580 us; of 3000, 106-1100 us and 100-1070 us.
-  static constexpr int64_t kSymAutoN = 16384;
-  static constexpr double kSymAutoMean = 2048;
+  // Mean system size (of the system that the average particle is in) from which
+  // the automatic mode evaluates each unordered pair once; below, sources go
+  // across the lanes.  Microseconds per call, ordered / symmetric:
+  //   wall UF    FP64 3000: 63 / 66, 4096: 85 / 77, 8192: 254 / 172
+  //              FP32 4096: 58 / 56, 8192: 155 / 110
+  //   wall 6x6   FP64 3000: 90 / 104, 4096: 129 / 125, 8192: 412 / 315
+  //              FP32 4096: 89 / 93, 6000: 151 / 139, 8192: 248 / 192
+  //   open UF    FP64 6000: 67 / 68, 8192: 100 / 90, 16384: 301 / 242
+  //              FP32 8192: 67 / 66, 12288: 116 / 105, 16384: 188 / 148
+  //   open 6x6   FP64 8192: 177 / 175, 16384: 572 / 535
+  //              FP32 8192: 115 / 123, 16384: 363 / 343
+  static constexpr double kSymWallN = 4096, kSymOpenN = 8192, kSymOpenFp32N = 16384;
+  // Ensembles of at least kSymKeepN particles fill the chip whatever the size
+  // of their systems: mean size 3900 (96 systems of 64 to 8192, half with a
+  // wall) 925 / 617 us FP32 UF, 2990 / 2050 FP64 6x6; mean size 1100 equal.
+  static constexpr double kSymEnsembleMean = 1500;
+  // Products that keep their order (keep_order_): particles in total.
+  static constexpr int64_t kSymKeepN = 16384;
+  // One wave per workgroup (tiles of 64) below this size, four (tiles of 256)
+  // from it: FP64 wall 6x6 at 8192 276 / 331 us, at 16384 1027 / 1042, at 32768
+  // 4138 / 4026; FP32 wall 6x6 163 / 194, 613 / 603, 2296 / 2116.  Two targets
+  // per lane for open systems from kSymTwoN: FP64 UF at 32768 813 / 779 us, 6x6
+  // 1780 / 1691, FP32 6x6 1020 / 968; below equal or slower, and with a wall
+  // slower at any size (FP32 wall 6x6 at 65536 8641 / 9648: registers).
+  static constexpr double kSymWaveN = 16384, kSymTwoN = 32768;
   // Mean system size up to which the ordered evaluation puts sources across
-  // the lanes (wide_kernels.hip has both sides' times; equal from about 8000).
-  static constexpr double kWideMaxSize = 8192;
+  // the lanes (wide_kernels.hip has both sides' times; equal from about 8000, and
+  // above only open angular FP32 products get there).
+  static constexpr double kWideMaxSize = 16384;
   // Units of work from which each is one wave instead of a workgroup of four
   // (which then only adds the waves' sums and a barrier): 20000 particles in
   // systems of 256, open UF FP64, take 11.1 us with one wave per unit and 14.8
@@ -355,7 +372,7 @@ class NBodySolver {
   struct SymPlan {
     DevBuf items, sys, rows, active_items;
     std::vector<SymItem> host_items;  // all passes, in launch order
-    int tpl = 0, nchunks = 0, hmax = 0, nitems = 0, nrows = 0, ang = -1;
+    int tpl = 0, waves = 0, nchunks = 0, per = 0, hmax = 0, nitems = 0, nrows = 0, ang = -1;
     int64_t N = -1, budget = 0;
     uint64_t structure = 0;
     std::vector<SymPass> passes, active_passes;
@@ -364,18 +381,25 @@ class NBodySolver {
   };
   static constexpr int64_t kDefaultSymBudget = (int64_t)4 << 30;
   int64_t sym_budget_ = kDefaultSymBudget;
-  SymPlan sym_;
+  // [1]: the plan of products that keep their order (keep_order_)
+  SymPlan sym_plan_[2];
+  SymPlan& sym() { return sym_plan_[keep_order_ ? 1 : 0]; }
+  int last_sym_tpl_ = 0, last_sym_chunks_ = 0;
   HostBuf sym_active_host_;
   int sym_mode_ = -1;
   bool last_sym_ = false;
   // (N, fp32, kind + 4 * systems, blocks) -> (targets per lane, offset chunks)
   std::map<std::tuple<int64_t, int, int, int>, std::pair<int, int>> sym_tuned_;
-  void sym_shape(bool special, int tpl_req, int nch_req, int& tpl, int& nch, int& ntiles,
-                 int& hmax) const;
-  bool use_sym(int blocks);
-  void ensure_sym_plan(int tpl, int nch, int h, bool ang);
+  struct SymShape {
+    int tpl = 1, waves = 4, nch = 0, ntiles = 0, hmax = 0;
+    int per[2] = {0, 0};  // offsets per item of open and wall systems (0: from nch)
+    bool keep = false;  // launch_pair_sym, else launch_pair_sym_unit
+  };
+  SymShape sym_shape(int blocks, bool fp32, int tpl_req, int nch_req);
+  bool use_sym(int blocks, bool fp32);
+  void ensure_sym_plan(const SymShape& sh, bool ang);
   void build_sym_active(const int* act);
-  void run_sym(int tpl, int nch, int h, int blocks, bool fp32, const void* rec, const double* F,
+  void run_sym(const SymShape& sh, int blocks, bool fp32, const void* rec, const double* F,
                const double* T, double* U, double* W);
   void launch_sym(int blocks, bool fp32, const void* rec, const double* F, const double* T,
                   double* U, double* W);
@@ -396,7 +420,7 @@ class NBodySolver {
   int64_t mean_size_N_ = -1;
   bool use_wide();
   // Products of a plain Lanczos recurrence over open systems: the summation
-  // order stays that of k_pair's chunks (k_pair_sym from kSymAutoN).  There the
+  // order stays that of k_pair's chunks (k_pair_sym from kSymKeepN).  There the
   // largest Ritz values converge to rounding within about 15 iterations, the
   // recurrence loses its orthogonality, and from then on a change in the last
   // bit grows some 200 times per iteration: at a tolerance of 1e-4 another
@@ -405,6 +429,10 @@ class NBodySolver {
   // being nearer to M^{1/2} W.  Above a wall and with the preconditioner the
   // same comparison gives 1e-15 to 1e-13 (FP64) and 1e-7 to 1e-6 (FP32).
   bool keep_order_ = false;
+  struct OrderGuard {
+    bool& f;
+    ~OrderGuard() { f = false; }
+  };
   void ensure_wide_plan();
   void launch_wide(int blocks, bool fp32, const void* rec, const double* F, const double* T,
                    double* U, double* W);

@@ -94,76 +94,72 @@ __device__ inline void wide_sources(const typename Rec<R>::T* __restrict__ pos,
   constexpr bool kNeedF = (BLK & (kUF | kWF)) != 0;
   constexpr bool kNeedT = (BLK & (kUT | kWT)) != 0;
   constexpr bool kAngular = (BLK & (kWT | kWF)) != 0;
-  constexpr bool kUF34 = !WALL && BLK == kUF;  // coefficients times 4/3 (rpy_far_uf34)
-  constexpr int G = T < 4 ? T : 4;             // pairs per overlap test
+  constexpr int G = T < 4 ? T : 4;  // pairs per overlap test
   const int lane = threadIdx.x & 63;
+  const Vec3<R> zero = {R(0), R(0), R(0)};
   R4 pi[T];  // uniform: scalar loads
 #pragma unroll
   for (int t = 0; t < T; ++t) pi[t] = pos[tgt0 + (t < ntgt ? t : ntgt - 1)];
-  PairAcc<R> acc[T];
+  Vec3<R> u[T], w[T], none = zero;
 #pragma unroll
-  for (int t = 0; t < T; ++t) acc_zero(acc[t]);
+  for (int t = 0; t < T; ++t) u[t] = w[t] = zero;
+  const R ta = R(r0 / rt0);  // 1/a: symmetric units (pair_math.hpp)
   for (; base < src1; base += 64 * (int64_t)stride) {
     const int64_t j = base + lane;
     R4 pj = far_record<R4>();
-    Vec3<R> fj = {R(0), R(0), R(0)}, tj = {R(0), R(0), R(0)};
+    Vec3<R> fj = zero, tj = zero;
     if (j < src1) {
       pj = pos[j];
-      if (kNeedF) fj = {R(F[3 * j]), R(F[3 * j + 1]), R(F[3 * j + 2])};
-      if (kNeedT) tj = {R(Tq[3 * j]), R(Tq[3 * j + 1]), R(Tq[3 * j + 2])};
+      const R b = WALL ? pj.w : R(1);  // the wall's damping goes with the force
+      if (kNeedF) fj = {b * R(F[3 * j]), b * R(F[3 * j + 1]), b * R(F[3 * j + 2])};
+      const R bt = b * ta;
+      if (kNeedT) tj = {bt * R(Tq[3 * j]), bt * R(Tq[3 * j + 1]), bt * R(Tq[3 * j + 2])};
     }
     if constexpr (WALL) {
 #pragma unroll
-      for (int t = 0; t < T; ++t)
-        wall_pair<R, BLK>(pi[t].x, pi[t].y, pi[t].z, pi[t].w, pj.x, pj.y, pj.z, pj.w, fj.x, fj.y,
-                          fj.z, tj.x, tj.y, tj.z, acc[t]);
+      for (int t = 0; t < T; ++t) {
+        PairGeo<R> g;
+        pair_distances<R, true>(pi[t].x, pi[t].y, pi[t].z, pj.x, pj.y, pj.z, g);
+        pair_inverses<R, true>(g);
+        pair_unit<R, true, BLK, false>(g, pj.z, fj, tj, zero, zero, u[t], w[t], none, none);
+      }
     } else {
 #pragma unroll
       for (int g = 0; g < T; g += G) {
-        R dx[G], dy[G], dz[G], r2[G], ir[G];
+        PairGeo<R> q[G];
         RpyCoef<R> cf[G];
         NearTestCmp<R> near;
 #pragma unroll
         for (int t = 0; t < G; ++t) {
-          dx[t] = pi[g + t].x - pj.x;
-          dy[t] = pi[g + t].y - pj.y;
-          dz[t] = pi[g + t].z - pj.z;
-          r2[t] = dx[t] * dx[t] + dy[t] * dy[t] + dz[t] * dz[t];
-          ir[t] = lm_rsqrt(r2[t]);
+          pair_distances<R, false>(pi[g + t].x, pi[g + t].y, pi[g + t].z, pj.x, pj.y, pj.z, q[t]);
+          pair_inverses<R, false>(q[t]);
           cf[t] = RpyCoef<R>{};
-          if constexpr (kUF34)
-            rpy_far_uf34<R>(ir[t], cf[t]);
-          else
-            rpy_far<R, BLK>(ir[t], cf[t]);
-          near.add(r2[t]);
+          rpy_unit_far<R, BLK>(q[t].ir, cf[t]);
+          near.add(q[t].r2);
         }
         if (__builtin_expect(near.hit(), 0)) {
           lm_rare_path();
 #pragma unroll
-          for (int t = 0; t < G; ++t) {
-            if constexpr (kUF34)
-              rpy_near_select_uf34<R>(r2[t], ir[t], cf[t]);
-            else
-              rpy_near_select<R, BLK>(r2[t], ir[t], cf[t]);
-          }
+          for (int t = 0; t < G; ++t) rpy_unit_near_select<R, BLK>(q[t].r2, q[t].ir, cf[t]);
         }
 #pragma unroll
         for (int t = 0; t < G; ++t)
-          open_accumulate<R, BLK>(dx[t], dy[t], dz[t], fj.x, fj.y, fj.z, tj.x, tj.y, tj.z, cf[t],
-                                  acc[g + t]);
+          open_unit<R, BLK, false>(q[t].dx, q[t].dy, q[t].dz, cf[t], fj, tj, zero, zero, u[g + t],
+                                   w[g + t], none, none);
       }
     }
   }
-  const double tuf = kUF34 ? 0.75 * t0 : t0;
 #pragma unroll
   for (int t = 0; t < T; ++t) {
-    v[3 * t + 0] = tuf * (double)acc[t].uf.x + rt0 * (double)acc[t].ut.x;
-    v[3 * t + 1] = tuf * (double)acc[t].uf.y + rt0 * (double)acc[t].ut.y;
-    v[3 * t + 2] = tuf * (double)acc[t].uf.z + rt0 * (double)acc[t].ut.z;
+    const double b = WALL ? (double)pi[t].w : 1.0;
+    const double us = 0.75 * t0 * b, ws = rt0 * b;
+    v[3 * t + 0] = us * (double)u[t].x;
+    v[3 * t + 1] = us * (double)u[t].y;
+    v[3 * t + 2] = us * (double)u[t].z;
     if constexpr (kAngular) {
-      v[3 * T + 3 * t + 0] = r0 * (double)acc[t].wt.x + rt0 * (double)acc[t].wf.x;
-      v[3 * T + 3 * t + 1] = r0 * (double)acc[t].wt.y + rt0 * (double)acc[t].wf.y;
-      v[3 * T + 3 * t + 2] = r0 * (double)acc[t].wt.z + rt0 * (double)acc[t].wf.z;
+      v[3 * T + 3 * t + 0] = ws * (double)w[t].x;
+      v[3 * T + 3 * t + 1] = ws * (double)w[t].y;
+      v[3 * T + 3 * t + 2] = ws * (double)w[t].z;
     }
   }
 }
