@@ -194,8 +194,8 @@ void launch_zero_open_systems(double* v, int64_t N, const int64_t* sys_off, int 
 // Normal(0,1) samples from Philox4x32-10 + Box-Muller: out[k], k < n.
 void launch_normal_fill(double* out, int64_t n, uint64_t seed, uint64_t stream, hipStream_t s);
 
-// Scratch for the single-pass reductions: partial sums + a self-resetting
-// arrival counter.  kReduceBlocks partials per reduction slot (measured: a
+// Scratch for the single-pass reductions of the checks: partial sums + a
+// self-resetting arrival counter.  kReduceBlocks partials per reduction slot (measured: a
 // wider grid costs more in contention on the arrival counter than it gains
 // in memory parallelism at n ~ 4e5).
 constexpr int kReduceBlocks = 256;
@@ -236,9 +236,9 @@ struct LanczosScalars {
 };
 
 // ||z|| and v0 = z / ||z||; resets the status (previous estimate in slot `old`)
-void launch_lanczos_start(const double* z, double* v0, int64_t n, ReduceScratch rs,
+void launch_lanczos_start(const double* z, double* v0, int64_t n, double* partial,
                           LanczosScalars* sc, int old, hipStream_t s);
-// One Lanczos step after the product, in one launch (n <= kLanczosFusedMaxN):
+// One Lanczos step after the product, in one or two launches (n <= kLanczosFusedMaxN):
 // w = M v_i (from `w`, or summed over the nch source-chunk slabs of the pair
 // kernel: entries k < n3 from slab_u, the rest from slab_w); w -= beta[i-1]
 // v_prev; alpha[i] = w . v_i; w -= alpha[i] v_i; beta[i] = ||w|| with the
@@ -258,10 +258,8 @@ struct LanczosStepArgs {
   double* v_next;
   double* w_out;
   double* partial;
-  unsigned int* counter;
-  // a workgroup that finds *stop != 0 when it starts skips the arithmetic
-  // (the step is past convergence; its outputs are then undefined) but still
-  // takes part in the arrival count (nullptr: never)
+  // a workgroup that finds *stop != 0 when it starts does nothing (the step is
+  // past convergence; its outputs are then undefined; nullptr: never)
   const int* stop;
   int64_t n;
   int i;
@@ -277,15 +275,12 @@ void launch_lanczos_step(const LanczosStepArgs& a, hipStream_t s);
 // rest.
 void launch_lanczos_reorth(const double* V, int64_t ldv, int i, int64_t n, double* partial,
                            unsigned int* counter, double* c, LanczosScalars* sc, hipStream_t s);
-// w -= beta[i-1] v_prev (if i > 0); alpha[i] = w . v_i
-void launch_lanczos_alpha(double* w, const double* v_i, const double* v_prev, int64_t n, int i,
-                          ReduceScratch rs, LanczosScalars* sc, hipStream_t s);
-// w -= alpha[i] v_i; beta[i] = ||w|| with the breakdown rule
-void launch_lanczos_beta(double* w, const double* v_i, int64_t n, int i, ReduceScratch rs,
-                         LanczosScalars* sc, hipStream_t s);
-// v_next = w / beta[i], or e1 after breakdown
-void launch_lanczos_next(const double* w, double* v_next, int64_t n, int i,
-                         const LanczosScalars* sc, hipStream_t s);
+// The step for longer vectors, in three launches: w -= beta[i-1] v_prev (if i >
+// 0), alpha[i] = w . v_i; w -= alpha[i] v_i, beta[i] = ||w|| with the breakdown
+// rule; v_next = w / beta[i], or e1 after a breakdown.  `partial` holds 2 *
+// kReduceBlocks doubles.
+void launch_lanczos_update(double* w, const double* v_i, const double* v_prev, double* v_next,
+                           int64_t n, int i, double* partial, LanczosScalars* sc, hipStream_t s);
 // s[0..m) = T_m^{1/2} e1 (FP64, one workgroup); work has tsqrt_scratch(m) doubles
 constexpr int kTsqrtNodes = 512;
 constexpr int64_t tsqrt_scratch(int m) { return (int64_t)m * (kTsqrtNodes + kTsqrtNodes / 64); }

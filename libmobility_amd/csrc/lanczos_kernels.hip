@@ -3,10 +3,11 @@
 //
 // Everything stays on the device: the Krylov basis V (column-major, n x m),
 // the three-term recurrence scalars alpha/beta, the tridiagonal square root
-// and the convergence estimate.  Reductions are single pass: each block
-// writes a partial, the last block to arrive (agent-scope counter that it
-// resets itself) sums the partials in a fixed order, so results are bitwise
-// reproducible and no host round trip is needed until the convergence test.
+// and the convergence estimate.  Every reduction adds per-block partials in a
+// fixed order, so results are bitwise reproducible and no host round trip is
+// needed until the convergence test: those of the recurrence in the launch
+// that follows, those of the checks in the last block to arrive (agent-scope
+// counter that it resets itself).
 //
 // Tridiagonal square root (replaces host LAPACKE ?steqr + cblas ?gemv,
 // LanczosAlgorithm.cu:48-85): for the SPD tridiagonal T,
@@ -22,6 +23,7 @@
 #include <cmath>
 
 #include "kernels.hpp"
+#include "lane_sums.hpp"
 #include "lm_common.hpp"
 #include "philox.hpp"
 
@@ -62,14 +64,13 @@ constexpr int kRT = 256;  // threads per reduction block
 
 // Sum over the block; the result is valid in every thread of wave 0.
 __device__ inline double block_sum(double v, double* sh) {
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+  v = wave_sum(v);
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   __syncthreads();
   if (lane == 0) sh[wid] = v;
   __syncthreads();
   double t = (threadIdx.x < (blockDim.x >> 6)) ? sh[threadIdx.x] : 0.0;
-  if (wid == 0)
-    for (int o = 32; o > 0; o >>= 1) t += __shfl_xor(t, o);
+  if (wid == 0) t = wave_sum(t);
   return t;
 }
 
@@ -110,56 +111,71 @@ static inline int reduce_blocks(int64_t n) {
 }
 
 // ---- Lanczos steps ------------------------------------------------------------
-// ||z|| -> sc->normz
+// The reductions of one step end in the next launch: each block writes its
+// partial sum, and every block of the launch that needs the total adds all
+// partials itself, in one fixed order (at most kReduceBlocks loads that hit the
+// L2).  The launch boundary orders them; with an arrival counter in the
+// reducing launch instead, its agent-scope fences cost 5-7 us each (three
+// launches per step at 60000 entries: 29 us with counters, 15 us without).
+
+// Fixed-order sum of the nb partials, in every thread of the block.
+__device__ inline double sum_partials(const double* __restrict__ partial, int nb, double* sh) {
+  double v = 0.0;
+  for (int b = threadIdx.x; b < nb; b += blockDim.x) v += partial[b];
+  v = block_sum(v, sh);
+  __shared__ double s_total;
+  if (threadIdx.x == 0) s_total = v;
+  __syncthreads();
+  return s_total;
+}
+
 __global__ __launch_bounds__(kRT) void k_norm_start(const double* __restrict__ z, int64_t n,
-                                                   double* partial, unsigned* counter,
-                                                   LanczosScalars* sc, int old) {
+                                                   double* partial) {
   __shared__ double sh[kRT / 64];
   double v = 0.0;
   for (int64_t i = (int64_t)blockIdx.x * kRT + threadIdx.x; i < n; i += (int64_t)gridDim.x * kRT)
     v += z[i] * z[i];
   v = block_sum(v, sh);
-  if (publish_and_arrive(partial, 1, &v, counter)) {
-    const double t = gather_partials(partial, 0, gridDim.x, sh);
-    if (threadIdx.x == 0) {
-      sc->normz = sqrt(t);
-      LanczosStatus st{};
-      st.conv = 0;
-      st.conv_iter = -1;
-      st.old = old;
-      st.result = -1;
-      st.first = -1;
-      st.nchk = 0;
-      sc->status = st;
-      *counter = 0;
-    }
-  }
+  if (threadIdx.x == 0) partial[blockIdx.x] = v;
 }
 
-__global__ void k_scale_start(const double* __restrict__ z, double* __restrict__ v0, int64_t n,
-                              const LanczosScalars* sc) {
-  const double inv = 1.0 / sc->normz;  // LanczosAlgorithm.cu:115-117
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x)
+// ||z|| -> sc->normz, v0 = z / ||z|| (LanczosAlgorithm.cu:110-118)
+__global__ __launch_bounds__(kRT) void k_scale_start(const double* __restrict__ z,
+                                                    double* __restrict__ v0, int64_t n,
+                                                    const double* __restrict__ partial,
+                                                    LanczosScalars* sc, int old) {
+  __shared__ double sh[kRT / 64];
+  const double normz = sqrt(sum_partials(partial, gridDim.x, sh));
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    sc->normz = normz;
+    LanczosStatus st{};
+    st.conv = 0;
+    st.conv_iter = -1;
+    st.old = old;
+    st.result = -1;
+    st.first = -1;
+    st.nchk = 0;
+    sc->status = st;
+  }
+  const double inv = 1.0 / normz;
+  for (int64_t i = (int64_t)blockIdx.x * kRT + threadIdx.x; i < n; i += (int64_t)gridDim.x * kRT)
     v0[i] = z[i] * inv;
 }
 
-void launch_lanczos_start(const double* z, double* v0, int64_t n, ReduceScratch rs,
+void launch_lanczos_start(const double* z, double* v0, int64_t n, double* partial,
                           LanczosScalars* sc, int old, hipStream_t s) {
   const int nb = reduce_blocks(n);
-  hipLaunchKernelGGL(k_norm_start, dim3(nb), dim3(kRT), 0, s, z, n, rs.partial, rs.counter, sc,
-                     old);
+  hipLaunchKernelGGL(k_norm_start, dim3(nb), dim3(kRT), 0, s, z, n, partial);
   LM_HIP(hipGetLastError());
-  hipLaunchKernelGGL(k_scale_start, dim3(nb), dim3(kRT), 0, s, z, v0, n, sc);
+  hipLaunchKernelGGL(k_scale_start, dim3(nb), dim3(kRT), 0, s, z, v0, n, partial, sc, old);
   LM_HIP(hipGetLastError());
 }
 
-// w -= beta[i-1] v_prev ; alpha[i] = w . v_i   (LanczosAlgorithm.cu:128-134)
+// w -= beta[i-1] v_prev; partials of alpha[i] = w . v_i   (LanczosAlgorithm.cu:128-134)
 __global__ __launch_bounds__(kRT) void k_alpha(double* __restrict__ w,
                                               const double* __restrict__ vi,
                                               const double* __restrict__ vp, int64_t n, int i,
-                                              double* partial, unsigned* counter,
-                                              LanczosScalars* sc) {
+                                              double* partial, const LanczosScalars* sc) {
   __shared__ double sh[kRT / 64];
   const double b = (i > 0) ? sc->beta[i - 1] : 0.0;
   double v = 0.0;
@@ -172,30 +188,17 @@ __global__ __launch_bounds__(kRT) void k_alpha(double* __restrict__ w,
     v += wk * vi[k];
   }
   v = block_sum(v, sh);
-  if (publish_and_arrive(partial, 1, &v, counter)) {
-    const double t = gather_partials(partial, 0, gridDim.x, sh);
-    if (threadIdx.x == 0) {
-      sc->alpha[i] = t;
-      *counter = 0;
-    }
-  }
+  if (threadIdx.x == 0) partial[blockIdx.x] = v;
 }
 
-void launch_lanczos_alpha(double* w, const double* v_i, const double* v_prev, int64_t n, int i,
-                          ReduceScratch rs, LanczosScalars* sc, hipStream_t s) {
-  hipLaunchKernelGGL(k_alpha, dim3(reduce_blocks(n)), dim3(kRT), 0, s, w, v_i, v_prev, n, i,
-                     rs.partial, rs.counter, sc);
-  LM_HIP(hipGetLastError());
-}
-
-// w -= alpha[i] v_i ; beta[i] = ||w||, zeroed below 1e-3 alpha/||z||
-// (LanczosAlgorithm.cu:136-143)
+// alpha[i]; w -= alpha[i] v_i; partials of ||w||^2 (LanczosAlgorithm.cu:134-138)
 __global__ __launch_bounds__(kRT) void k_beta(double* __restrict__ w,
                                              const double* __restrict__ vi, int64_t n, int i,
-                                             double* partial, unsigned* counter,
-                                             LanczosScalars* sc) {
+                                             const double* __restrict__ partial_a,
+                                             double* partial_b, LanczosScalars* sc) {
   __shared__ double sh[kRT / 64];
-  const double al = sc->alpha[i];
+  const double al = sum_partials(partial_a, gridDim.x, sh);
+  if (blockIdx.x == 0 && threadIdx.x == 0) sc->alpha[i] = al;
   double v = 0.0;
   for (int64_t k = (int64_t)blockIdx.x * kRT + threadIdx.x; k < n; k += (int64_t)gridDim.x * kRT) {
     const double wk = w[k] - al * vi[k];
@@ -203,79 +206,69 @@ __global__ __launch_bounds__(kRT) void k_beta(double* __restrict__ w,
     v += wk * wk;
   }
   v = block_sum(v, sh);
-  if (publish_and_arrive(partial, 1, &v, counter)) {
-    const double t = gather_partials(partial, 0, gridDim.x, sh);
-    if (threadIdx.x == 0) {
-      double be = sqrt(t);
-      const double tol = 1e-3 * sc->alpha[i] / sc->normz;
-      if (be < tol) be = 0.0;
-      sc->beta[i] = be;
-      *counter = 0;
-    }
-  }
+  if (threadIdx.x == 0) partial_b[blockIdx.x] = v;
 }
 
-void launch_lanczos_beta(double* w, const double* v_i, int64_t n, int i, ReduceScratch rs,
-                         LanczosScalars* sc, hipStream_t s) {
-  hipLaunchKernelGGL(k_beta, dim3(reduce_blocks(n)), dim3(kRT), 0, s, w, v_i, n, i, rs.partial,
-                     rs.counter, sc);
-  LM_HIP(hipGetLastError());
-}
-
-// v_{i+1} = w / beta[i], or e1 after a breakdown (LanczosAlgorithm.cu:144-152)
-__global__ void k_next(const double* __restrict__ w, double* __restrict__ vn, int64_t n, int i,
-                       const LanczosScalars* sc) {
-  const double be = sc->beta[i];
+// beta[i] = ||w||, zeroed below 1e-3 alpha/||z||; v_{i+1} = w / beta[i], or e1
+// after a breakdown (LanczosAlgorithm.cu:138-152)
+__global__ __launch_bounds__(kRT) void k_next(const double* __restrict__ w,
+                                             double* __restrict__ vn, int64_t n, int i,
+                                             const double* __restrict__ partial_b,
+                                             LanczosScalars* sc) {
+  __shared__ double sh[kRT / 64];
+  double be = sqrt(sum_partials(partial_b, gridDim.x, sh));
+  if (be < 1e-3 * sc->alpha[i] / sc->normz) be = 0.0;
+  if (blockIdx.x == 0 && threadIdx.x == 0) sc->beta[i] = be;
   const double inv = be > 0.0 ? 1.0 / be : 0.0;
-  for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < n;
-       k += (int64_t)gridDim.x * blockDim.x)
+  for (int64_t k = (int64_t)blockIdx.x * kRT + threadIdx.x; k < n; k += (int64_t)gridDim.x * kRT)
     vn[k] = be > 0.0 ? w[k] * inv : (k == 0 ? 1.0 : 0.0);
 }
 
-void launch_lanczos_next(const double* w, double* v_next, int64_t n, int i,
-                         const LanczosScalars* sc, hipStream_t s) {
-  hipLaunchKernelGGL(k_next, dim3(reduce_blocks(n)), dim3(kRT), 0, s, w, v_next, n, i, sc);
+void launch_lanczos_update(double* w, const double* v_i, const double* v_prev, double* v_next,
+                           int64_t n, int i, double* partial, LanczosScalars* sc, hipStream_t s) {
+  const dim3 grid(reduce_blocks(n)), block(kRT);
+  double* pa = partial;
+  double* pb = partial + kReduceBlocks;
+  hipLaunchKernelGGL(k_alpha, grid, block, 0, s, w, v_i, v_prev, n, i, pa, sc);
+  LM_HIP(hipGetLastError());
+  hipLaunchKernelGGL(k_beta, grid, block, 0, s, w, v_i, n, i, pa, pb, sc);
+  LM_HIP(hipGetLastError());
+  hipLaunchKernelGGL(k_next, grid, block, 0, s, w, v_next, n, i, pb, sc);
   LM_HIP(hipGetLastError());
 }
 
-// Sum over a workgroup of kLanczosFusedThreads in a fixed order; every thread
-// gets the total.  `sh` holds one double per wave plus one.
+// Sum over a workgroup of kLanczosFusedThreads in a fixed order, in every
+// thread; `sh` holds one double per wave and is not reused.
+constexpr int kFusedWaves = kLanczosFusedThreads / 64;
 __device__ inline double group_sum_all(double v, double* sh) {
-  constexpr int kW = kLanczosFusedThreads / 64;
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  if (lane == 0) sh[wid] = v;
+  v = wave_sum(v);
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    double t = 0.0;
-    for (int k = 0; k < kW; ++k) t += sh[k];
-    sh[kW] = t;
-  }
-  __syncthreads();
-  const double t = sh[kW];
-  __syncthreads();  // sh is reused by the next sum
+  double t = 0.0;
+#pragma unroll
+  for (int k = 0; k < kFusedWaves; ++k) t += sh[k];
   return t;
 }
 
-// The step of LanczosAlgorithm.cu:128-152 in one launch.  Every workgroup
+// The step of LanczosAlgorithm.cu:128-152 in two launches: every workgroup
 // forms its entries of w = M v_i (summing the chunk slabs) - beta[i-1]
-// v_{i-1}, stores them and publishes its part of alpha = w . v_i; the last
-// workgroup to arrive finishes alone (the vectors are short): w -= alpha v_i,
-// beta = ||w|| with the breakdown rule, v_next = w / beta or e1.
+// v_{i-1}, stores them and its part of alpha = w . v_i; one workgroup then
+// finishes (the vectors are short): w -= alpha v_i, beta = ||w|| with the
+// breakdown rule, v_next = w / beta or e1.  As one launch whose last workgroup
+// to arrive finished, its two agent-scope fences cost more than the second
+// launch: 13.6 us against 4.6 + 7.5 us at 12000 entries.
 __global__ __launch_bounds__(kLanczosFusedThreads) void k_lanczos_step(LanczosStepArgs a) {
-  __shared__ double sh[kLanczosFusedThreads / 64 + 1];
-  constexpr int R = kLanczosFusedPerThread;
+  __shared__ double sh[kFusedWaves];
   const int t = threadIdx.x;
   const int64_t n = a.n;
   const int i = a.i;
-  LanczosScalars* sc = a.sc;
   __shared__ int s_stop;
   if (t == 0) s_stop = a.stop != nullptr ? *(volatile const int*)a.stop : 0;
   __syncthreads();
-  const bool skip = s_stop != 0;  // the same in every thread of the workgroup
-  const double bprev = i > 0 ? sc->beta[i - 1] : 0.0;
+  if (s_stop != 0) return;
+  const double bprev = i > 0 ? a.sc->beta[i - 1] : 0.0;
   double p = 0.0;
-  for (int64_t k = (int64_t)blockIdx.x * kLanczosFusedThreads + t; !skip && k < n;
+  for (int64_t k = (int64_t)blockIdx.x * kLanczosFusedThreads + t; k < n;
        k += (int64_t)gridDim.x * kLanczosFusedThreads) {
     double v = 0.0;
     if (a.w) {
@@ -298,42 +291,44 @@ __global__ __launch_bounds__(kLanczosFusedThreads) void k_lanczos_step(LanczosSt
     p += v * a.v_i[k];
   }
   const double part = group_sum_all(p, sh);
-  __shared__ bool s_last;
-  if (t == 0) {
-    __hip_atomic_store(&a.partial[blockIdx.x], part, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __threadfence();
-    const unsigned prev =
-        __hip_atomic_fetch_add(a.counter, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-    s_last = (prev == gridDim.x - 1);
-  }
-  __syncthreads();
-  if (!s_last) return;
-  if (skip) {
-    if (t == 0) *a.counter = 0;
-    return;
-  }
-  __threadfence();
-  double q = 0.0;
-  for (int b = t; b < (int)gridDim.x; b += kLanczosFusedThreads)
-    q += __hip_atomic_load(&a.partial[b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  const double alpha = group_sum_all(q, sh);
-  double w[R];
-  p = 0.0;
+  if (t == 0) a.partial[blockIdx.x] = part;
+}
+
+__global__ __launch_bounds__(kLanczosFusedThreads) void k_lanczos_finish(LanczosStepArgs a,
+                                                                         int nb) {
+  __shared__ double sh[2][kFusedWaves];
+  constexpr int R = kLanczosFusedPerThread;
+  const int t = threadIdx.x;
+  const int64_t n = a.n;
+  LanczosScalars* sc = a.sc;
+  __shared__ int s_stop;
+  if (t == 0) s_stop = a.stop != nullptr ? *(volatile const int*)a.stop : 0;
+  double w[R], vi[R];
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     const int64_t k = t + (int64_t)r * kLanczosFusedThreads;
-    w[r] = 0.0;
+    w[r] = k < n ? a.w_out[k] : 0.0;
+    vi[r] = k < n ? a.v_i[k] : 0.0;
+  }
+  double q = 0.0;
+  for (int b = t; b < nb; b += kLanczosFusedThreads) q += a.partial[b];
+  __syncthreads();
+  if (s_stop != 0) return;
+  const double alpha = group_sum_all(q, sh[0]);
+  double p = 0.0;
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int64_t k = t + (int64_t)r * kLanczosFusedThreads;
     if (k < n) {
-      w[r] = a.w_out[k] - alpha * a.v_i[k];
+      w[r] -= alpha * vi[r];
       p += w[r] * w[r];
     }
   }
-  double beta = sqrt(group_sum_all(p, sh));
+  double beta = sqrt(group_sum_all(p, sh[1]));
   if (beta < 1e-3 * alpha / sc->normz) beta = 0.0;  // LanczosAlgorithm.cu:140-142
   if (t == 0) {
-    sc->alpha[i] = alpha;
-    sc->beta[i] = beta;
-    *a.counter = 0;
+    sc->alpha[a.i] = alpha;
+    sc->beta[a.i] = beta;
   }
   const double inv = beta > 0.0 ? 1.0 / beta : 0.0;
 #pragma unroll
@@ -352,12 +347,10 @@ constexpr int kStep1R = 4;
 constexpr int64_t kStep1Max = (int64_t)kLanczosFusedThreads * kStep1R;
 
 __global__ __launch_bounds__(kLanczosFusedThreads) void k_lanczos_step_1wg(LanczosStepArgs a) {
-  __shared__ double sh[kLanczosFusedThreads / 64 + 1];
+  __shared__ double sh[2][kFusedWaves];
   __shared__ int s_stop;
   const int t = threadIdx.x;
   if (t == 0) s_stop = a.stop != nullptr ? *(volatile const int*)a.stop : 0;
-  __syncthreads();
-  if (s_stop != 0) return;  // past convergence (one workgroup: nothing to keep consistent)
   const int64_t n = a.n;
   const int i = a.i;
   LanczosScalars* sc = a.sc;
@@ -404,7 +397,9 @@ __global__ __launch_bounds__(kLanczosFusedThreads) void k_lanczos_step_1wg(Lancz
       p += w[r] * vi[r];
     }
   }
-  const double alpha = group_sum_all(p, sh);
+  __syncthreads();
+  if (s_stop != 0) return;  // past convergence (one workgroup: nothing to keep consistent)
+  const double alpha = group_sum_all(p, sh[0]);
   p = 0.0;
 #pragma unroll
   for (int r = 0; r < kStep1R; ++r) {
@@ -414,7 +409,7 @@ __global__ __launch_bounds__(kLanczosFusedThreads) void k_lanczos_step_1wg(Lancz
       p += w[r] * w[r];
     }
   }
-  double beta = sqrt(group_sum_all(p, sh));
+  double beta = sqrt(group_sum_all(p, sh[1]));
   if (beta < 1e-3 * alpha / sc->normz) beta = 0.0;  // LanczosAlgorithm.cu:140-142
   if (t == 0) {
     sc->alpha[i] = alpha;
@@ -438,10 +433,12 @@ void launch_lanczos_step(const LanczosStepArgs& a, hipStream_t s) {
     LM_HIP(hipGetLastError());
     return;
   }
-  if (!a.w_out || !a.partial || !a.counter)
+  if (!a.w_out || !a.partial)
     throw Error("[libmobility_amd] fused Lanczos step: no workspace");
   const int grid = (int)((a.n + kLanczosFusedThreads - 1) / kLanczosFusedThreads);
   hipLaunchKernelGGL(k_lanczos_step, dim3(grid), dim3(kLanczosFusedThreads), 0, s, a);
+  LM_HIP(hipGetLastError());
+  hipLaunchKernelGGL(k_lanczos_finish, dim3(1), dim3(kLanczosFusedThreads), 0, s, a, grid);
   LM_HIP(hipGetLastError());
 }
 

@@ -60,12 +60,16 @@ __device__ inline void pair_item(const PairItem& it, const typename Rec<R>::T* _
     const int cnt = (int)min((int64_t)kPairThreads, it.src1 - base);
     __syncthreads();
     if (j < it.src1) {
-      const R4 pj = pos[j];
-      s_pos[tid] = pj;
-      // wall: symmetric units (pair_math.hpp), the damping with the force
-      const R bf = WALL ? pj.w : R(1), bt = WALL ? pj.w * R(r0 / rt0) : R(1);
-      if (kNeedF) s_f[tid] = R4{bf * R(F[3 * j]), bf * R(F[3 * j + 1]), bf * R(F[3 * j + 2]), R(0)};
-      if (kNeedT) s_t[tid] = R4{bt * R(T[3 * j]), bt * R(T[3 * j + 1]), bt * R(T[3 * j + 2]), R(0)};
+      s_pos[tid] = pos[j];
+      if constexpr (WALL) {
+        // symmetric units (pair_math.hpp), the damping with the force
+        const R bf = s_pos[tid].w, bt = bf * R(r0 / rt0);
+        if (kNeedF) s_f[tid] = R4{bf * R(F[3 * j]), bf * R(F[3 * j + 1]), bf * R(F[3 * j + 2]), R(0)};
+        if (kNeedT) s_t[tid] = R4{bt * R(T[3 * j]), bt * R(T[3 * j + 1]), bt * R(T[3 * j + 2]), R(0)};
+      } else {
+        if (kNeedF) s_f[tid] = R4{R(F[3 * j]), R(F[3 * j + 1]), R(F[3 * j + 2]), R(0)};
+        if (kNeedT) s_t[tid] = R4{R(T[3 * j]), R(T[3 * j + 1]), R(T[3 * j + 2]), R(0)};
+      }
     } else {
       s_pos[tid] = far_record<R4>();
       if (kNeedF) s_f[tid] = R4{R(0), R(0), R(0), R(0)};

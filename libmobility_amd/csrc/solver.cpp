@@ -1100,10 +1100,6 @@ int NBodySolver::lanczos_run(const double* z, double** result) {
   const bool fused = n <= kLanczosFusedMaxN;
   // workspace
   red_partial_.reserve(sizeof(double) * 4 * kReduceBlocks);
-  if (red_counter_.capacity() == 0) {
-    red_counter_.reserve(sizeof(unsigned int) * 64);
-    launch_zero_u32(red_counter_.as<unsigned int>(), 64, stream_);
-  }
   scalars_.reserve(sizeof(LanczosScalars));
   tsq_work_.reserve(sizeof(double) * kCheckBatch * tsqrt_scratch(iter_limit_));
   coef_.reserve(sizeof(double) * kCheckBatch * kLanczosMaxIterations);
@@ -1118,7 +1114,7 @@ int NBodySolver::lanczos_run(const double* z, double** result) {
     chk_counter_.reserve(sizeof(unsigned int) * 64);
     launch_zero_u32(chk_counter_.as<unsigned int>(), 64, stream_);
   }
-  ReduceScratch rs{red_partial_.as<double>(), red_counter_.as<unsigned int>()};
+  double* partial = red_partial_.as<double>();
   ReduceScratch rs_chk{chk_partial_.as<double>(), chk_counter_.as<unsigned int>()};
   hipStream_t cs = chk_stream_;
   LanczosScalars* sc = scalars_.as<LanczosScalars>();
@@ -1178,7 +1174,7 @@ int NBodySolver::lanczos_run(const double* z, double** result) {
   ensure_cols(2);
   double* V = V_.as<double>();
   double* w = w_.as<double>();
-  launch_lanczos_start(z, V, n, rs, sc, old_host_, stream_);  // LanczosAlgorithm.cu:110-118
+  launch_lanczos_start(z, V, n, partial, sc, old_host_, stream_);  // LanczosAlgorithm.cu:110-118
   pair_stop_ = &sc->status.conv;
   const int check = std::min(check_steps_, iter_limit_ - 2);
   LanczosStatus* mirror = lz_status_.as<LanczosStatus>();
@@ -1259,8 +1255,7 @@ int NBodySolver::lanczos_run(const double* z, double** result) {
       }
       sa.n3 = 3 * N_;
       sa.w_out = w;
-      sa.partial = rs.partial;
-      sa.counter = rs.counter;
+      sa.partial = partial;
       sa.stop = pair_stop_;
       sa.v_prev = vp;
       sa.v_i = vi;
@@ -1271,9 +1266,7 @@ int NBodySolver::lanczos_run(const double* z, double** result) {
       launch_lanczos_step(sa, stream_);  // LanczosAlgorithm.cu:120-153
     } else {
       lanczos_product(vi, w);
-      launch_lanczos_alpha(w, vi, vp, n, i, rs, sc, stream_);
-      launch_lanczos_beta(w, vi, n, i, rs, sc, stream_);
-      launch_lanczos_next(w, vn, n, i, sc, stream_);
+      launch_lanczos_update(w, vi, vp, vn, n, i, partial, sc, stream_);
     }
     if (reorth_)
       launch_lanczos_reorth(V, n, i, n, reorth_partial_.as<double>(),

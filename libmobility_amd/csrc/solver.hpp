@@ -327,7 +327,7 @@ class NBodySolver {
   // staging for host arrays
   DevBuf st_pos_, st_f_, st_t_, st_u_, st_w_;
   // Lanczos
-  DevBuf V_, w_, coef_, noise_, red_partial_, red_counter_, scalars_, tsq_work_;
+  DevBuf V_, w_, coef_, noise_, red_partial_, scalars_, tsq_work_;
   int64_t V_cols_ = 0, V_n_ = 0;
   // Estimates of the convergence checks: a ring of ring_slots_ vectors of
   // ring_stride_ doubles; old_host_ names the slot holding the previous

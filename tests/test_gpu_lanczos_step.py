@@ -1,0 +1,44 @@
+"""The Lanczos recurrence at the vector lengths where its step changes its
+launches (lanczos_kernels.hip: one workgroup up to 4096 entries, two launches
+up to 16384, three beyond), against the oracle's restatement of the algorithm."""
+import numpy as np
+import pytest
+
+import oracle
+from tests.test_gpu_mdot import _solver
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-6
+
+
+@pytest.mark.parametrize("angular,N", [
+    (False, 1), (False, 342), (False, 1365), (False, 1366), (False, 5461), (False, 5462),
+    (True, 682), (True, 683), (True, 2730), (True, 2731)])
+def test_step_lengths_vs_oracle(angular, N):
+    rng = np.random.default_rng(N)
+    eta, a = 1 / (6 * np.pi), 1.0
+    # dilute, above a wall: the solve converges before orthogonality is lost,
+    # so both sides follow the same iterates
+    side = 6.0 * max(1.0, (N / 2) ** 0.5)
+    pos = rng.uniform(0, side, (N, 3))
+    pos[:, 2] = rng.uniform(1.5, 12.0, N)
+    s = _solver(True, a, eta)
+    s.initialize(viscosity=eta, hydrodynamicRadius=a, includeAngular=angular, tolerance=TOL)
+    s.setPositions(pos)
+
+    def product(v):
+        F, T = (v[:3 * N], v[3 * N:]) if angular else (v, None)
+        U, W = oracle.mdot(pos, eta, a, F=F, T=T, angular=angular, wall=True)
+        return np.concatenate([U, W]) if angular else U
+
+    lz = oracle.LanczosOracle()
+    for _ in range(2):  # the second call keeps the first one's schedule and estimate
+        W = rng.normal(size=(6 if angular else 3) * N)
+        u, w = s.sqrtMdotW_with_noise(W)
+        got = np.concatenate([u.ravel(), w.ravel()]) if angular else u.ravel()
+        ref, it = lz.run(product, W, TOL)
+        # an estimate at the tolerance may fall on either side of it: one
+        # iteration apart, and then the two differ by about the tolerance
+        assert abs(s.lastLanczosIterations() - it) <= 1
+        assert np.linalg.norm(got - ref) <= 2 * TOL * np.linalg.norm(ref)
