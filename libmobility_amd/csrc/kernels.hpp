@@ -175,7 +175,9 @@ struct SymReduceArgs {
 };
 void launch_sym_reduce(const SymReduceArgs& r, hipStream_t s);
 void launch_pair_multi(const PairMultiArgs& a, hipStream_t s);
-void launch_chunk_reduce(const double* part, int nchunks, int64_t n, double* out, hipStream_t s);
+// out[r][i] = sum over c of part[r][c][i], r < nvec
+void launch_chunk_reduce(const double* part, int nchunks, int64_t n, double* out, hipStream_t s,
+                         int nvec = 1);
 
 // setPositions: per-system bounding boxes (6 doubles each: min xyz, max xyz)
 // of the wall-shifted positions.

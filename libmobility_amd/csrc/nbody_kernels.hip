@@ -975,20 +975,24 @@ void launch_sym_reduce(const SymReduceArgs& r, hipStream_t s) {
   LM_HIP(hipGetLastError());
 }
 
-__global__ void k_chunk_reduce(const double* __restrict__ part, int nch, int64_t n,
-                               double* __restrict__ out) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+// out[r] = sum over the chunks c of part[r][c], for the vectors r = blockIdx.y
+// of n entries each.  Bound by latency up to some 10^5 entries: 16 loads in
+// flight instead of one (4 vectors of 24576 entries, 32 chunks: four launches of
+// 9.2 us -> one of 6 us).
+__global__ __launch_bounds__(kPairThreads) void k_chunk_reduce(const double* __restrict__ part,
+                                                              int nch, int64_t n,
+                                                              double* __restrict__ out) {
+  const int64_t i = (int64_t)blockIdx.x * kPairThreads + threadIdx.x;
   if (i >= n) return;
-  double s = 0.0;
-  for (int c = 0; c < nch; ++c) s += part[(int64_t)c * n + i];
-  out[i] = s;
+  const int64_t r = blockIdx.y;
+  out[r * n + i] = add_slabs(0.0, part + r * nch * n + i, nch, n);
 }
 
-void launch_chunk_reduce(const double* part, int nch, int64_t n, double* out, hipStream_t s) {
-  if (n <= 0) return;
-  const int nt = 256;
-  hipLaunchKernelGGL(k_chunk_reduce, dim3((unsigned)((n + nt - 1) / nt)), dim3(nt), 0, s, part,
-                     nch, n, out);
+void launch_chunk_reduce(const double* part, int nch, int64_t n, double* out, hipStream_t s,
+                         int nvec) {
+  if (n <= 0 || nvec <= 0) return;
+  const dim3 grid((unsigned)((n + kPairThreads - 1) / kPairThreads), (unsigned)nvec);
+  hipLaunchKernelGGL(k_chunk_reduce, grid, dim3(kPairThreads), 0, s, part, nch, n, out);
   LM_HIP(hipGetLastError());
 }
 

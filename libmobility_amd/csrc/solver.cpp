@@ -1668,9 +1668,7 @@ void NBodySolver::mdot_multi_dev(const double* F, int nrhs, double* U) {
       part_multi_.reserve(sizeof(double) * (size_t)nr * L.nch * n3);
       a.U = part_multi_.as<double>();
       launch_pair_multi(a, stream_);
-      for (int r = 0; r < nr; ++r)
-        launch_chunk_reduce(part_multi_.as<double>() + (int64_t)r * L.nch * n3, L.nch, n3,
-                            U + (int64_t)(r0 + r) * n3, stream_);
+      launch_chunk_reduce(part_multi_.as<double>(), L.nch, n3, U + (int64_t)r0 * n3, stream_, nr);
     }
     r0 += nr;
   }
