@@ -56,10 +56,10 @@ class SideStream {
   hipEvent_t block = nullptr, done = nullptr;
 };
 
-// One matrix, one launch per step: in place A -> L (lower; tiles above the
-// diagonal keep stale values), X = L^{-1}, Xt = X^T, Dinv = inverses of the
-// diagonal tiles; info[0] = 1 if A is not positive definite.  n is a
-// multiple of kCoarseTile.  The steps of X run on side.stream, each block of
+// One matrix, a launch per tile column: in place A -> L (lower; tiles above the
+// diagonal keep stale values; Xt holds the diagonal tiles of L until the end),
+// X = L^{-1}, Xt = X^T, Dinv = inverses of the diagonal tiles; info[0] = 1 if A
+// is not positive definite.  n is a multiple of kCoarseTile.  The steps of X run on side.stream, each block of
 // X behind an event on s that follows the block's columns of L; s waits for
 // the whole of X before it goes on.
 void launch_coarse_factor(double* A, double* X, double* Xt, double* Dinv, int* info, int64_t ld,

@@ -200,8 +200,42 @@ __global__ void k_pad_identity(double* __restrict__ A, const CoarseSys* __restri
 
 // ---- dense 64 x 64 tiles in LDS ------------------------------------------------
 
+constexpr int kTT = 256;                 // threads of the tile operations
+constexpr int kTQ = kT * kT / kTT;       // tile entries per thread
+
+// A tile on its way from memory to LDS: every load of a thread is in flight at
+// once (one at a time, a tile took 5 us, most of an operation).
+struct TileRegs {
+  double v[kTQ];
+  __device__ void fetch(const double* __restrict__ g, int64_t ld) {
+#pragma unroll
+    for (int q = 0; q < kTQ; ++q) {
+      const int e = (int)threadIdx.x + kTT * q;
+      v[q] = g[(e >> 6) * ld + (e & 63)];
+    }
+  }
+  __device__ void stage(double (*S)[kP]) const {
+#pragma unroll
+    for (int q = 0; q < kTQ; ++q) {
+      const int e = (int)threadIdx.x + kTT * q;
+      S[e >> 6][e & 63] = v[q];
+    }
+  }
+};
+
 __device__ inline void tile_load(double (*S)[kP], const double* __restrict__ g, int64_t ld) {
-  for (int e = threadIdx.x; e < kT * kT; e += blockDim.x) S[e >> 6][e & 63] = g[(e >> 6) * ld + (e & 63)];
+  TileRegs t;
+  t.fetch(g, ld);
+  t.stage(S);
+}
+
+__device__ inline void tile_load2(double (*S0)[kP], const double* __restrict__ g0, int64_t ld0,
+                                  double (*S1)[kP], const double* __restrict__ g1, int64_t ld1) {
+  TileRegs t0, t1;
+  t0.fetch(g0, ld0);
+  t1.fetch(g1, ld1);
+  t0.stage(S0);
+  t1.stage(S1);
 }
 
 typedef double d4 __attribute__((ext_vector_type(4)));
@@ -236,21 +270,40 @@ __device__ inline void tile_mm_mfma(const double (*A)[kP], const double (*B)[kP]
   }
 }
 
-// out[row][col] (= or -=) the quadrant result of tile_mm_mfma
-template <bool SUB>
-__device__ inline void tile_store_mfma(double* __restrict__ out, int64_t ld, const d4 acc[2][2]) {
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int R0 = (w >> 1) * 32, C0 = (w & 1) * 32;
-  const int li = lane & 15, lk = lane >> 4;
+// Entry (a, b, r) of a lane in the layout of tile_mm_mfma's result: row and column.
+__device__ inline int mfma_row(int a, int r) {
+  return ((int)threadIdx.x >> 7) * 32 + 16 * a + 4 * r + (((int)threadIdx.x & 63) >> 4);
+}
+__device__ inline int mfma_col(int b) {
+  return (((int)threadIdx.x >> 6) & 1) * 32 + 16 * b + ((int)threadIdx.x & 15);
+}
+
+// d = the tile at g in the layout of tile_mm_mfma's result (all loads in flight)
+__device__ inline void tile_fetch_mfma(const double* __restrict__ g, int64_t ld, d4 d[2][2]) {
 #pragma unroll
   for (int a = 0; a < 2; ++a)
 #pragma unroll
     for (int b = 0; b < 2; ++b)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        double* o = out + (int64_t)(R0 + 16 * a + 4 * r + lk) * ld + C0 + 16 * b + li;
-        *o = SUB ? *o - acc[a][b][r] : acc[a][b][r];
-      }
+      for (int r = 0; r < 4; ++r) d[a][b][r] = g[mfma_row(a, r) * ld + mfma_col(b)];
+}
+
+// out[row][col] = the result of tile_mm_mfma
+__device__ inline void tile_store_mfma(double* __restrict__ out, int64_t ld, const d4 acc[2][2]) {
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) out[mfma_row(a, r) * ld + mfma_col(b)] = acc[a][b][r];
+}
+
+// d -= acc
+__device__ inline void tile_sub(d4 d[2][2], const d4 acc[2][2]) {
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b) d[a][b] -= acc[a][b];
 }
 
 // acc += A * (TB ? B^T : B) for 64 x 64 tiles in LDS, the whole tile by one
@@ -276,27 +329,30 @@ __device__ inline void tile_mm_wave(const double (*A)[kP], const double (*B)[kP]
   }
 }
 
-// out[row][col] -= the tile result of tile_mm_wave
+// out[row][col] -= the tile result of tile_mm_wave, 16 entries in flight
 __device__ inline void tile_sub_wave(double* __restrict__ out, int64_t ld, const d4 acc[4][4]) {
   const int lane = threadIdx.x & 63;
   const int li = lane & 15, lk = lane >> 4;
 #pragma unroll
-  for (int p = 0; p < 4; ++p)
+  for (int p = 0; p < 4; ++p) {
+    double* o = out + (int64_t)(16 * p + lk) * ld + li;
+    double v[4][4];
 #pragma unroll
     for (int q = 0; q < 4; ++q)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        double* o = out + (int64_t)(16 * p + 4 * r + lk) * ld + 16 * q + li;
-        *o -= acc[p][q][r];
-      }
+      for (int r = 0; r < 4; ++r) v[q][r] = o[4 * r * ld + 16 * q];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[4 * r * ld + 16 * q] = v[q][r] - acc[p][q][r];
+  }
 }
 
 // ---- tile operations of the factorisation (256 threads each) -------------------
 // Every operation starts with a workgroup barrier, so that one workgroup can
 // run a sequence of them on the same LDS tiles and matrices.  The Cholesky
-// is right-looking, blocked by kKB tile columns: inside a block [kb, kend)
-// the step k updates only the block's own columns, and the tiles right of
-// the block receive the block's kKB products in one read-modify-write.
+// is blocked by kKB tile columns: a block [kb, kend) is finished first, and
+// the tiles right of it receive its kKB products in one read-modify-write.
 // X = L^{-1} is the block forward substitution on L X = I, blocked the same
 // way.
 
@@ -308,59 +364,122 @@ __device__ inline double lane_value(double v, int lane) {
   return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned int)lo);
 }
 
-// Factor the diagonal tile k, write L_kk (upper part zeroed) and its inverse
-// Dinv_k.  One wave (lanes 0..63 of the caller): lane r holds row r in
-// registers, and column j of the right-looking factorisation reaches the
-// other lanes by readlane.  Then lane c forms column c of L_kk^{-1} by
-// forward substitution, the rows of L_kk read from Ls (same address in every
-// lane).  info[0] = 1 when a pivot is not positive.
-__device__ __attribute__((always_inline)) inline void chol_diag_wave(double* __restrict__ A,
-                                                                     int64_t ld, int k,
-                                                                     double* __restrict__ Dinv,
-                                                                     int* __restrict__ info,
-                                                                     double (*Ls)[kP]) {
-  const int r = threadIdx.x & 63;
-  double* Akk = A + (int64_t)k * kT * ld + (int64_t)k * kT;
-  double a[kT];
+// Cholesky factor of one 64 x 64 tile in LDS (256 threads).  S: the lower part
+// of an SPD tile on entry, L on exit (the part above the diagonal holds
+// anything); W: L^{-T} on exit.  The column operations that turn A into L turn
+// the identity below it into L^{-T}, so the tile is factored as the 128 x 64
+// matrix [A; I], in four panels of 16 columns.  In a panel every wave holds the
+// panel's 16 diagonal rows in lanes 0-15 and eliminates them redundantly,
+// lanes 16-63 hold further rows (wave 0 those of A, waves 1 and 2 those of W;
+// rows of W above the panel's end only, the others are still zero there); a
+// column's multipliers reach the lanes by readlane.  The columns to the right
+// get the panel's product from the matrix cores.  Bound by the chain of 64
+// pivots: one wave with the whole tile in registers, and a forward
+// substitution for the inverse, took 43 us; a whole column of L around this
+// (k_chol_column) takes 19.
+// Returns false if a pivot is not positive.
+__device__ inline bool chol_tile(double (*S)[kP], double (*W)[kP]) {
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int li = lane & 15, lk = lane >> 4;
+  bool ok = true;
 #pragma unroll
-  for (int c = 0; c < kT; ++c) a[c] = Akk[(int64_t)r * ld + c];
-  bool bad = false;
-#pragma unroll
-  for (int j = 0; j < kT; ++j) {
-    double d = lane_value(a[j], j);
-    if (!(d > 0.0)) {
-      bad = true;
-      d = 1.0;
+  for (int q = 0; q < kTQ; ++q) {
+    const int e = (int)threadIdx.x + kTT * q;
+    W[e >> 6][e & 63] = (e >> 6) == (e & 63);
+  }
+  __syncthreads();
+#pragma unroll 1
+  for (int p = 0; p < kT / 16; ++p) {
+    const int c0 = 16 * p;
+    // the row of this lane: of S where it is below 64, of W from 64 on, -1 none
+    int row = -1;
+    if (wave == 0) {
+      if (c0 + lane < kT) row = c0 + lane;
+    } else if (wave < 3) {
+      const int q = 32 * (wave - 1) + lane - 16;
+      if (lane < 16) row = c0 + lane;
+      else if (lane < 48 && q < c0 + 16) row = kT + q;
     }
-    const double piv = sqrt(d);
-    const double ipiv = 1.0 / piv;
-    a[j] = r == j ? piv : (r > j ? a[j] * ipiv : a[j]);
-    // rows r >= c: A_rc -= L_rj L_cj (rows r < c hold the unused upper part)
+    double* r = row < 0 ? S[0] : (row < kT ? S[row] : W[row - kT]);
+    double a[16];
 #pragma unroll
-    for (int c = j + 1; c < kT; ++c) a[c] = __builtin_fma(-a[j], lane_value(a[j], c), a[c]);
+    for (int c = 0; c < 16; ++c) a[c] = row < 0 ? 0.0 : r[c0 + c];
+    __syncthreads();  // every wave has read the diagonal rows
+    if (wave < 3) {
+#pragma unroll
+      for (int j = 0; j < 16; ++j) {
+        double d = lane_value(a[j], j);
+        if (!(d > 0.0)) {
+          ok = false;
+          d = 1.0;
+        }
+        // sqrt(d) and its reciprocal, each corrected once by its residual
+        double ipiv = lm_rsqrt(d);
+        double piv = d * ipiv;
+        piv = __builtin_fma(0.5 * ipiv, __builtin_fma(-piv, piv, d), piv);
+        ipiv = __builtin_fma(ipiv, __builtin_fma(-piv, ipiv, 1.0), ipiv);
+        a[j] = lane == j ? piv : a[j] * ipiv;
+#pragma unroll
+        for (int c = j + 1; c < 16; ++c) a[c] = __builtin_fma(-a[j], lane_value(a[j], c), a[c]);
+      }
+      if (row >= 0 && (wave == 0 || lane >= 16)) {
+#pragma unroll
+        for (int c = 0; c < 16; ++c) r[c0 + c] = a[c];
+      }
+    }
+    __syncthreads();
+    // 16 x 16 tiles (tr, tc), tc > p: rows tr >= tc of S, rows tr <= p of W
+    const int rem = kT / 16 - 1 - p;
+    const int ns = rem * (rem + 1) / 2, nw = (p + 1) * rem;
+    for (int t = wave; t < ns + nw; t += 4) {  // uniform per wave
+      int tr, tc;
+      double(*X)[kP] = S;
+      if (t < ns) {
+        tri_index(t, tr, tc);
+        tr += p + 1;
+        tc += p + 1;
+      } else {
+        X = W;
+        tr = (t - ns) / rem;
+        tc = p + 1 + (t - ns) % rem;
+      }
+      d4 acc = d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int kk = 0; kk < 16; kk += 4)
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(X[16 * tr + li][c0 + kk + lk],
+                                                   S[16 * tc + li][c0 + kk + lk], acc, 0, 0, 0);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) X[16 * tr + 4 * q + lk][16 * tc + li] -= acc[q];
+    }
+    __syncthreads();
   }
+  return ok;
+}
+
+// L_kk and Dinv_k = L_kk^{-1} from chol_tile's tiles to memory
+__device__ inline void store_diag(double* __restrict__ Lkk, int64_t ld, double* __restrict__ D,
+                                  const double (*S)[kP], const double (*W)[kP]) {
 #pragma unroll
-  for (int c = 0; c < kT; ++c) {
-    const double v = c <= r ? a[c] : 0.0;
-    Ls[r][c] = v;
-    Akk[(int64_t)r * ld + c] = v;
+  for (int q = 0; q < kTQ; ++q) {
+    const int e = (int)threadIdx.x + kTT * q;
+    const int r = e >> 6, c = e & 63;
+    Lkk[(int64_t)r * ld + c] = c <= r ? S[r][c] : 0.0;
+    D[e] = W[c][r];
   }
-  if (bad && r == 0) info[0] = 1;
-  // The wave's LDS writes complete before its reads.  No workgroup barrier:
-  // the caller may be one wave of a larger workgroup.
-  __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
-  __builtin_amdgcn_wave_barrier();
-  double x[kT];
-#pragma unroll
-  for (int i = 0; i < kT; ++i) {
-    double s[4] = {i == r ? 1.0 : 0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-    for (int m = 0; m < i; ++m) s[m & 3] = __builtin_fma(-Ls[i][m], x[m], s[m & 3]);
-    x[i] = ((s[0] + s[1]) + (s[2] + s[3])) * (1.0 / Ls[i][i]);
-  }
-  double* D = Dinv + (int64_t)k * kT * kT;
-#pragma unroll
-  for (int i = 0; i < kT; ++i) D[i * kT + r] = x[i];
+}
+
+// Factor the diagonal tile k in place and write its inverse Dinv_k; info[0] = 1
+// when a pivot is not positive.
+__device__ inline void op_chol_diag(double* __restrict__ A, int64_t ld, int k,
+                                    double* __restrict__ Dinv, int* __restrict__ info,
+                                    double (*P0)[kP], double (*P1)[kP]) {
+  __syncthreads();
+  double* Akk = A + (int64_t)k * kT * ld + (int64_t)k * kT;
+  tile_load(P0, Akk, ld);
+  __syncthreads();
+  if (!chol_tile(P0, P1) && threadIdx.x == 0) info[0] = 1;
+  store_diag(Akk, ld, Dinv + (int64_t)k * kT * kT, P0, P1);
 }
 
 // L_ik = A_ik L_kk^{-T}
@@ -369,28 +488,49 @@ __device__ inline void op_panel(double* __restrict__ A, int64_t ld, int k, int i
                                 double (*P1)[kP]) {
   __syncthreads();
   double* Aik = A + (int64_t)i * kT * ld + (int64_t)k * kT;
-  tile_load(P0, Aik, ld);
-  tile_load(P1, Dinv + (int64_t)k * kT * kT, kT);
+  tile_load2(P0, Aik, ld, P1, Dinv + (int64_t)k * kT * kT, kT);
   __syncthreads();
   d4 acc[2][2];
   tile_zero(acc);
   tile_mm_mfma<true>(P0, P1, acc);
-  tile_store_mfma<false>(Aik, ld, acc);
+  tile_store_mfma(Aik, ld, acc);
+}
+
+// out -= sum over s < count of a_s (TB ? b_s^T : b_s), the tiles a_s at a + s sa,
+// b_s at b + s sb; the tiles of a step are loaded while the matrix cores work on
+// the step before.
+template <bool TB>
+__device__ inline void op_update(double* out, const double* a, int64_t sa, const double* b,
+                                 int64_t sb, int count, int64_t ld, double (*P0)[kP],
+                                 double (*P1)[kP]) {
+  d4 acc[2][2], d[2][2];
+  TileRegs ta, tb;
+  __syncthreads();  // what the tiles hold is in memory and LDS is free
+  ta.fetch(a, ld);
+  tb.fetch(b, ld);
+  tile_fetch_mfma(out, ld, d);
+  tile_zero(acc);
+  for (int s = 0; s < count; ++s) {
+    if (s > 0) __syncthreads();
+    ta.stage(P0);
+    tb.stage(P1);
+    __syncthreads();
+    if (s + 1 < count) {
+      ta.fetch(a + (s + 1) * sa, ld);
+      tb.fetch(b + (s + 1) * sb, ld);
+    }
+    tile_mm_mfma<TB>(P0, P1, acc);
+  }
+  tile_sub(d, acc);
+  tile_store_mfma(out, ld, d);
 }
 
 // A_ij -= sum_{k in [k0, k1)} L_ik L_jk^T
-__device__ inline void op_chol_update(double* __restrict__ A, int64_t ld, int i, int j, int k0,
-                                      int k1, double (*P0)[kP], double (*P1)[kP]) {
-  d4 acc[2][2];
-  tile_zero(acc);
-  for (int k = k0; k < k1; ++k) {
-    __syncthreads();
-    tile_load(P0, A + (int64_t)i * kT * ld + (int64_t)k * kT, ld);
-    tile_load(P1, A + (int64_t)j * kT * ld + (int64_t)k * kT, ld);
-    __syncthreads();
-    tile_mm_mfma<true>(P0, P1, acc);
-  }
-  tile_store_mfma<true>(A + (int64_t)i * kT * ld + (int64_t)j * kT, ld, acc);
+__device__ inline void op_chol_update(double* A, int64_t ld, int i, int j, int k0, int k1,
+                                      double (*P0)[kP], double (*P1)[kP]) {
+  double* Ai = A + (int64_t)i * kT * ld;
+  op_update<true>(Ai + (int64_t)j * kT, Ai + (int64_t)k0 * kT, kT,
+                  A + (int64_t)j * kT * ld + (int64_t)k0 * kT, kT, k1 - k0, ld, P0, P1);
 }
 
 // X_km = Dinv_k X_km
@@ -399,29 +539,20 @@ __device__ inline void op_trinv_scale(double* __restrict__ X, int64_t ld, int k,
                                       double (*P1)[kP]) {
   __syncthreads();
   double* Xkm = X + (int64_t)k * kT * ld + (int64_t)m * kT;
-  tile_load(P0, Xkm, ld);
-  tile_load(P1, Dinv + (int64_t)k * kT * kT, kT);
+  tile_load2(P0, Xkm, ld, P1, Dinv + (int64_t)k * kT * kT, kT);
   __syncthreads();
   d4 acc[2][2];
   tile_zero(acc);
   tile_mm_mfma<false>(P1, P0, acc);
-  tile_store_mfma<false>(Xkm, ld, acc);
+  tile_store_mfma(Xkm, ld, acc);
 }
 
 // X_im -= sum_{k in [k0, k1)} L_ik X_km
-__device__ inline void op_trinv_update(double* __restrict__ X, const double* __restrict__ L,
-                                       int64_t ld, int i, int m, int k0, int k1,
-                                       double (*P0)[kP], double (*P1)[kP]) {
-  d4 acc[2][2];
-  tile_zero(acc);
-  for (int k = k0; k < k1; ++k) {
-    __syncthreads();
-    tile_load(P0, L + (int64_t)i * kT * ld + (int64_t)k * kT, ld);
-    tile_load(P1, X + (int64_t)k * kT * ld + (int64_t)m * kT, ld);
-    __syncthreads();
-    tile_mm_mfma<false>(P0, P1, acc);
-  }
-  tile_store_mfma<true>(X + (int64_t)i * kT * ld + (int64_t)m * kT, ld, acc);
+__device__ inline void op_trinv_update(double* X, const double* L, int64_t ld, int i, int m, int k0,
+                                       int k1, double (*P0)[kP], double (*P1)[kP]) {
+  op_update<false>(X + (int64_t)i * kT * ld + (int64_t)m * kT,
+                   L + (int64_t)i * kT * ld + (int64_t)k0 * kT, kT,
+                   X + (int64_t)k0 * kT * ld + (int64_t)m * kT, kT * ld, k1 - k0, ld, P0, P1);
 }
 
 // Xt tile (bj, bi) = (X tile (bi, bj))^T
@@ -431,35 +562,80 @@ __device__ inline void op_transpose(const double* __restrict__ X, double* __rest
   tile_load(P0, X + (int64_t)bi * kT * ld + (int64_t)bj * kT, ld);
   __syncthreads();
   double* o = Xt + (int64_t)bj * kT * ld + (int64_t)bi * kT;
-  for (int e = threadIdx.x; e < kT * kT; e += blockDim.x) o[(e >> 6) * ld + (e & 63)] = P0[e & 63][e >> 6];
+#pragma unroll
+  for (int q = 0; q < kTQ; ++q) {
+    const int e = (int)threadIdx.x + kTT * q;
+    o[(e >> 6) * ld + (e & 63)] = P0[e & 63][e >> 6];
+  }
 }
 
 // ---- one matrix, one launch per step ---------------------------------------------
 
-__global__ __launch_bounds__(64) void k_chol_diag(double* __restrict__ A, int64_t ld, int k,
-                                                  double* __restrict__ Dinv,
-                                                  int* __restrict__ info) {
-  __shared__ double Ls[kT][kP];
-  chol_diag_wave(A, ld, k, Dinv, info, Ls);
+// S = d, in LDS
+__device__ inline void tile_put_mfma(double (*S)[kP], const d4 d[2][2]) {
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) S[mfma_row(a, r)][mfma_col(b)] = d[a][b][r];
 }
 
-__global__ __launch_bounds__(256) void k_chol_panel(double* __restrict__ A, int64_t ld, int k,
-                                                    const double* __restrict__ Dinv) {
-  __shared__ double P0[kT][kP];
-  __shared__ double P1[kT][kP];
-  op_panel(A, ld, k, k + 1 + blockIdx.x, Dinv, P0, P1);
-}
-
-// A_ij -= L_ik L_jk^T for the block's columns k < j < kend, rows j <= i < nb
-__global__ __launch_bounds__(256) void k_chol_local(double* __restrict__ A, int64_t ld, int k,
-                                                    int kend) {
-  __shared__ double P0[kT][kP];
-  __shared__ double P1[kT][kP];
-  const int jcount = kend - k - 1;
-  const int j = k + 1 + (int)(blockIdx.x % jcount);
-  const int i = k + 1 + (int)(blockIdx.x / jcount);
-  if (i < j) return;  // uniform per workgroup
-  op_chol_update(A, ld, i, j, k, k + 1, P0, P1);
+// Tile column k of L, one workgroup per tile row i = k + blockIdx.x, from the
+// block's columns before it (left-looking inside the block of kKB columns):
+//   A_ik -= sum_{k' in [kb, k)} L_ik' L_kk'^T,   L_ik = A_ik L_kk^{-T}.
+// Every workgroup updates and factors the diagonal tile itself, so a column is
+// one launch: with launches of their own for the diagonal tile, the column and
+// the update of the block's later columns a column took 71 us on average, of
+// which most was one wave's chain and the launches' latency; now 19 to 37 us,
+// 28 on average (36 tiles).  A_kk is read by all and written by none: workgroup 0 leaves L_kk in
+// `Lkk` (row pitch ld) until the whole of L is done.
+__global__ __launch_bounds__(256) void k_chol_column(double* __restrict__ A, int64_t ld, int kb,
+                                                     int k, double* __restrict__ Lkk,
+                                                     double* __restrict__ Dinv,
+                                                     int* __restrict__ info) {
+  __shared__ double P[4][kT][kP];
+  const int i = k + (int)blockIdx.x;
+  const bool below = i > k;  // uniform per workgroup
+  const double* rowk = A + (int64_t)k * kT * ld;
+  double* rowi = A + (int64_t)i * kT * ld;
+  d4 dk[2][2], di[2][2], ak[2][2], ai[2][2];
+  TileRegs tk, ti;
+  if (kb < k) {
+    tk.fetch(rowk + (int64_t)kb * kT, ld);
+    if (below) ti.fetch(rowi + (int64_t)kb * kT, ld);
+  }
+  tile_fetch_mfma(rowk + (int64_t)k * kT, ld, dk);
+  tile_fetch_mfma(rowi + (int64_t)k * kT, ld, di);
+  tile_zero(ak);
+  tile_zero(ai);
+  for (int q = kb; q < k; ++q) {
+    if (q > kb) __syncthreads();
+    tk.stage(P[0]);
+    if (below) ti.stage(P[1]);
+    __syncthreads();
+    if (q + 1 < k) {
+      tk.fetch(rowk + (int64_t)(q + 1) * kT, ld);
+      if (below) ti.fetch(rowi + (int64_t)(q + 1) * kT, ld);
+    }
+    tile_mm_mfma<true>(P[0], P[0], ak);
+    if (below) tile_mm_mfma<true>(P[1], P[0], ai);
+  }
+  tile_sub(dk, ak);
+  tile_put_mfma(P[2], dk);
+  __syncthreads();  // the tiles of the last step are read, P[2] is written
+  const bool ok = chol_tile(P[2], P[3]);
+  if (!below) {
+    if (!ok && threadIdx.x == 0) info[0] = 1;
+    store_diag(Lkk, ld, Dinv + (int64_t)k * kT * kT, P[2], P[3]);
+    return;
+  }
+  tile_sub(di, ai);
+  tile_put_mfma(P[1], di);
+  __syncthreads();
+  tile_zero(ai);
+  tile_mm_mfma<false>(P[1], P[3], ai);
+  tile_store_mfma(rowi + (int64_t)k * kT, ld, ai);
 }
 
 // A_ij -= sum_{k in [kb, kend)} L_ik L_jk^T for kend <= j <= i < nb
@@ -586,22 +762,22 @@ __global__ __launch_bounds__(256) void k_trinv_trailing2(double* __restrict__ X,
   if (live) tile_sub_wave(X + (int64_t)i * kT * ld + (int64_t)m * kT, ld, acc);
 }
 
-__global__ __launch_bounds__(256) void k_trinv_scale(double* __restrict__ X, int64_t ld, int k,
+// Tile rows [kb, kend) of X, one workgroup per tile column m < kend:
+//   X_km = Dinv_k (X_km - sum_{k' in [max(kb, m), k)} L_kk' X_k'm)
+// One launch for the block's 4 rows, which depend on each other, instead of two
+// per row (15 us each): 43 to 52 us.
+__global__ __launch_bounds__(256) void k_trinv_block(double* __restrict__ X,
+                                                     const double* __restrict__ L, int64_t ld,
+                                                     int kb, int kend,
                                                      const double* __restrict__ Dinv) {
   __shared__ double P0[kT][kP];
   __shared__ double P1[kT][kP];
-  op_trinv_scale(X, ld, k, blockIdx.x, Dinv, P0, P1);
-}
-
-// X_im -= L_ik X_km for the block's rows k < i < kend, m <= k
-__global__ __launch_bounds__(256) void k_trinv_local(double* __restrict__ X,
-                                                     const double* __restrict__ L, int64_t ld,
-                                                     int k) {
-  __shared__ double P0[kT][kP];
-  __shared__ double P1[kT][kP];
-  const int m = blockIdx.x % (k + 1);
-  const int i = k + 1 + blockIdx.x / (k + 1);
-  op_trinv_update(X, L, ld, i, m, k, k + 1, P0, P1);
+  const int m = blockIdx.x;
+  const int k0 = m > kb ? m : kb;
+  for (int k = k0; k < kend; ++k) {
+    if (k > k0) op_trinv_update(X, L, ld, k, m, k0, k, P0, P1);
+    op_trinv_scale(X, ld, k, m, Dinv, P0, P1);
+  }
 }
 
 // X_im -= sum_{k in [max(kb, m), kend)} L_ik X_km for kend <= i < nb, m < kend
@@ -624,9 +800,15 @@ __global__ void k_identity(double* __restrict__ X, int64_t ld, int n) {
   }
 }
 
-__global__ __launch_bounds__(256) void k_transpose(const double* __restrict__ X,
-                                                   double* __restrict__ Xt, int64_t ld) {
+// Xt = X^T; the diagonal tiles of L, until now in Xt, go to A
+__global__ __launch_bounds__(256) void k_transpose(const double* __restrict__ X, double* Xt,
+                                                   double* __restrict__ A, int64_t ld) {
   __shared__ double P0[kT][kP];
+  if (blockIdx.x == blockIdx.y) {
+    const int64_t t = (int64_t)blockIdx.x * kT * (ld + 1);
+    for (int e = threadIdx.x; e < kT * kT; e += blockDim.x)
+      A[t + (e >> 6) * ld + (e & 63)] = Xt[t + (e >> 6) * ld + (e & 63)];
+  }
   op_transpose(X, Xt, ld, blockIdx.y, blockIdx.x, P0);
 }
 
@@ -650,8 +832,7 @@ __global__ __launch_bounds__(256) void k_factor_small(double* __restrict__ A,
   for (int kb = 0; kb < nb; kb += kKB) {
     const int kend = kb + kKB < nb ? kb + kKB : nb;
     for (int k = kb; k < kend; ++k) {
-      __syncthreads();
-      if (threadIdx.x < 64) chol_diag_wave(a, n, k, dinv, info, P0);
+      op_chol_diag(a, n, k, dinv, info, P0, P1);
       for (int i = k + 1; i < nb; ++i) op_panel(a, n, k, i, dinv, P0, P1);
       for (int j = k + 1; j < kend; ++j)
         for (int i = j; i < nb; ++i) op_chol_update(a, n, i, j, k, k + 1, P0, P1);
@@ -825,25 +1006,15 @@ void launch_coarse_factor(double* A, double* X, double* Xt, double* Dinv, int* i
                      n);
   for (int kb = 0; kb < nb; kb += kKB) {
     const int kend = kb + kKB < nb ? kb + kKB : nb;
-    for (int k = kb; k < kend; ++k) {
-      hipLaunchKernelGGL(k_chol_diag, dim3(1), dim3(64), 0, s, A, ld, k, Dinv, info);
-      const int below = nb - k - 1;
-      if (below > 0) hipLaunchKernelGGL(k_chol_panel, dim3(below), dim3(256), 0, s, A, ld, k, Dinv);
-      if (kend - k - 1 > 0)
-        hipLaunchKernelGGL(k_chol_local, dim3((unsigned)((kend - k - 1) * below)), dim3(256), 0, s,
-                           A, ld, k, kend);
-    }
-    // Columns [kb, kend) of L and their diagonal inverses are final here.
-    // Block kb of X reads nothing else of L, and the trailing update of L
-    // below writes only columns >= kend.
+    for (int k = kb; k < kend; ++k)
+      hipLaunchKernelGGL(k_chol_column, dim3(nb - k), dim3(256), 0, s, A, ld, kb, k,
+                         Xt + (int64_t)k * kT * (ld + 1), Dinv, info);
+    // Columns [kb, kend) of L and their diagonal inverses are final here (the
+    // diagonal tiles of L are in Xt).  Block kb of X reads nothing else of L,
+    // and the trailing update of L below writes only columns >= kend.
     LM_HIP(hipEventRecord(side.block, s));
     LM_HIP(hipStreamWaitEvent(x, side.block, 0));
-    for (int k = kb; k < kend; ++k) {
-      hipLaunchKernelGGL(k_trinv_scale, dim3(k + 1), dim3(256), 0, x, X, ld, k, Dinv);
-      if (kend - k - 1 > 0)
-        hipLaunchKernelGGL(k_trinv_local, dim3((unsigned)((kend - k - 1) * (k + 1))), dim3(256), 0,
-                           x, X, A, ld, k);
-    }
+    hipLaunchKernelGGL(k_trinv_block, dim3(kend), dim3(256), 0, x, X, A, ld, kb, kend, Dinv);
     const int T = nb - kend;
     const int64_t xtiles = (int64_t)T * kend;
     if (xtiles >= kQuadTiles)
@@ -859,7 +1030,7 @@ void launch_coarse_factor(double* A, double* X, double* Xt, double* Dinv, int* i
       hipLaunchKernelGGL(k_chol_trailing, dim3((unsigned)tiles), dim3(256), 0, s, A, ld, kb, kend);
   }
   LM_HIP(hipGetLastError());
-  hipLaunchKernelGGL(k_transpose, dim3(nb, nb), dim3(256), 0, x, X, Xt, ld);
+  hipLaunchKernelGGL(k_transpose, dim3(nb, nb), dim3(256), 0, x, X, Xt, A, ld);
   LM_HIP(hipGetLastError());
   LM_HIP(hipEventRecord(side.done, x));
   LM_HIP(hipStreamWaitEvent(s, side.done, 0));
