@@ -203,14 +203,15 @@ void CoarseLevel::build(const void* rec64, const void* rec32, const std::vector<
                  .count();
 }
 
-void CoarseLevel::apply(Op op, const double* in, double* out, int64_t n, hipStream_t s) {
+void CoarseLevel::apply(Op op, const double* in, double* out, int64_t n, hipStream_t s,
+                        const ParticleBlocks& before, const ParticleBlocks& after) {
   if (cells_.C == 0) throw Error("[libmobility_amd] coarse level not built");
   if (n < 3 * N_) throw Error("[libmobility_amd] coarse level: vector too short");
   const double* T = op == kG ? X_.as<double>() : (op == kGt ? Xt_.as<double>() : A_.as<double>());
   launch_coarse_apply(T, sys_dev_.as<CoarseSys>(), row_sys_.as<int>(), 3 * cells_.C, max_row_,
                       op != kGt, in, out, N_, n, perm_.as<int>(), start_.as<int>(),
                       cell_of_.as<int>(), scale_.as<double>(), cells_.C, cvec_.as<double>(),
-                      yvec_.as<double>(), s);
+                      yvec_.as<double>(), before, after, s);
 }
 
 void CoarseLevel::factors(int q, double* L, double* X, hipStream_t st) const {

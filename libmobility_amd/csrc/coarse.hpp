@@ -67,14 +67,25 @@ void launch_coarse_factor(double* A, double* X, double* Xt, double* Dinv, int* i
 // The same for the systems list[0..count), one workgroup each (small blocks).
 void launch_coarse_factor_small(double* A, double* X, double* Xt, double* Dinv, int* info,
                                 const CoarseSys* sys, const int* list, int count, hipStream_t s);
-// out = in + Q (T - I) Q^T in on entries [0, 3N), out = in on [3N, n); T the
+// One dense dim x dim block per particle (3: translational entries, 6: linear and
+// angular ones), applied as B_i or B_i^T; B = nullptr: none.
+struct ParticleBlocks {
+  const double* B = nullptr;
+  int dim = 0;
+  int transpose = 0;
+};
+// out = in + Q (T - I) Q^T in on entries [0, 3N), out = in on [3N, n), with the
+// particles' blocks `before` applied to `in` first or `after` to the result (not
+// both); T the
 // systems' lower (m <= r) or upper (m >= r) triangular blocks; row_sys[r] is
 // the system of coarse row r < rows; max_row = the largest 3 C_s (selects one
 // wave or one workgroup per row).  in may equal out.
 void launch_coarse_apply(const double* T, const CoarseSys* sys, const int* row_sys, int rows,
                          int max_row, bool lower, const double* in, double* out, int64_t N,
                          int64_t n, const int* perm, const int* start, const int* cell_of,
-                         const double* scale, int C, double* cvec, double* yvec, hipStream_t s);
+                         const double* scale, int C, double* cvec, double* yvec,
+                         const ParticleBlocks& before, const ParticleBlocks& after,
+                         hipStream_t s);
 
 // Cell assignment of positions in units of a (x, y, z per particle, host):
 // g_k cells along axis k, cell edge ~ (volume / (N / ppc))^{1/3}; empty cells
@@ -110,8 +121,10 @@ class CoarseLevel {
   void build(const void* rec64, const void* rec32, const std::vector<int64_t>& off,
              const std::vector<int>& wall, int ppc, int64_t max_dim, bool fp64, hipStream_t s);
   // out = Gc in (kG), Gc^T in (kGt) or Gc^{-1} in (kGinv); vectors of length
-  // n >= 3N whose entries past 3N pass through.  in may equal out.
-  void apply(Op op, const double* in, double* out, int64_t n, hipStream_t s);
+  // n >= 3N whose entries past 3N pass through; the particles' blocks `before`
+  // or `after` it in the same launches.  in may equal out.
+  void apply(Op op, const double* in, double* out, int64_t n, hipStream_t s,
+             const ParticleBlocks& before = {}, const ParticleBlocks& after = {});
 
   int cells() const { return cells_.C; }
   int dim() const { return 3 * cells_.C; }

@@ -859,9 +859,35 @@ __global__ __launch_bounds__(256) void k_factor_small(double* __restrict__ A,
 
 // ---- per-application kernels ------------------------------------------------------
 
-// cvec[3c+a] = scale[c] * sum over the particles of cell c of in[3i+a]; one
+// One particle's entries of a vector: the three translational ones, and with D =
+// 6 the angular ones (from 3N on).
+template <int D>
+__device__ inline int64_t entry(int64_t i, int k, int64_t N) {
+  return k < 3 ? 3 * i + k : 3 * N + 3 * i + (k - 3);
+}
+
+// y = B_i x or B_i^T x for the D x D block of particle i
+template <int D>
+__device__ inline void block_times(const double* __restrict__ B, int64_t i, int transpose,
+                                   const double x[D], double y[D]) {
+  const double* b = B + (int64_t)D * D * i;
+#pragma unroll
+  for (int r = 0; r < D; ++r) {
+    double s = 0.0;
+#pragma unroll
+    for (int k = 0; k < D; ++k) s += (transpose ? b[D * k + r] : b[D * r + k]) * x[k];
+    y[r] = s;
+  }
+}
+
+// cvec[3c+a] = scale[c] * sum over the particles of cell c of v[3i+a]; one
 // wave per cell, lanes stride the cell's sorted list, fixed-order butterfly.
-__global__ __launch_bounds__(256) void k_coarse_restrict(const double* __restrict__ in,
+// D = 0: v = in.  D = 3, 6: v = B_i in or B_i^T in, which also goes to `out`
+// (every particle is in one cell); the blocks in a launch of their own cost 5 us
+// more (32768 particles).
+template <int D>
+__global__ __launch_bounds__(256) void k_coarse_restrict(const double* in, const double* B,
+                                                         int transpose, int64_t N, double* out,
                                                          const int* __restrict__ perm,
                                                          const int* __restrict__ start,
                                                          const double* __restrict__ scale, int C,
@@ -871,10 +897,23 @@ __global__ __launch_bounds__(256) void k_coarse_restrict(const double* __restric
   if (c >= C) return;  // uniform per wave
   double s0 = 0.0, s1 = 0.0, s2 = 0.0;
   for (int k = start[c] + lane; k < start[c + 1]; k += 64) {
-    const int64_t p = 3 * (int64_t)perm[k];
-    s0 += in[p];
-    s1 += in[p + 1];
-    s2 += in[p + 2];
+    const int64_t i = perm[k];
+    constexpr int M = D > 0 ? D : 3;
+    double v[M];
+#pragma unroll
+    for (int q = 0; q < M; ++q) v[q] = in[entry<M>(i, q, N)];
+    if constexpr (D > 0) {
+      double t[M];
+      block_times<D>(B, i, transpose, v, t);
+#pragma unroll
+      for (int q = 0; q < M; ++q) {
+        v[q] = t[q];
+        out[entry<M>(i, q, N)] = t[q];
+      }
+    }
+    s0 += v[0];
+    s1 += v[1];
+    s2 += v[2];
   }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
@@ -939,20 +978,47 @@ __global__ __launch_bounds__(256) void k_coarse_gemv_wave(const double* __restri
 }
 
 // out[k] = in[k] + scale[c] * y[3c + a] for k = 3i + a < 3N (c = cell of i),
-// out[k] = in[k] beyond (in may equal out)
-__global__ void k_coarse_prolong(const double* in, const int* __restrict__ cell_of,
+// out[k] = rest[k] beyond (in and rest may equal out)
+__global__ void k_coarse_prolong(const double* in, const double* rest,
+                                 const int* __restrict__ cell_of,
                                  const double* __restrict__ scale, const double* __restrict__ y,
                                  int64_t n3, int64_t n, double* out) {
   const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= n) return;
-  double v = in[k];
   if (k < n3) {
     const int64_t i = k / 3;
-    const int a = (int)(k - 3 * i);
     const int c = cell_of[i];
-    v += scale[c] * y[3 * c + a];
+    out[k] = in[k] + scale[c] * y[3 * c + (int)(k - 3 * i)];
+  } else {
+    out[k] = rest[k];
   }
-  out[k] = v;
+}
+
+// The same followed by out = B_i (.) or B_i^T (.) per particle, D x D blocks (one
+// launch instead of two); with D = 3 entries from 3N on pass through.
+template <int D>
+__global__ void k_coarse_prolong_blocks(const double* in, const int* __restrict__ cell_of,
+                                        const double* __restrict__ scale,
+                                        const double* __restrict__ y,
+                                        const double* __restrict__ B, int transpose, int64_t N,
+                                        int64_t n, double* out) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < N) {
+    const int c = cell_of[i];
+    double v[D], t[D];
+#pragma unroll
+    for (int q = 0; q < D; ++q) {
+      v[q] = in[entry<D>(i, q, N)];
+      if (q < 3) v[q] += scale[c] * y[3 * c + q];
+    }
+    block_times<D>(B, i, transpose, v, t);
+#pragma unroll
+    for (int q = 0; q < D; ++q) out[entry<D>(i, q, N)] = t[q];
+  }
+  if (D == 3) {
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t k = 3 * N + i; k < n; k += stride) out[k] = in[k];
+  }
 }
 
 inline unsigned blocks_for(int64_t n, int nt) { return (unsigned)((n + nt - 1) / nt); }
@@ -1046,17 +1112,43 @@ void launch_coarse_factor_small(double* A, double* X, double* Xt, double* Dinv, 
 void launch_coarse_apply(const double* T, const CoarseSys* sys, const int* row_sys, int rows,
                          int max_row, bool lower, const double* in, double* out, int64_t N,
                          int64_t n, const int* perm, const int* start, const int* cell_of,
-                         const double* scale, int C, double* cvec, double* yvec, hipStream_t s) {
-  hipLaunchKernelGGL(k_coarse_restrict, dim3(blocks_for(C, 4)), dim3(256), 0, s, in, perm, start,
-                     scale, C, cvec);
+                         const double* scale, int C, double* cvec, double* yvec,
+                         const ParticleBlocks& before, const ParticleBlocks& after,
+                         hipStream_t s) {
+  for (const ParticleBlocks* b : {&before, &after})
+    if (b->B != nullptr && b->dim != 3 && !(b->dim == 6 && n == 6 * N))
+      throw Error("[libmobility_amd] 6x6 preconditioner blocks need linear and angular entries");
+  const dim3 cells(blocks_for(C, 4)), block(256);
+  const int bd = before.B ? before.dim : 0, ad = after.B ? after.dim : 0;
+  auto restrict_with = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, cells, block, 0, s, in, before.B, before.transpose, N, out, perm,
+                       start, scale, C, cvec);
+  };
+  if (bd == 0) restrict_with(k_coarse_restrict<0>);
+  else if (bd == 3) restrict_with(k_coarse_restrict<3>);
+  else restrict_with(k_coarse_restrict<6>);
+  LM_HIP(hipGetLastError());
   if (max_row <= kWaveRowMax)
-    hipLaunchKernelGGL(k_coarse_gemv_wave, dim3(blocks_for(rows, 4)), dim3(256), 0, s, T, sys,
-                       row_sys, rows, lower ? 1 : 0, cvec, yvec);
+    hipLaunchKernelGGL(k_coarse_gemv_wave, dim3(blocks_for(rows, 4)), block, 0, s, T, sys, row_sys,
+                       rows, lower ? 1 : 0, cvec, yvec);
   else
-    hipLaunchKernelGGL(k_coarse_gemv, dim3(rows), dim3(256), 0, s, T, sys, row_sys, lower ? 1 : 0,
+    hipLaunchKernelGGL(k_coarse_gemv, dim3(rows), block, 0, s, T, sys, row_sys, lower ? 1 : 0,
                        cvec, yvec);
-  hipLaunchKernelGGL(k_coarse_prolong, dim3(blocks_for(n, 256)), dim3(256), 0, s, in, cell_of,
-                     scale, yvec, 3 * N, n, out);
+  LM_HIP(hipGetLastError());
+  const double* trans = bd > 0 ? out : in;  // translational entries so far, and the rest
+  const double* rest = bd == 6 ? out : in;
+  if (ad == 0) {
+    hipLaunchKernelGGL(k_coarse_prolong, dim3(blocks_for(n, 256)), block, 0, s, trans, rest,
+                       cell_of, scale, yvec, 3 * N, n, out);
+  } else {
+    if (bd > 0) throw Error("[libmobility_amd] coarse level: blocks on both sides");
+    auto prolong_with = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3(blocks_for(N, 256)), block, 0, s, in, cell_of, scale, yvec,
+                         after.B, after.transpose, N, n, out);
+    };
+    if (ad == 3) prolong_with(k_coarse_prolong_blocks<3>);
+    else prolong_with(k_coarse_prolong_blocks<6>);
+  }
   LM_HIP(hipGetLastError());
 }
 

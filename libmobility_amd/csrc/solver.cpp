@@ -1910,34 +1910,34 @@ void NBodySolver::ensure_pre() {
   ensure_coarse();
 }
 
+// The learned blocks of the preconditioner, or those of their inverses.
+ParticleBlocks NBodySolver::pre_blocks(const DevBuf& G, int transpose) const {
+  return precond_ ? ParticleBlocks{G.as<double>(), precond_->kind() == 1 ? 6 : 3, transpose}
+                  : ParticleBlocks{};
+}
+
 // G = D Gc: t = G^T v = Gc^T D^T v
 void NBodySolver::pre_forward(const double* v, double* t, int64_t n) {
-  if (precond_) {
+  if (coarse_ppc_ > 0)
+    coarse_.apply(CoarseLevel::kGt, v, t, n, stream_, pre_blocks(pc_G_, 1));
+  else
     launch_apply_blocks(pc_G_.as<double>(), v, N_, n, precond_->kind(), 1, t, stream_);
-    if (coarse_ppc_ > 0) coarse_.apply(CoarseLevel::kGt, t, t, n, stream_);
-  } else {
-    coarse_.apply(CoarseLevel::kGt, v, t, n, stream_);
-  }
 }
 
 // w = G u = D Gc u
 void NBodySolver::pre_back(double* u, double* w, int64_t n) {
-  if (precond_) {
-    if (coarse_ppc_ > 0) coarse_.apply(CoarseLevel::kG, u, u, n, stream_);
+  if (coarse_ppc_ > 0)
+    coarse_.apply(CoarseLevel::kG, u, w, n, stream_, {}, pre_blocks(pc_G_, 0));
+  else
     launch_apply_blocks(pc_G_.as<double>(), u, N_, n, precond_->kind(), 0, w, stream_);
-  } else {
-    coarse_.apply(CoarseLevel::kG, u, w, n, stream_);
-  }
 }
 
 // out = G^{-1} y = Gc^{-1} D^{-1} y
 void NBodySolver::pre_inverse(const double* y, double* out, int64_t n) {
-  if (precond_) {
+  if (coarse_ppc_ > 0)
+    coarse_.apply(CoarseLevel::kGinv, y, out, n, stream_, pre_blocks(pc_Gi_, 0));
+  else
     launch_apply_blocks(pc_Gi_.as<double>(), y, N_, n, precond_->kind(), 0, out, stream_);
-    if (coarse_ppc_ > 0) coarse_.apply(CoarseLevel::kGinv, out, out, n, stream_);
-  } else {
-    coarse_.apply(CoarseLevel::kGinv, y, out, n, stream_);
-  }
 }
 
 int NBodySolver::coarseCells(int* cell_of, int* grid) const {

@@ -261,6 +261,7 @@ class NBodySolver {
   bool pre_on() const { return precond_ != nullptr || coarse_ppc_ > 0; }
   void ensure_pre();
   bool pre_current(uint64_t layout, uint64_t structure, double a) const;
+  ParticleBlocks pre_blocks(const DevBuf& G, int transpose) const;
   void pre_forward(const double* v, double* t, int64_t n);
   void pre_back(double* u, double* w, int64_t n);
   void pre_inverse(const double* y, double* out, int64_t n);
