@@ -183,11 +183,19 @@ void launch_chunk_reduce(const double* part, int nchunks, int64_t n, double* out
 // of the wall-shifted positions.
 // kinds[s] (0 open, 1 wall) selects per system; nullptr: all systems `wall`.
 void launch_system_bbox(const double* pos, const int64_t* sys_off, int nsys, double wall_shift,
-                        const int* kinds, int wall, double* bbox, hipStream_t s);
+                        const int* kinds, int wall, double* bbox, hipStream_t s,
+                        double* host = nullptr);
 // Records for the pair kernels; `shifted` receives the wall-shifted AoS copy.
 void launch_make_records(const double* pos, int64_t N, const int64_t* sys_off, int nsys,
                          const double* bbox, const int* kinds, int wall, double wall_shift,
                          double a, double* shifted, void* rec64, void* rec32, hipStream_t s);
+// Both for open systems of at most kPlaceMax particles each, in one launch.
+constexpr int kPlaceMax = 1024;
+void launch_place_small(const double* pos, const int64_t* sys_off, int nsys, double* bbox, double a,
+                        double* shifted, void* rec64, void* rec32, hipStream_t s);
+// y0 = x0 and y1 = x1, n entries each (null: not)
+void launch_copy2(const double* x0, double* y0, const double* x1, double* y1, int64_t n,
+                  hipStream_t s);
 // v[3i..3i+2] = 0 for the particles of open systems (kinds[s] == 0)
 void launch_zero_open_systems(double* v, int64_t N, const int64_t* sys_off, int nsys,
                               const int* kinds, hipStream_t s);

@@ -1022,49 +1022,134 @@ void launch_seg_chunk_reduce(const double* part, int nch, int64_t n, double* out
 
 // ---- setPositions -----------------------------------------------------------
 
+// Corners of a box grown by this thread's particles, reduced over the 256
+// threads: lo and hi of component c end in sh[c][0] and sh[3 + c][0].
+struct BoxSum {
+  double mn[3] = {1e300, 1e300, 1e300}, mx[3] = {-1e300, -1e300, -1e300};
+  __device__ void add(double x, double y, double z) {
+    mn[0] = fmin(mn[0], x);
+    mx[0] = fmax(mx[0], x);
+    mn[1] = fmin(mn[1], y);
+    mx[1] = fmax(mx[1], y);
+    mn[2] = fmin(mn[2], z);
+    mx[2] = fmax(mx[2], z);
+  }
+  __device__ void reduce(double (*sh)[4]) {
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    for (int c = 0; c < 3; ++c) {
+      for (int o = 32; o > 0; o >>= 1) {
+        mn[c] = fmin(mn[c], __shfl_xor(mn[c], o));
+        mx[c] = fmax(mx[c], __shfl_xor(mx[c], o));
+      }
+      if (lane == 0) {
+        sh[c][wid] = mn[c];
+        sh[3 + c][wid] = mx[c];
+      }
+    }
+    __syncthreads();
+    if (threadIdx.x < 6) {
+      const int c = threadIdx.x;
+      double v = sh[c][0];
+      for (int w = 1; w < 4; ++w) v = (c < 3) ? fmin(v, sh[c][w]) : fmax(v, sh[c][w]);
+      sh[c][0] = v;
+    }
+    __syncthreads();
+  }
+};
+
+// host (may be null): a copy of bbox in mapped host memory, where reading it
+// takes no transfer of its own.
 __global__ __launch_bounds__(256) void k_system_bbox(const double* __restrict__ pos,
                                                      const int64_t* __restrict__ off,
                                                      double wall_shift_in,
                                                      const int* __restrict__ kinds, int wall,
-                                                     double* __restrict__ bbox) {
+                                                     double* __restrict__ bbox, double* host) {
+  __shared__ double sh[6][4];
   const int s = blockIdx.x;
   const int64_t b = off[s], e = off[s + 1];
   const double wall_shift = (kinds ? kinds[s] : wall) ? wall_shift_in : 0.0;
-  double mn[3] = {1e300, 1e300, 1e300}, mx[3] = {-1e300, -1e300, -1e300};
-  for (int64_t i = b + threadIdx.x; i < e; i += blockDim.x) {
-    for (int c = 0; c < 3; ++c) {
-      double v = pos[3 * i + c];
-      if (c == 2) v -= wall_shift;
-      mn[c] = fmin(mn[c], v);
-      mx[c] = fmax(mx[c], v);
-    }
-  }
-  __shared__ double sh[6][4];
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  for (int c = 0; c < 3; ++c) {
-    for (int o = 32; o > 0; o >>= 1) {
-      mn[c] = fmin(mn[c], __shfl_xor(mn[c], o));
-      mx[c] = fmax(mx[c], __shfl_xor(mx[c], o));
-    }
-    if (lane == 0) {
-      sh[c][wid] = mn[c];
-      sh[3 + c][wid] = mx[c];
-    }
-  }
-  __syncthreads();
+  BoxSum box;
+  for (int64_t i = b + threadIdx.x; i < e; i += 256)
+    box.add(pos[3 * i], pos[3 * i + 1], pos[3 * i + 2] - wall_shift);
+  box.reduce(sh);
   if (threadIdx.x < 6) {
-    const int c = threadIdx.x;
-    double v = sh[c][0];
-    for (int w = 1; w < (int)(blockDim.x >> 6); ++w) v = (c < 3) ? fmin(v, sh[c][w]) : fmax(v, sh[c][w]);
-    bbox[6 * s + c] = v;
+    bbox[6 * s + threadIdx.x] = sh[threadIdx.x][0];
+    if (host != nullptr) host[6 * s + threadIdx.x] = sh[threadIdx.x][0];
   }
 }
 
 void launch_system_bbox(const double* pos, const int64_t* sys_off, int nsys, double wall_shift,
-                        const int* kinds, int wall, double* bbox, hipStream_t s) {
+                        const int* kinds, int wall, double* bbox, hipStream_t s, double* host) {
   if (nsys <= 0) return;
   hipLaunchKernelGGL(k_system_bbox, dim3(nsys), dim3(256), 0, s, pos, sys_off, wall_shift, kinds,
-                     wall, bbox);
+                     wall, bbox, host);
+  LM_HIP(hipGetLastError());
+}
+
+// The records of a particle of an open (wall: bottom-wall) system at (x, y, z),
+// in units of a: FP64, and FP32 relative to the centre c of its system's box.
+__device__ inline void put_records(int64_t i, int wall, double x, double y, double z, double a,
+                                   double cx, double cy, double cz, double4* __restrict__ rec64,
+                                   float4* __restrict__ rec32) {
+  const double ia = 1.0 / a;
+  if (wall) {
+    const double h = fmax(z, a) * ia;
+    const double b = fmin(fmax(z * ia, 0.0), 1.0);
+    rec64[i] = double4{x * ia, y * ia, h, b};
+    rec32[i] = float4{(float)((x - cx) * ia), (float)((y - cy) * ia), (float)h, (float)b};
+  } else {
+    rec64[i] = double4{x * ia, y * ia, z * ia, 1.0};
+    rec32[i] = float4{(float)((x - cx) * ia), (float)((y - cy) * ia), (float)((z - cz) * ia), 1.0f};
+  }
+}
+
+// Boxes, shifted positions and records of small open systems (at most
+// kPlaceMax particles) in one launch, a workgroup per system that keeps its
+// particles in registers: positions are read once, which matters where they
+// lie in host memory, and one launch less of the few that a small step has.
+__global__ __launch_bounds__(256) void k_place_small(const double* __restrict__ pos,
+                                                     const int64_t* __restrict__ off,
+                                                     double* __restrict__ bbox, double a,
+                                                     double* __restrict__ shifted,
+                                                     double4* __restrict__ rec64,
+                                                     float4* __restrict__ rec32) {
+  __shared__ double sh[6][4];
+  constexpr int kQ = kPlaceMax / 256;
+  const int s = blockIdx.x;
+  const int64_t b = off[s], e = off[s + 1];
+  double p[kQ][3];
+  BoxSum box;
+#pragma unroll
+  for (int q = 0; q < kQ; ++q) {
+    const int64_t i = b + threadIdx.x + 256 * q;
+    if (i < e) {
+#pragma unroll
+      for (int c = 0; c < 3; ++c) p[q][c] = pos[3 * i + c];
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < kQ; ++q)
+    if (b + threadIdx.x + 256 * q < e) box.add(p[q][0], p[q][1], p[q][2]);
+  box.reduce(sh);
+  if (threadIdx.x < 6) bbox[6 * s + threadIdx.x] = sh[threadIdx.x][0];
+  const double cx = 0.5 * (sh[0][0] + sh[3][0]), cy = 0.5 * (sh[1][0] + sh[4][0]),
+               cz = 0.5 * (sh[2][0] + sh[5][0]);
+#pragma unroll
+  for (int q = 0; q < kQ; ++q) {
+    const int64_t i = b + threadIdx.x + 256 * q;
+    if (i < e) {
+#pragma unroll
+      for (int c = 0; c < 3; ++c) shifted[3 * i + c] = p[q][c];
+      put_records(i, 0, p[q][0], p[q][1], p[q][2], a, cx, cy, cz, rec64, rec32);
+    }
+  }
+}
+
+void launch_place_small(const double* pos, const int64_t* sys_off, int nsys, double* bbox, double a,
+                        double* shifted, void* rec64, void* rec32, hipStream_t s) {
+  if (nsys <= 0) return;
+  hipLaunchKernelGGL(k_place_small, dim3(nsys), dim3(256), 0, s, pos, sys_off, bbox, a, shifted,
+                     static_cast<double4*>(rec64), static_cast<float4*>(rec32));
   LM_HIP(hipGetLastError());
 }
 
@@ -1089,17 +1174,8 @@ __global__ void k_make_records(const double* __restrict__ pos, int64_t N,
     shifted[3 * i + 1] = y;
     shifted[3 * i + 2] = z;
   }
-  const double ia = 1.0 / a;
-  const double cx = 0.5 * (bb[0] + bb[3]), cy = 0.5 * (bb[1] + bb[4]), cz = 0.5 * (bb[2] + bb[5]);
-  if (wall) {
-    const double h = fmax(z, a) * ia;
-    const double b = fmin(fmax(z * ia, 0.0), 1.0);
-    rec64[i] = double4{x * ia, y * ia, h, b};
-    rec32[i] = float4{(float)((x - cx) * ia), (float)((y - cy) * ia), (float)h, (float)b};
-  } else {
-    rec64[i] = double4{x * ia, y * ia, z * ia, 1.0};
-    rec32[i] = float4{(float)((x - cx) * ia), (float)((y - cy) * ia), (float)((z - cz) * ia), 1.0f};
-  }
+  put_records(i, wall, x, y, z, a, 0.5 * (bb[0] + bb[3]), 0.5 * (bb[1] + bb[4]),
+              0.5 * (bb[2] + bb[5]), rec64, rec32);
 }
 
 void launch_make_records(const double* pos, int64_t N, const int64_t* sys_off, int nsys,
@@ -1110,6 +1186,21 @@ void launch_make_records(const double* pos, int64_t N, const int64_t* sys_off, i
   hipLaunchKernelGGL(k_make_records, dim3((unsigned)((N + nt - 1) / nt)), dim3(nt), 0, s, pos, N,
                      sys_off, nsys, bbox, kinds, wall, wall_shift, a, shifted,
                      static_cast<double4*>(rec64), static_cast<float4*>(rec32));
+  LM_HIP(hipGetLastError());
+}
+
+__global__ void k_copy2(const double* __restrict__ x0, double* __restrict__ y0,
+                        const double* __restrict__ x1, double* __restrict__ y1, int64_t n) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  if (y0 != nullptr) y0[i] = x0[i];
+  if (y1 != nullptr) y1[i] = x1[i];
+}
+
+void launch_copy2(const double* x0, double* y0, const double* x1, double* y1, int64_t n,
+                  hipStream_t s) {
+  if (n <= 0 || (y0 == nullptr && y1 == nullptr)) return;
+  hipLaunchKernelGGL(k_copy2, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, x0, y0, x1, y1, n);
   LM_HIP(hipGetLastError());
 }
 

@@ -34,6 +34,7 @@ NBodySolver::NBodySolver(int px, int py, int pz) {
 }
 
 NBodySolver::~NBodySolver() {
+  if (pos_host_busy_) (void)hipStreamSynchronize(pos_host_stream_);
   if (chk_stream_) (void)hipStreamSynchronize(chk_stream_);
   for (auto& e : lz_ev_)
     if (e) (void)hipEventDestroy(e);
@@ -176,26 +177,47 @@ void NBodySolver::setPositions(const double* pos, int64_t n3, bool dev) {
   }
   bool any_wall = false, any_open = false;
   for (int k : kinds) (k ? any_wall : any_open) = true;
+  bool staged = false;  // the positions are in our pinned buffer
   if (N > 0) {
     const double* src = pos;
+    int64_t largest = 0;
+    for (int s = 0; s < nsys; ++s) largest = std::max(largest, off[s + 1] - off[s]);
+    const bool place = !any_wall && largest <= kPlaceMax;
     if (!dev) {
-      st_pos_.reserve(sizeof(double) * n3);
-      LM_HIP(hipMemcpyAsync(st_pos_.as<double>(), pos, sizeof(double) * n3,
-                            hipMemcpyHostToDevice, stream_));
-      src = st_pos_.as<double>();
+      staged = (size_t)n3 * sizeof(double) <= kStageBytes;
+      if (staged) {
+        pos_host_wait();  // kernels of the call before may still read the buffer
+        pos_host_.reserve(kStageBytes, hipHostMallocMapped | hipHostMallocCoherent);
+        std::copy(pos, pos + n3, pos_host_.as<double>());
+        src = pos_host_.device_as<double>();
+        if (!place) {  // read more than once
+          st_pos_.reserve(sizeof(double) * n3);
+          launch_copy2(src, st_pos_.as<double>(), nullptr, nullptr, n3, stream_);
+          src = st_pos_.as<double>();
+        }
+      } else {
+        st_pos_.reserve(sizeof(double) * n3);
+        LM_HIP(hipMemcpyAsync(st_pos_.as<double>(), pos, sizeof(double) * n3,
+                              hipMemcpyHostToDevice, stream_));
+        src = st_pos_.as<double>();
+      }
     }
-    sys_off_.reserve(sizeof(int64_t) * off.size());
-    LM_HIP(hipMemcpyAsync(sys_off_.as<int64_t>(), off.data(), sizeof(int64_t) * off.size(),
-                          hipMemcpyHostToDevice, stream_));
+    // the offsets only when they are not the ones the device has
+    if (off != sys_off_dev_) {
+      sys_off_dev_.clear();
+      sys_off_.reserve(sizeof(int64_t) * off.size());
+      LM_HIP(hipMemcpyAsync(sys_off_.as<int64_t>(), off.data(), sizeof(int64_t) * off.size(),
+                            hipMemcpyHostToDevice, stream_));
+      sys_off_dev_ = off;
+    }
     bbox_.reserve(sizeof(double) * 6 * nsys);
     const double shift = wall_height_;
-    launch_system_bbox(src, sys_off_.as<int64_t>(), nsys, shift, kinds_d, wall_ ? 1 : 0,
-                       bbox_.as<double>(), stream_);
     if (any_wall) {
-      std::vector<double> bb(6 * (size_t)nsys);
-      LM_HIP(hipMemcpyAsync(bb.data(), bbox_.as<double>(), sizeof(double) * bb.size(),
-                            hipMemcpyDeviceToHost, stream_));
+      bbox_host_.reserve(sizeof(double) * 6 * nsys, hipHostMallocMapped | hipHostMallocCoherent);
+      launch_system_bbox(src, sys_off_.as<int64_t>(), nsys, shift, kinds_d, wall_ ? 1 : 0,
+                         bbox_.as<double>(), stream_, bbox_host_.device_as<double>());
       LM_HIP(hipStreamSynchronize(stream_));
+      const double* bb = bbox_host_.as<double>();
       double minz = 1e300;
       for (int s = 0; s < nsys; ++s)
         if (off[s + 1] > off[s] && kinds[s]) minz = std::min(minz, bb[6 * s + 2]);
@@ -203,13 +225,20 @@ void NBodySolver::setPositions(const double* pos, int64_t n3, bool dev) {
         throw Error(
             "[Mobility] The center of a particle has fallen below the wall. Check your "
             "configuration and forces to ensure particle centers stay above the wall.");
+    } else if (!place) {
+      launch_system_bbox(src, sys_off_.as<int64_t>(), nsys, shift, kinds_d, 0, bbox_.as<double>(),
+                         stream_);
     }
     shifted_.reserve(sizeof(double) * n3);
     rec64_.reserve(sizeof(double) * 4 * N);
     rec32_.reserve(sizeof(float) * 4 * N);
-    launch_make_records(src, N, sys_off_.as<int64_t>(), nsys, bbox_.as<double>(), kinds_d,
-                        wall_ ? 1 : 0, shift, a_, shifted_.as<double>(), rec64_.as<void>(),
-                        rec32_.as<void>(), stream_);
+    if (place)
+      launch_place_small(src, sys_off_.as<int64_t>(), nsys, bbox_.as<double>(), a_,
+                         shifted_.as<double>(), rec64_.as<void>(), rec32_.as<void>(), stream_);
+    else
+      launch_make_records(src, N, sys_off_.as<int64_t>(), nsys, bbox_.as<double>(), kinds_d,
+                          wall_ ? 1 : 0, shift, a_, shifted_.as<double>(), rec64_.as<void>(),
+                          rec32_.as<void>(), stream_);
     rec_a_ = a_;
   }
   // Work lists depend on N, the system offsets and kinds only: a new
@@ -230,7 +259,25 @@ void NBodySolver::setPositions(const double* pos, int64_t n3, bool dev) {
   if (!valid)
     throw Error(
         "[Mobility] Invalid batch parameters for NBody. If in doubt, use the defaults.");
-  if (!dev || wall_) LM_HIP(hipStreamSynchronize(stream_));
+  // The caller's array may change after the return: positions that a transfer
+  // still reads are waited for, those in our own buffer are not.
+  if (staged) {
+    pos_host_stream_ = stream_;
+    pos_host_busy_ = true;
+  } else if (!dev) {
+    LM_HIP(hipStreamSynchronize(stream_));
+  }
+}
+
+void NBodySolver::pos_host_wait() {
+  if (!pos_host_busy_) return;
+  LM_HIP(hipStreamSynchronize(pos_host_stream_));
+  pos_host_busy_ = false;
+}
+
+void NBodySolver::setStream(hipStream_t s) {
+  if (s != stream_) pos_host_wait();  // work on the new stream uses the records
+  stream_ = s;
 }
 
 // Work decomposition: target tiles of 256*tpl particles x source chunks.
@@ -1040,21 +1087,44 @@ void NBodySolver::Mdot(const double* F, int64_t nF, const double* T, int64_t nT,
     return;
   }
   double *df = nullptr, *dt = nullptr;
+  const bool few = (size_t)n3 * sizeof(double) <= kStageBytes;
+  constexpr size_t kPart = kStageBytes / sizeof(double);
   if (f) {
     st_f_.reserve(sizeof(double) * n3);
     df = st_f_.as<double>();
-    LM_HIP(hipMemcpyAsync(df, f, sizeof(double) * n3, hipMemcpyHostToDevice, stream_));
   }
   if (t) {
     st_t_.reserve(sizeof(double) * n3);
     dt = st_t_.as<double>();
-    LM_HIP(hipMemcpyAsync(dt, t, sizeof(double) * n3, hipMemcpyHostToDevice, stream_));
+  }
+  if (few) {
+    // few values: a kernel fetches them from mapped host memory (no call before
+    // this one still uses it: each of them has waited for its result)
+    in_host_.reserve(2 * kStageBytes, hipHostMallocMapped | hipHostMallocCoherent);
+    if (f) std::copy(f, f + n3, in_host_.as<double>());
+    if (t) std::copy(t, t + n3, in_host_.as<double>() + kPart);
+    const double* h = in_host_.device_as<double>();
+    launch_copy2(h, df, h + kPart, dt, n3, stream_);
+  } else {
+    if (f) LM_HIP(hipMemcpyAsync(df, f, sizeof(double) * n3, hipMemcpyHostToDevice, stream_));
+    if (t) LM_HIP(hipMemcpyAsync(dt, t, sizeof(double) * n3, hipMemcpyHostToDevice, stream_));
+  }
+  const bool want_w = angular_ && W != nullptr;
+  if (few) {  // the kernels write to mapped host memory
+    out_host_.reserve(2 * kStageBytes, hipHostMallocMapped | hipHostMallocCoherent);
+    double* hu = out_host_.as<double>();
+    double* du = out_host_.device_as<double>();
+    mdot_dev(df, dt, du, angular_ ? du + kPart : nullptr);
+    LM_HIP(hipStreamSynchronize(stream_));
+    std::copy(hu, hu + n3, U);
+    if (want_w) std::copy(hu + kPart, hu + kPart + n3, W);
+    return;
   }
   st_u_.reserve(sizeof(double) * n3);
   st_w_.reserve(sizeof(double) * n3);
   mdot_dev(df, dt, st_u_.as<double>(), angular_ ? st_w_.as<double>() : nullptr);
   LM_HIP(hipMemcpyAsync(U, st_u_.as<double>(), sizeof(double) * n3, hipMemcpyDeviceToHost, stream_));
-  if (angular_ && W)
+  if (want_w)
     LM_HIP(hipMemcpyAsync(W, st_w_.as<double>(), sizeof(double) * n3, hipMemcpyDeviceToHost, stream_));
   LM_HIP(hipStreamSynchronize(stream_));
 }

@@ -126,6 +126,15 @@ def _zeros(shape, framework, device):
     return np.zeros(shape, dtype=np.float64)
 
 
+def _empty(shape, framework, device):
+    """The same for an output that the library writes in full."""
+    if framework == "torch":
+        import torch
+
+        return torch.empty(shape, dtype=torch.float64, device=device)
+    return np.empty(shape, dtype=np.float64)
+
+
 def _ptr(x):
     if x is None:
         return None
@@ -144,6 +153,7 @@ class _Solver:
     C-ABI functions lm_<prefix>_*."""
 
     _prefix = ""
+    _mdot_out = staticmethod(_zeros)
 
     def _f(self, name):
         return getattr(self._lib, "lm_" + self._prefix + "_" + name)
@@ -189,7 +199,7 @@ class _Solver:
         _ffi.check(self._f("set_positions")(self._h, arr.ptr, arr.size, arr.mem))
         _last_shape = arr.shape
 
-    def _setup_arrays(self, forces, torques):
+    def _setup_arrays(self, forces, torques, make=_zeros):
         """pythonify.h:109-149."""
         global _last_framework, _last_device
         N = self.getNumberParticles()
@@ -206,7 +216,7 @@ class _Solver:
         f = f.moved_to(mem, device)
         t = t.moved_to(mem, device)
         f_shape = _check_and_get_shape(f) if f.size > 0 else _check_and_get_shape(t)
-        mf = _zeros(f_shape, framework, device)
+        mf = make(f_shape, framework, device)
         mt = None
         if not self._include_angular:
             if t.size > 0:
@@ -215,12 +225,12 @@ class _Solver:
                     "includeAngular to true when initializing if you want to use torques")
         else:
             t_shape = f_shape if t.size == 0 else _check_and_get_shape(t)
-            mt = _zeros(t_shape, framework, device)
+            mt = make(t_shape, framework, device)
         return f, t, mf, mt, mem, device
 
     def Mdot(self, forces=None, torques=None):
         """pythonify.h:208-216 -> NBody::Mdot (mobility.h:166-182)."""
-        f, t, mf, mt, mem, device = self._setup_arrays(forces, torques)
+        f, t, mf, mt, mem, device = self._setup_arrays(forces, torques, self._mdot_out)
         self._bind_stream(mem, device)
         _ffi.check(self._f("mdot")(self._h, f.ptr, f.size, t.ptr, t.size, _ptr(mf),
                                            _ptr(mt), mem))
@@ -296,6 +306,7 @@ class NBody(_Solver):
     precision = "double"
     version = "1.1"
     _prefix = "nbody"
+    _mdot_out = staticmethod(_empty)
 
     def __init__(self, periodicityX, periodicityY, periodicityZ):
         # string2Periodicity, pythonify.h:38-52
