@@ -187,9 +187,7 @@ void NBodySolver::setPositions(const double* pos, int64_t n3, bool dev) {
       staged = (size_t)n3 * sizeof(double) <= kStageBytes;
       if (staged) {
         pos_host_wait();  // kernels of the call before may still read the buffer
-        pos_host_.reserve(kStageBytes, hipHostMallocMapped | hipHostMallocCoherent);
-        std::copy(pos, pos + n3, pos_host_.as<double>());
-        src = pos_host_.device_as<double>();
+        src = stage_in(kStagePos, pos, n3);
         if (!place) {  // read more than once
           st_pos_.reserve(sizeof(double) * n3);
           launch_copy2(src, st_pos_.as<double>(), nullptr, nullptr, n3, stream_);
@@ -273,6 +271,27 @@ void NBodySolver::pos_host_wait() {
   if (!pos_host_busy_) return;
   LM_HIP(hipStreamSynchronize(pos_host_stream_));
   pos_host_busy_ = false;
+}
+
+// One part of the mapped host buffer for n values, host and device address.  A
+// larger buffer replaces the old one once no kernel reads it.
+double* NBodySolver::stage_out(StagePart part, int64_t n, const double** host) {
+  if (n > stage_cap_) {
+    pos_host_wait();
+    const int64_t cap = std::max<int64_t>(n, std::min<int64_t>(2 * stage_cap_, kStageBytes / 8));
+    stage_cap_ = 0;
+    stage_.reserve(sizeof(double) * kStageParts * cap, hipHostMallocMapped | hipHostMallocCoherent);
+    stage_cap_ = cap;
+  }
+  if (host) *host = stage_.as<double>() + part * stage_cap_;
+  return stage_.device_as<double>() + part * stage_cap_;
+}
+
+const double* NBodySolver::stage_in(StagePart part, const double* x, int64_t n) {
+  const double* host;
+  double* dev = stage_out(part, n, &host);
+  std::copy(x, x + n, const_cast<double*>(host));
+  return dev;
 }
 
 void NBodySolver::setStream(hipStream_t s) {
@@ -508,34 +527,51 @@ void NBodySolver::ensure_sym_plan(const SymShape& sh, bool ang) {
       ps.nch = (width + least - 1) / least;
     }
     ps.diag = first ? 1 : 0;
-    std::vector<std::pair<double, SymItem>> pass_items;
-    for (int s = 0; s < nsys; ++s) {
-      const SymSys& S = systems[s];
-      const double wgt = S.wall ? 5.0 : 1.0;
-      const int ws = std::min(ob, S.hmax + 1) - oa;  // this system's offsets in the pass
-      const int cs = ws <= 0 ? 0 : (S.per > 0 ? (ws + S.per - 1) / S.per : std::min(ps.nch, ws));
-      for (int I = 0; I < S.ntiles; ++I)
-        for (int c = 0; c < cs; ++c) {
-          SymItem it;
-          it.sys = s;
-          it.tile = I;
-          it.o0 = oa + (S.per > 0 ? c * S.per : (int)((int64_t)c * ws / cs));
-          it.o1 = oa + (S.per > 0 ? std::min(ws, (c + 1) * S.per) : (int)((int64_t)(c + 1) * ws / cs));
-          it.chunk = c;
-          pass_items.emplace_back(wgt * (it.o1 - it.o0), it);
-        }
-      if (first)
-        for (int I = 0; I < S.ntiles; ++I) {
-          const double nt = (double)std::min<int64_t>(bt, S.n - (int64_t)I * bt) / bt;
-          pass_items.emplace_back(0.5 * wgt * nt * nt, SymItem{s, I, 0, 0, ps.nch});
-        }
+    // This system's offsets in the pass and its items per tile.
+    auto widths = [&](const SymSys& S, int& ws, int& cs) {
+      ws = std::min(ob, S.hmax + 1) - oa;
+      cs = ws <= 0 ? 0 : (S.per > 0 ? (ws + S.per - 1) / S.per : std::min(ps.nch, ws));
+    };
+    size_t count = 0;
+    for (const SymSys& S : systems) {
+      int ws, cs;
+      widths(S, ws, cs);
+      count += (size_t)S.ntiles * (cs + (first ? 1 : 0));
     }
-    if (nsys > 1)
-      std::stable_sort(pass_items.begin(), pass_items.end(),
-                       [](const std::pair<double, SymItem>& x, const std::pair<double, SymItem>& y) {
-                         return x.first > y.first;
-                       });
-    for (const auto& pi : pass_items) items.push_back(pi.second);
+    // Longest first in an ensemble: a counting sort by weight in eighths of an
+    // open offset.  Two walks over the items, the first to count.
+    const bool sorted = nsys > 1;
+    std::vector<int> bins;
+    auto walk = [&](auto&& put) {
+      for (int s = 0; s < nsys; ++s) {
+        const SymSys& S = systems[s];
+        const int wgt = S.wall ? 40 : 8;
+        int ws, cs;
+        widths(S, ws, cs);
+        for (int I = 0; I < S.ntiles; ++I)
+          for (int c = 0; c < cs; ++c) {
+            const int a = S.per > 0 ? c * S.per : (int)((int64_t)c * ws / cs);
+            const int b = S.per > 0 ? std::min(ws, a + S.per) : (int)((int64_t)(c + 1) * ws / cs);
+            put(wgt * (b - a), SymItem{s, I, oa + a, oa + b, c});
+          }
+        if (first)
+          for (int I = 0; I < S.ntiles; ++I) {
+            const int64_t n = std::min<int64_t>(bt, S.n - (int64_t)I * bt);
+            put((int)(wgt * n * n / (2 * bt * bt)), SymItem{s, I, 0, 0, ps.nch});
+          }
+      }
+    };
+    items.resize(items.size() + count);
+    SymItem* out = items.data() + ps.item0;
+    if (sorted) {
+      const int top = 40 * std::max(1, width);
+      bins.assign((size_t)top + 2, 0);
+      walk([&](int w, const SymItem&) { ++bins[top - w + 1]; });
+      for (size_t k = 1; k < bins.size(); ++k) bins[k] += bins[k - 1];
+      walk([&](int w, const SymItem& it) { out[bins[top - w]++] = it; });
+    } else {
+      walk([&](int, const SymItem& it) { *out++ = it; });
+    }
     ps.nitems = (int)items.size() - ps.item0;
     plan.max_slabs = std::max(plan.max_slabs, (size_t)(ps.nch + ps.diag + width));
     plan.passes.push_back(ps);
@@ -1088,7 +1124,6 @@ void NBodySolver::Mdot(const double* F, int64_t nF, const double* T, int64_t nT,
   }
   double *df = nullptr, *dt = nullptr;
   const bool few = (size_t)n3 * sizeof(double) <= kStageBytes;
-  constexpr size_t kPart = kStageBytes / sizeof(double);
   if (f) {
     st_f_.reserve(sizeof(double) * n3);
     df = st_f_.as<double>();
@@ -1098,33 +1133,28 @@ void NBodySolver::Mdot(const double* F, int64_t nF, const double* T, int64_t nT,
     dt = st_t_.as<double>();
   }
   if (few) {
-    // few values: a kernel fetches them from mapped host memory (no call before
-    // this one still uses it: each of them has waited for its result)
-    in_host_.reserve(2 * kStageBytes, hipHostMallocMapped | hipHostMallocCoherent);
-    if (f) std::copy(f, f + n3, in_host_.as<double>());
-    if (t) std::copy(t, t + n3, in_host_.as<double>() + kPart);
-    const double* h = in_host_.device_as<double>();
-    launch_copy2(h, df, h + kPart, dt, n3, stream_);
-  } else {
-    if (f) LM_HIP(hipMemcpyAsync(df, f, sizeof(double) * n3, hipMemcpyHostToDevice, stream_));
-    if (t) LM_HIP(hipMemcpyAsync(dt, t, sizeof(double) * n3, hipMemcpyHostToDevice, stream_));
-  }
-  const bool want_w = angular_ && W != nullptr;
-  if (few) {  // the kernels write to mapped host memory
-    out_host_.reserve(2 * kStageBytes, hipHostMallocMapped | hipHostMallocCoherent);
-    double* hu = out_host_.as<double>();
-    double* du = out_host_.device_as<double>();
-    mdot_dev(df, dt, du, angular_ ? du + kPart : nullptr);
+    // a kernel fetches them from the host buffer (no call before this one still
+    // uses these parts of it: each has waited for its result), and the product
+    // writes its results there
+    const double* hf = f ? stage_in(kStageF, f, n3) : nullptr;
+    const double* ht = t ? stage_in(kStageT, t, n3) : nullptr;
+    launch_copy2(hf, df, ht, dt, n3, stream_);
+    const double *hu, *hw;
+    double* du = stage_out(kStageU, n3, &hu);
+    double* dw = stage_out(kStageW, n3, &hw);
+    mdot_dev(df, dt, du, angular_ ? dw : nullptr);
     LM_HIP(hipStreamSynchronize(stream_));
     std::copy(hu, hu + n3, U);
-    if (want_w) std::copy(hu + kPart, hu + kPart + n3, W);
+    if (angular_ && W) std::copy(hw, hw + n3, W);
     return;
   }
+  if (f) LM_HIP(hipMemcpyAsync(df, f, sizeof(double) * n3, hipMemcpyHostToDevice, stream_));
+  if (t) LM_HIP(hipMemcpyAsync(dt, t, sizeof(double) * n3, hipMemcpyHostToDevice, stream_));
   st_u_.reserve(sizeof(double) * n3);
   st_w_.reserve(sizeof(double) * n3);
   mdot_dev(df, dt, st_u_.as<double>(), angular_ ? st_w_.as<double>() : nullptr);
   LM_HIP(hipMemcpyAsync(U, st_u_.as<double>(), sizeof(double) * n3, hipMemcpyDeviceToHost, stream_));
-  if (want_w)
+  if (angular_ && W)
     LM_HIP(hipMemcpyAsync(W, st_w_.as<double>(), sizeof(double) * n3, hipMemcpyDeviceToHost, stream_));
   LM_HIP(hipStreamSynchronize(stream_));
 }

@@ -330,11 +330,14 @@ class NBodySolver {
   // Host arrays of up to kStageBytes go through mapped host memory, which kernels
   // read and write, instead of a transfer each.  A step (setPositions and Mdot,
   // open, FP64) of 96 particles takes 28 us against 64 with transfers, of 4097
-  // 61 against 96, of 16384 298 against 383; the buffers (6 of this size at
-  // most) stay small.
+  // 61 against 96, of 16384 298 against 383; the buffer stays small.
   static constexpr size_t kStageBytes = 24 * 16384;
-  HostBuf pos_host_, in_host_, out_host_, bbox_host_;
-  hipStream_t pos_host_stream_ = nullptr;  // of the kernels that read pos_host_
+  enum StagePart : int { kStagePos, kStageF, kStageT, kStageU, kStageW, kStageParts };
+  HostBuf stage_, bbox_host_;
+  int64_t stage_cap_ = 0;  // values per part of stage_
+  double* stage_out(StagePart part, int64_t n, const double** host);
+  const double* stage_in(StagePart part, const double* x, int64_t n);
+  hipStream_t pos_host_stream_ = nullptr;  // of the kernels that read the positions there
   bool pos_host_busy_ = false;
   void pos_host_wait();
   std::vector<int64_t> sys_off_dev_;  // what sys_off_ holds
