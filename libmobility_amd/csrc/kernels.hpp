@@ -126,6 +126,18 @@ struct SymRows {
   int32_t np;
   int32_t sys;
 };
+// Items of a tile in a pass over `ws` of the system's offsets (from offset oa), and
+// the c-th of them; nch: the pass's chunks.
+__host__ __device__ inline int sym_ring_chunks(const SymSys& S, int ws, int nch) {
+  return ws <= 0 ? 0 : (S.per > 0 ? (ws + S.per - 1) / S.per : (nch < ws ? nch : ws));
+}
+__host__ __device__ inline SymItem sym_ring_item(const SymSys& S, int sys, int tile, int c, int cs,
+                                                 int oa, int ws) {
+  const int a = S.per > 0 ? c * S.per : (int)((int64_t)c * ws / cs);
+  int b = S.per > 0 ? a + S.per : (int)((int64_t)(c + 1) * ws / cs);
+  if (b > ws) b = ws;
+  return SymItem{sys, tile, oa + a, oa + b, c};
+}
 struct SymArgs {
   int fp32;
   int tpl;
@@ -153,6 +165,10 @@ struct SymArgs {
 // The open translational block in FP32, and (open blocks) the order of
 // operations that plain Lanczos products keep; 4 waves per workgroup.
 void launch_pair_sym(const SymArgs& a, hipStream_t s);
+// The items of a pass over offsets [oa, ob) of one system, tile by tile, then its
+// diagonal tiles; also the system itself and its row blocks.
+void launch_sym_items(SymItem* items, int nitems, const SymSys& S, int oa, int ob, int nch, int diag,
+                      SymSys* sys, SymRows* rows, int64_t nrows, hipStream_t s);
 // Every form, in symmetric units.
 void launch_pair_sym_unit(const SymArgs& a, hipStream_t s);
 // Per row block: out (= or +=, accumulate) the system's target slabs of the

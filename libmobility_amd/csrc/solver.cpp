@@ -503,13 +503,14 @@ void NBodySolver::ensure_sym_plan(const SymShape& sh, bool ang) {
     S.wall = s < (int)sys_kind_host_.size() ? sys_kind_host_[s] : (wall_ ? 1 : 0);
     S.per = sh.per[S.wall ? 1 : 0];
     S.pad = 0;
-    for (int64_t p0 = b; p0 < e; p0 += kPairThreads)
+    for (int64_t p0 = b; p0 < e && nsys > 1; p0 += kPairThreads)
       rows.push_back(SymRows{p0, (int32_t)std::min<int64_t>(kPairThreads, e - p0), s});
   }
   const double unit = 8.0 * 3.0 * (double)N_ * (ang ? 2.0 : 1.0);  // bytes per slab (U and W)
   const double per_offset = 1.0 + (h > 0 ? (double)nch / h : 0.0);
   const int span = std::max(1, (int)(((double)sym_budget_ / unit - 2.0) / per_offset));
   std::vector<SymItem> items;
+  size_t nitems = 0;
   plan.passes.clear();
   plan.max_slabs = 0;
   int oa = 1;
@@ -518,7 +519,7 @@ void NBodySolver::ensure_sym_plan(const SymShape& sh, bool ang) {
     const bool first = oa == 1;
     const int width = ob - oa;
     SymPass ps;
-    ps.item0 = (int)items.size();
+    ps.item0 = (int)nitems;
     ps.oa = oa;
     ps.ob = ob;
     ps.nch = width > 0 ? std::max(1, std::min(width, (int)(((int64_t)nch * width + h - 1) / h))) : 0;
@@ -530,7 +531,7 @@ void NBodySolver::ensure_sym_plan(const SymShape& sh, bool ang) {
     // This system's offsets in the pass and its items per tile.
     auto widths = [&](const SymSys& S, int& ws, int& cs) {
       ws = std::min(ob, S.hmax + 1) - oa;
-      cs = ws <= 0 ? 0 : (S.per > 0 ? (ws + S.per - 1) / S.per : std::min(ps.nch, ws));
+      cs = sym_ring_chunks(S, ws, ps.nch);
     };
     size_t count = 0;
     for (const SymSys& S : systems) {
@@ -538,10 +539,10 @@ void NBodySolver::ensure_sym_plan(const SymShape& sh, bool ang) {
       widths(S, ws, cs);
       count += (size_t)S.ntiles * (cs + (first ? 1 : 0));
     }
-    // Longest first in an ensemble: a counting sort by weight in eighths of an
-    // open offset.  Two walks over the items, the first to count.
-    const bool sorted = nsys > 1;
-    std::vector<int> bins;
+    nitems += count;
+    ps.nitems = (int)count;
+    // An ensemble's items go longest first: a counting sort by weight in eighths
+    // of an open offset, two walks over the items, the first to count.
     auto walk = [&](auto&& put) {
       for (int s = 0; s < nsys; ++s) {
         const SymSys& S = systems[s];
@@ -550,9 +551,8 @@ void NBodySolver::ensure_sym_plan(const SymShape& sh, bool ang) {
         widths(S, ws, cs);
         for (int I = 0; I < S.ntiles; ++I)
           for (int c = 0; c < cs; ++c) {
-            const int a = S.per > 0 ? c * S.per : (int)((int64_t)c * ws / cs);
-            const int b = S.per > 0 ? std::min(ws, a + S.per) : (int)((int64_t)(c + 1) * ws / cs);
-            put(wgt * (b - a), SymItem{s, I, oa + a, oa + b, c});
+            const SymItem it = sym_ring_item(S, s, I, c, cs, oa, ws);
+            put(wgt * (it.o1 - it.o0), it);
           }
         if (first)
           for (int I = 0; I < S.ntiles; ++I) {
@@ -561,32 +561,39 @@ void NBodySolver::ensure_sym_plan(const SymShape& sh, bool ang) {
           }
       }
     };
-    items.resize(items.size() + count);
-    SymItem* out = items.data() + ps.item0;
-    if (sorted) {
+    if (nsys > 1) {
+      items.resize(nitems);
+      SymItem* out = items.data() + ps.item0;
       const int top = 40 * std::max(1, width);
-      bins.assign((size_t)top + 2, 0);
+      std::vector<int> bins((size_t)top + 2, 0);
       walk([&](int w, const SymItem&) { ++bins[top - w + 1]; });
       for (size_t k = 1; k < bins.size(); ++k) bins[k] += bins[k - 1];
       walk([&](int w, const SymItem& it) { out[bins[top - w]++] = it; });
-    } else {
-      walk([&](int, const SymItem& it) { *out++ = it; });
     }
-    ps.nitems = (int)items.size() - ps.item0;
     plan.max_slabs = std::max(plan.max_slabs, (size_t)(ps.nch + ps.diag + width));
     plan.passes.push_back(ps);
     oa = ob;
   } while (oa <= h);
-  plan.items.reserve(sizeof(SymItem) * std::max<size_t>(items.size(), 1));
+  const int64_t nrows = nsys > 1 ? (int64_t)rows.size() : (N_ + kPairThreads - 1) / kPairThreads;
+  plan.items.reserve(sizeof(SymItem) * std::max<size_t>(nitems, 1));
   plan.sys.reserve(sizeof(SymSys) * systems.size());
-  plan.rows.reserve(sizeof(SymRows) * rows.size());
-  LM_HIP(hipMemcpyAsync(plan.items.as<void>(), items.data(), sizeof(SymItem) * items.size(),
-                        hipMemcpyHostToDevice, stream_));
-  LM_HIP(hipMemcpyAsync(plan.sys.as<void>(), systems.data(), sizeof(SymSys) * systems.size(),
-                        hipMemcpyHostToDevice, stream_));
-  LM_HIP(hipMemcpyAsync(plan.rows.as<void>(), rows.data(), sizeof(SymRows) * rows.size(),
-                        hipMemcpyHostToDevice, stream_));
-  LM_HIP(hipStreamSynchronize(stream_));  // the host vectors go out of scope (items are kept)
+  plan.rows.reserve(sizeof(SymRows) * std::max<int64_t>(nrows, 1));
+  if (nsys > 1) {
+    LM_HIP(hipMemcpyAsync(plan.items.as<void>(), items.data(), sizeof(SymItem) * items.size(),
+                          hipMemcpyHostToDevice, stream_));
+    LM_HIP(hipMemcpyAsync(plan.sys.as<void>(), systems.data(), sizeof(SymSys) * systems.size(),
+                          hipMemcpyHostToDevice, stream_));
+    LM_HIP(hipMemcpyAsync(plan.rows.as<void>(), rows.data(), sizeof(SymRows) * rows.size(),
+                          hipMemcpyHostToDevice, stream_));
+    LM_HIP(hipStreamSynchronize(stream_));  // the host vectors go out of scope (items are kept)
+  } else {
+    // one system: a kernel writes what its formula gives (the upload of some
+    // thousand items took 0.13 ms of a first product)
+    for (const SymPass& ps : plan.passes)
+      launch_sym_items(plan.items.as<SymItem>() + ps.item0, ps.nitems, systems[0], ps.oa, ps.ob,
+                       ps.nch, ps.diag, plan.sys.as<SymSys>(), plan.rows.as<SymRows>(), nrows,
+                       stream_);
+  }
   plan.host_items = std::move(items);
   plan.N = N_;
   plan.structure = struct_id_;
@@ -597,8 +604,8 @@ void NBodySolver::ensure_sym_plan(const SymShape& sh, bool ang) {
   plan.hmax = h;
   plan.ang = ang ? 1 : 0;
   plan.budget = sym_budget_;
-  plan.nitems = (int)plan.host_items.size();
-  plan.nrows = (int)rows.size();
+  plan.nitems = (int)nitems;
+  plan.nrows = (int)nrows;
   plan.active_valid = false;
 }
 

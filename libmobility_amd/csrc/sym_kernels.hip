@@ -39,6 +39,35 @@ __global__ __launch_bounds__(64 * NW, kSymWaves<R>) void k_pair_sym_unit(SymArgs
   if constexpr (KIND != 1) sym_unit<R, false, BLK, TPL, NW>(it, S, a, lds);
 }
 
+__global__ __launch_bounds__(256) void k_sym_items(SymItem* __restrict__ items, int nitems, SymSys S,
+                                                  int oa, int ws, int cs, int nch, SymSys* sys,
+                                                  SymRows* __restrict__ rows, int64_t nrows) {
+  const int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (k == 0) *sys = S;
+  const int ring = S.ntiles * cs;
+  if (k < ring)
+    items[k] = sym_ring_item(S, 0, (int)(k / cs), (int)(k % cs), cs, oa, ws);
+  else if (k < nitems)
+    items[k] = SymItem{0, (int)k - ring, 0, 0, nch};
+  if (k < nrows) {
+    const int64_t left = S.n - 256 * k;
+    rows[k] = SymRows{S.off + 256 * k, (int32_t)(left < 256 ? left : 256), 0};
+  }
+}
+
+void launch_sym_items(SymItem* items, int nitems, const SymSys& S, int oa, int ob, int nch, int diag,
+                      SymSys* sys, SymRows* rows, int64_t nrows, hipStream_t s) {
+  const int ws = (ob < S.hmax + 1 ? ob : S.hmax + 1) - oa;
+  const int cs = sym_ring_chunks(S, ws, nch);
+  if (nitems != S.ntiles * (cs + diag))
+    throw Error("[libmobility_amd] symmetric work list of another size");
+  const int64_t n = nitems > nrows ? nitems : nrows;
+  if (n <= 0) return;
+  hipLaunchKernelGGL(k_sym_items, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, items, nitems,
+                     S, oa, ws, cs, nch, sys, rows, nrows);
+  LM_HIP(hipGetLastError());
+}
+
 template <class R, int KIND, int BLK>
 static void launch_unit_shape(const SymArgs& a, hipStream_t s) {
   const dim3 grid((unsigned)a.nitems);

@@ -1,0 +1,72 @@
+"""The symmetric evaluation with its default shapes, forced on at sizes around
+its tiles (64 particles per wave, one wave per item below 16384 particles):
+one tile, odd and even tile counts, nearly empty last tiles, several passes
+over the ring, one system and ensembles, against the CPU oracle."""
+import numpy as np
+import pytest
+
+import oracle
+
+pytestmark = pytest.mark.gpu
+
+ETA, A = 0.9, 1.1
+TOL = {"fp64": 1e-12, "fp32": 1e-5}
+
+
+def _cloud(N, wall, seed):
+    rng = np.random.default_rng(seed)
+    pos = rng.uniform(0, 2.2 * A * max(1.0, N ** (1 / 3)), (N, 3))
+    if wall:
+        pos[:, 2] = rng.uniform(0.3 * A, 8 * A, N)
+    return pos, rng.normal(size=(N, 3)), rng.normal(size=(N, 3))
+
+
+def _check(s, pos, F, T, angular, wall, sizes, tol):
+    for f, t in ((F, None), (F, T), (None, T)) if angular else ((F, None),):
+        U, W = s.Mdot(f, t)
+        assert s.lastPairSymmetric()
+        Uo, Wo = oracle.mdot(pos, ETA, A, F=f, T=t, angular=angular, wall=wall, sys_sizes=sizes)
+        for got, ref in ((U, Uo), (W, Wo)) if angular else ((U, Uo),):
+            assert np.linalg.norm(got.ravel() - ref) <= tol * max(np.linalg.norm(ref), 1e-300)
+
+
+@pytest.mark.parametrize("N,slabs", [(1, 0), (64, 0), (65, 0), (128, 0), (129, 0), (255, 0),
+                                     (257, 0), (513, 0), (1000, 0), (1000, 6), (2111, 9)])
+@pytest.mark.parametrize("wall,angular", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_one_system_vs_oracle(N, slabs, wall, angular, precision):
+    """slabs: room for that many partial sums, so the ring takes several passes."""
+    from libmobility_amd import NBody
+    pos, F, T = _cloud(N, wall, N)
+    s = NBody("open", "open", "single_wall" if wall else "open")
+    s.setParameters(**({"wallHeight": 0.0} if wall else {}))
+    s.setPairPrecision(precision)
+    s.setPairSymmetric(1, memoryBytes=slabs * 24 * N * (2 if angular else 1))
+    s.initialize(viscosity=ETA, hydrodynamicRadius=A, includeAngular=angular)
+    s.setPositions(pos)
+    _check(s, pos, F, T, angular, wall, None, TOL[precision])
+
+
+@pytest.mark.parametrize("sizes", [(64, 65, 0, 1, 300), (1500, 130, 129), (200,) * 7])
+@pytest.mark.parametrize("kinds", ["open", "wall", "mixed"])
+@pytest.mark.parametrize("angular", [False, True])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_ensembles_vs_oracle(sizes, kinds, angular, precision):
+    from libmobility_amd import NBody
+    walls = [kinds == "wall" or (kinds == "mixed" and k % 2 == 0) for k in range(len(sizes))]
+    parts = [_cloud(n, w, 7 + k) for k, (n, w) in enumerate(zip(sizes, walls))]
+    pos, F, T = (np.concatenate([p[k] for p in parts]) for k in range(3))
+    s = NBody("open", "open", "single_wall")
+    s.setParameters(wallHeight=0.0)
+    s.setPairPrecision(precision)
+    s.setPairSymmetric(1)
+    s.initialize(viscosity=ETA, hydrodynamicRadius=A, includeAngular=angular)
+    s.setSystems(sizes, ["single_wall" if w else "open" for w in walls])
+    s.setPositions(pos)
+    for f, t in ((F, None), (F, T)) if angular else ((F, None),):
+        U, W = s.Mdot(f, t)
+        assert s.lastPairSymmetric()
+        Uo, Wo = oracle.mdot(pos, ETA, A, F=f, T=t, angular=angular, wall=walls, sys_sizes=sizes)
+        assert np.linalg.norm(U.ravel() - Uo) <= TOL[precision] * np.linalg.norm(Uo)
+        if angular:
+            assert np.linalg.norm(W.ravel() - Wo) <= TOL[precision] * np.linalg.norm(Wo)
