@@ -17,6 +17,21 @@ struct PairItem {
   int32_t sys;   // system index (items of inactive systems are skipped)
 };
 
+// A Lanczos step that the product after it finishes (lanczos_head.hpp):
+// w = M v_i - beta[i-1] v_{i-1}, alpha[i] = w . v_i, w -= alpha[i] v_i, beta[i] =
+// ||w|| with the breakdown rule, v_{i+1} = w / beta[i] or e1.
+struct LanczosScalars;
+constexpr int kLanczosHeadMax = 4096;  // largest n
+struct LanczosHead {
+  const double* w;   // M v_i
+  const double* v;   // v_i
+  const double* vp;  // v_{i-1} (not read for i = 0)
+  double* v_next;
+  LanczosScalars* sc;
+  int n;  // entries; 0: no step
+  int i;
+};
+
 struct PairArgs {
   int wall;       // 0 open RPY, 1 bottom wall, 2 per item (mixed ensembles)
   int persistent; // 1: grid of `grid` workgroups fetching items through `counter`
@@ -39,6 +54,9 @@ struct PairArgs {
   // never).  Its outputs are then undefined.
   const int* stop;
   double t0, rt0, r0;
+  // n > 0: the launch first finishes this Lanczos step, and the forces (and
+  // torques) of the product are the vector that comes out of it (F, T unused)
+  LanczosHead head;
 };
 
 constexpr int kPairThreads = 256;  // threads per workgroup = sources per LDS tile

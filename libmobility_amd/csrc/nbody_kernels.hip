@@ -16,6 +16,7 @@
 #include <type_traits>
 
 #include "kernels.hpp"
+#include "lanczos_head.hpp"
 #include "lm_common.hpp"
 #include "pair_device.hpp"
 #include "pair_math.hpp"
@@ -655,6 +656,31 @@ __global__ __launch_bounds__(kPairThreads) void k_pair_sym(SymArgs a) {
     sym_item_gen<R, BLK, TPL>(it, a, lds.pos, lds.f, lds.t, lds.red);
 }
 
+// Products of plain Lanczos over small open systems: the launch first finishes
+// the step before (lanczos_head.hpp), in every workgroup, and reads the forces
+// from LDS.  1024 particles, FP64, a step and a product: 17.8 us in two launches
+// (this and the chunk sums), 20.4 as product and one-workgroup step.
+template <class R, int BLK>
+__global__ __launch_bounds__(kPairThreads) void k_pair_head(
+    const PairItem* __restrict__ items, const typename Rec<R>::T* __restrict__ pos,
+    double* __restrict__ U, double* __restrict__ W, int64_t slab, const int* stop, double t0,
+    double rt0, double r0, LanczosHead h) {
+  using R4 = typename Rec<R>::T;
+  constexpr bool kNeedT = (BLK & (kUT | kWT)) != 0;
+  __shared__ R4 s_pos[kPairThreads];
+  __shared__ R4 s_f[kPairThreads];
+  __shared__ R4 s_t[kNeedT ? kPairThreads : 1];
+  __shared__ double s_v[kLanczosHeadMax];
+  __shared__ double sh[2][16];
+  __shared__ int s_stop;
+  // one read per workgroup, so that all its threads take the same branch
+  if (threadIdx.x == 0) s_stop = stop != nullptr ? *(volatile const int*)stop : 0;
+  const PairItem it = items[blockIdx.x];
+  lanczos_head(h, s_v, sh, blockIdx.x == 0);
+  if (s_stop != 0) return;  // read after the barriers of the head
+  pair_item<R, false, BLK, 1>(it, pos, s_v, s_v + slab, U, W, slab, t0, rt0, r0, s_pos, s_f, s_t);
+}
+
 // ---- several force vectors per pass (translational block) ----------------------
 // Same tiling as pair_item; each pair's geometry and coefficients are computed
 // once and applied to the NR force vectors staged side by side in LDS.
@@ -866,8 +892,28 @@ static void launch_pair_kind(const PairArgs& a, hipStream_t s) {
   }
 }
 
+template <class R, int BLK>
+static void launch_pair_head(const PairArgs& a, hipStream_t s) {
+  hipLaunchKernelGGL((k_pair_head<R, BLK>), dim3(a.nitems), dim3(kPairThreads), 0, s, a.items,
+                     static_cast<const typename Rec<R>::T*>(a.pos), a.U, a.W, a.slab, a.stop, a.t0,
+                     a.rt0, a.r0, a.head);
+  LM_HIP(hipGetLastError());
+}
+
 void launch_pair(const PairArgs& a, hipStream_t s) {
   if (a.nitems <= 0) return;
+  if (a.head.n > 0) {
+    constexpr int kAll = kUF | kUT | kWT | kWF;
+    if (a.wall != 0 || a.persistent || a.tpl != 1 || a.active || a.slab <= 0 ||
+        a.head.n > kLanczosHeadMax || (a.blocks != kUF && a.blocks != kAll) ||
+        a.head.n != a.slab * (a.blocks == kAll ? 2 : 1))
+      throw Error("[libmobility_amd] this product cannot finish a Lanczos step");
+    if (a.fp32)
+      a.blocks == kUF ? launch_pair_head<float, kUF>(a, s) : launch_pair_head<float, kAll>(a, s);
+    else
+      a.blocks == kUF ? launch_pair_head<double, kUF>(a, s) : launch_pair_head<double, kAll>(a, s);
+    return;
+  }
   if (a.fp32)
     launch_pair_kind<float>(a, s);
   else

@@ -889,6 +889,8 @@ void NBodySolver::launch_pair_items(const PairItem* list, int count, int tpl, in
   a.nitems = count;
   a.active = pair_active_;
   a.stop = a.persistent ? nullptr : pair_stop_;
+  a.head = pair_head_;
+  pair_head_.n = 0;
   a.t0 = t0_;
   a.rt0 = rt0_;
   a.r0 = r0_;
@@ -1336,14 +1338,31 @@ int NBodySolver::lanczos_run(const double* z, double** result) {
     LM_HIP(hipStreamWaitEvent(stream_, lz_ev_[(nbatches - 1) % kLzSlots], 0));
     return last_iters_;
   };
+  // Where the next product can finish a step (small open systems), steps that no
+  // check follows are left to it; `head_step` is the one that waits for that.
+  const bool lazy = fused && !pre_on() && !reorth_ && n <= kLanczosHeadMax && head_route();
+  int head_step = -1;
+  struct HeadGuard {
+    LanczosHead& h;
+    ~HeadGuard() { h.n = 0; }
+  } head_guard{pair_head_};
   for (int i = 0; i < iter_limit_; ++i) {
     ensure_cols(i + 2);
     V = V_.as<double>();
     const double* vi = V + (int64_t)i * n;
     const double* vp = i > 0 ? V + (int64_t)(i - 1) * n : nullptr;
     double* vn = V + (int64_t)(i + 1) * n;
+    const bool checked = (i >= check || cb_ != nullptr) &&
+                         (i - (bfirst < 0 ? i : bfirst) + 1 >= batch || i == iter_limit_ - 1);
     if (fused) {
-      defer_chunk_sum_ = defer;
+      if (head_step >= 0) {
+        const int h = head_step;
+        pair_head_ = LanczosHead{w, V + (int64_t)h * n, h > 0 ? V + (int64_t)(h - 1) * n : nullptr,
+                                 V + (int64_t)(h + 1) * n, sc, (int)n, h};
+        head_step = -1;
+      }
+      const bool leave = lazy && !checked;
+      defer_chunk_sum_ = defer && !leave;
       try {
         lanczos_product(vi, w);
       } catch (...) {
@@ -1352,6 +1371,10 @@ int NBodySolver::lanczos_run(const double* z, double** result) {
         throw;
       }
       defer_chunk_sum_ = false;
+      if (pair_head_.n != 0) {
+        drain();
+        throw Error("[libmobility_amd] a Lanczos step was left unfinished");
+      }
       LanczosStepArgs sa{};
       if (deferred_nch_ > 0) {
         sa.slab_u = part_u_.as<double>();
@@ -1370,7 +1393,10 @@ int NBodySolver::lanczos_run(const double* z, double** result) {
       sa.n = n;
       sa.i = i;
       sa.sc = sc;
-      launch_lanczos_step(sa, stream_);  // LanczosAlgorithm.cu:120-153
+      if (leave)
+        head_step = i;
+      else
+        launch_lanczos_step(sa, stream_);  // LanczosAlgorithm.cu:120-153
     } else {
       lanczos_product(vi, w);
       launch_lanczos_update(w, vi, vp, vn, n, i, partial, sc, stream_);
@@ -1423,6 +1449,16 @@ int NBodySolver::lanczos_run(const double* z, double** result) {
     if (settle_oldest()) return finish();
   drain();
   throw Error("[Lanczos] Could not converge");
+}
+
+// Whether the products of a plain recurrence can finish the step before them:
+// ordered pair kernel over open systems, one target per lane, chunk slabs (which
+// keep w apart from what the launch writes).
+bool NBodySolver::head_route() const {
+  if (kind_code() != 0 || use_persistent() || autotune_ || tile_tpl_ > 1 || algorithm_ == kNaive ||
+      pair_active_ != nullptr || sym_mode_ == 1)
+    return false;
+  return resolve_nch(1, algorithm_ == kBlock ? 32 : tile_nch_) > 1;
 }
 
 // w = M v ; torques are stored after the forces (MobilityInterface.h:164-176).

@@ -322,6 +322,9 @@ class NBodySolver {
   int deferred_nch_ = 0;
   // device flag that stops non-persistent pair workgroups (PairArgs::stop)
   const int* pair_stop_ = nullptr;
+  // Lanczos step that the next product finishes first (n = 0: none)
+  LanczosHead pair_head_{};
+  bool head_route() const;
   int tile_tpl_ = 0, tile_nch_ = 0;  // user override (0 = auto)
   bool autotune_ = false;
   std::map<std::tuple<int64_t, int, int, int, int>, std::pair<int, int>> tuned_;
