@@ -95,6 +95,31 @@ struct WideArgs {
 };
 void launch_pair_wide(const WideArgs& a, hipStream_t s);
 
+// A Lanczos step around the product of small bottom-wall systems, two launches:
+// the wide kernel normalises the vector that the step before left (v_i = w /
+// beta[i-1], or e1 after a breakdown), multiplies and subtracts beta[i-1] v_{i-1},
+// and launch_wide_orthogonalise subtracts alpha[i] v_i.  Both leave partial sums
+// that the launch after them adds.  WideArgs gives the systems and the blocks
+// (kUF or all four; kind 1; F, T, U, W unused).
+constexpr int kWideStepMax = 16384;  // entries: at most 64 partials of ||w||^2
+struct WideStep {
+  const double* w;   // what step i - 1 left; i = 0: not read
+  const double* e1;  // n entries: 1, 0, 0, ...
+  double* v;         // v_i: read for i = 0, else written
+  const double* vp;  // v_{i-1}, for i > 0
+  double* w_out;     // n entries, not w
+  double* partial_a;        // out: one per unit
+  const double* partial_b;  // in, for i > 0
+  LanczosScalars* sc;
+  int n, i;
+};
+void launch_wide_step(const WideArgs& a, const WideStep& h, hipStream_t s);
+// alpha[i] from the na partials; w -= alpha[i] v_i; partials of ||w||^2
+void launch_wide_orthogonalise(double* w, const double* v, int n, int i, const double* partial_a,
+                               int na, double* partial_b, LanczosScalars* sc, const int* stop,
+                               hipStream_t s);
+void launch_unit_vector(double* e1, int64_t n, hipStream_t s);
+
 // Translational product with several force vectors in one pass over the pairs:
 // U_r = t0 * M F_r, r < nrhs.  F holds nrhs consecutive 3N vectors; the
 // partial of vector r and chunk c goes to U + (r * nch + c) * n3.

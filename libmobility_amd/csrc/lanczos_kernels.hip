@@ -237,6 +237,47 @@ void launch_lanczos_update(double* w, const double* v_i, const double* v_prev, d
   LM_HIP(hipGetLastError());
 }
 
+__global__ __launch_bounds__(kRT) void k_wide_orthogonalise(double* __restrict__ w,
+                                                           const double* __restrict__ v, int n,
+                                                           int i,
+                                                           const double* __restrict__ partial_a,
+                                                           int na, double* partial_b,
+                                                           LanczosScalars* sc, const int* stop) {
+  __shared__ double sh[kRT / 64];
+  __shared__ int s_stop;
+  if (threadIdx.x == 0) s_stop = stop != nullptr ? *(volatile const int*)stop : 0;
+  const int k = blockIdx.x * kRT + threadIdx.x;
+  double wk = k < n ? w[k] : 0.0;
+  const double vk = k < n ? v[k] : 0.0;
+  const double alpha = sum_partials(partial_a, na, sh);
+  if (s_stop != 0) return;  // read after the barriers of the sum
+  if (blockIdx.x == 0 && threadIdx.x == 0) sc->alpha[i] = alpha;
+  wk -= alpha * vk;
+  if (k < n) w[k] = wk;
+  const double p = block_sum(wk * wk, sh);
+  if (threadIdx.x == 0) partial_b[blockIdx.x] = p;
+}
+
+void launch_wide_orthogonalise(double* w, const double* v, int n, int i, const double* partial_a,
+                               int na, double* partial_b, LanczosScalars* sc, const int* stop,
+                               hipStream_t s) {
+  static_assert(kRT == kPairThreads && kWideStepMax == 64 * kRT, "partials of one wave");
+  hipLaunchKernelGGL(k_wide_orthogonalise, dim3((n + kRT - 1) / kRT), dim3(kRT), 0, s, w, v, n, i,
+                     partial_a, na, partial_b, sc, stop);
+  LM_HIP(hipGetLastError());
+}
+
+__global__ void k_unit_vector(double* e1, int64_t n) {
+  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (k < n) e1[k] = k == 0 ? 1.0 : 0.0;
+}
+
+void launch_unit_vector(double* e1, int64_t n, hipStream_t s) {
+  if (n <= 0) return;
+  hipLaunchKernelGGL(k_unit_vector, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, e1, n);
+  LM_HIP(hipGetLastError());
+}
+
 // Sum over a workgroup of kLanczosFusedThreads in a fixed order, in every
 // thread; `sh` holds one double per wave and is not reused.
 constexpr int kFusedWaves = kLanczosFusedThreads / 64;

@@ -830,8 +830,7 @@ void NBodySolver::ensure_wide_plan() {
   wide_.N = N_;
 }
 
-void NBodySolver::launch_wide(int blocks, bool fp32, const void* rec, const double* F,
-                              const double* T, double* U, double* W) {
+WideArgs NBodySolver::wide_args(int blocks, bool fp32, const void* rec) {
   ensure_wide_plan();
   WideArgs a{};
   a.kind = kind_code();
@@ -839,10 +838,6 @@ void NBodySolver::launch_wide(int blocks, bool fp32, const void* rec, const doub
   a.blocks = blocks;
   a.split = wide_.nunits >= kWideWaveUnits && mean_system_size() <= kWideWaveMean ? 1 : 4;
   a.pos = rec;
-  a.F = F;
-  a.T = (blocks & (kUT | kWT)) ? T : nullptr;
-  a.U = U;
-  a.W = (blocks & (kWT | kWF)) ? W : nullptr;
   a.items = wide_.listed ? wide_.items.as<WideItem>() : nullptr;
   a.sys = wide_.listed ? wide_.sys.as<SymSys>() : nullptr;
   a.nunits = wide_.nunits;
@@ -853,6 +848,16 @@ void NBodySolver::launch_wide(int blocks, bool fp32, const void* rec, const doub
   a.t0 = t0_;
   a.rt0 = rt0_;
   a.r0 = r0_;
+  return a;
+}
+
+void NBodySolver::launch_wide(int blocks, bool fp32, const void* rec, const double* F,
+                              const double* T, double* U, double* W) {
+  WideArgs a = wide_args(blocks, fp32, rec);
+  a.F = F;
+  a.T = (blocks & (kUT | kWT)) ? T : nullptr;
+  a.U = U;
+  a.W = (blocks & (kWT | kWF)) ? W : nullptr;
   launch_pair_wide(a, stream_);
 }
 
@@ -1212,7 +1217,18 @@ int NBodySolver::lanczos_run(const double* z, double** result) {
   scalars_.reserve(sizeof(LanczosScalars));
   tsq_work_.reserve(sizeof(double) * kCheckBatch * tsqrt_scratch(iter_limit_));
   coef_.reserve(sizeof(double) * kCheckBatch * kLanczosMaxIterations);
-  w_.reserve(sizeof(double) * n);
+  const bool wide_step = fused && !reorth_ && wide_step_route();
+  w_.reserve(sizeof(double) * n * (wide_step ? 2 : 1));
+  if (wide_step) {
+    ensure_wide_plan();
+    wide_a_.reserve(sizeof(double) * wide_.nunits);
+    wide_b_.reserve(sizeof(double) * 64);
+    if (wide_e1_n_ < n) {
+      wide_e1_.reserve(sizeof(double) * n);
+      launch_unit_vector(wide_e1_.as<double>(), n, stream_);
+      wide_e1_n_ = n;
+    }
+  }
   lz_status_.reserve(kLzSlots * sizeof(LanczosStatus), hipHostMallocMapped | hipHostMallocCoherent);
   for (auto& e : lz_ev_)
     if (!e) LM_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
@@ -1354,7 +1370,18 @@ int NBodySolver::lanczos_run(const double* z, double** result) {
     double* vn = V + (int64_t)(i + 1) * n;
     const bool checked = (i >= check || cb_ != nullptr) &&
                          (i - (bfirst < 0 ? i : bfirst) + 1 >= batch || i == iter_limit_ - 1);
-    if (fused) {
+    if (wide_step) {
+      const bool fp32 = pair_prec_ == kPairFP32;
+      const WideArgs a = wide_args(angular_ ? kUF | kUT | kWT | kWF : kUF, fp32,
+                                   fp32 ? rec32_.as<void>() : rec64_.as<void>());
+      double* wi = w + (int64_t)(i % 2) * n;
+      launch_wide_step(a, WideStep{w + (int64_t)((i + 1) % 2) * n, wide_e1_.as<double>(),
+                                   V + (int64_t)i * n, vp, wi, wide_a_.as<double>(),
+                                   wide_b_.as<double>(), sc, (int)n, i},
+                       stream_);
+      launch_wide_orthogonalise(wi, vi, (int)n, i, wide_a_.as<double>(), a.nunits,
+                                wide_b_.as<double>(), sc, pair_stop_, stream_);
+    } else if (fused) {
       if (head_step >= 0) {
         const int h = head_step;
         pair_head_ = LanczosHead{w, V + (int64_t)h * n, h > 0 ? V + (int64_t)(h - 1) * n : nullptr,
@@ -1449,6 +1476,19 @@ int NBodySolver::lanczos_run(const double* z, double** result) {
     if (settle_oldest()) return finish();
   drain();
   throw Error("[Lanczos] Could not converge");
+}
+
+// Whether a plain recurrence can run on launch_wide_step: bottom-wall systems
+// whose products the wide kernel takes (open ones keep their order of operations).
+bool NBodySolver::wide_step_route() {
+  static_assert(kWideStepMax == kLanczosFusedMaxN, "the vectors of the fused steps");
+  if (pre_on() || kind_code() != 1 || pair_active_ != nullptr) return false;
+  const bool fp32 = pair_prec_ == kPairFP32;
+  if (use_sym(angular_ ? kUF | kUT | kWT | kWF : kUF, fp32) || !use_wide()) return false;
+  last_sym_ = false;
+  last_wide_ = true;
+  deferred_nch_ = 0;
+  return true;
 }
 
 // Whether the products of a plain recurrence can finish the step before them:

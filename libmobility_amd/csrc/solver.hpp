@@ -325,6 +325,10 @@ class NBodySolver {
   // Lanczos step that the next product finishes first (n = 0: none)
   LanczosHead pair_head_{};
   bool head_route() const;
+  DevBuf wide_a_, wide_b_, wide_e1_;  // partial sums and e1 of launch_wide_step
+  int64_t wide_e1_n_ = 0;
+  bool wide_step_route();
+  WideArgs wide_args(int blocks, bool fp32, const void* rec);
   int tile_tpl_ = 0, tile_nch_ = 0;  // user override (0 = auto)
   bool autotune_ = false;
   std::map<std::tuple<int64_t, int, int, int, int>, std::pair<int, int>> tuned_;

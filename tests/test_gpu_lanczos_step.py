@@ -42,3 +42,25 @@ def test_step_lengths_vs_oracle(angular, N):
         # iteration apart, and then the two differ by about the tolerance
         assert abs(s.lastLanczosIterations() - it) <= 1
         assert np.linalg.norm(got - ref) <= 2 * TOL * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("sizes", [(2,) * 2730, (40,) * 30, (300, 0, 17, 1, 1000)])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_one_recurrence_over_systems_vs_oracle(sizes, precision):
+    """A recurrence over bottom-wall systems: one wave and four per unit of the
+    product (many tiny systems and few), equal systems and a list."""
+    rng = np.random.default_rng(len(sizes))
+    eta, a, N = 1 / (6 * np.pi), 1.0, sum(sizes)
+    pos = np.concatenate([rng.uniform(0, 6.0 * max(1.0, (n / 2) ** 0.5), (n, 3)) for n in sizes])
+    pos[:, 2] = rng.uniform(1.5, 12.0, N)
+    s = _solver(True, a, eta, precision=precision)
+    s.initialize(viscosity=eta, hydrodynamicRadius=a, tolerance=TOL)
+    s.setSystems(sizes)
+    s.setPositions(pos)
+    lz = oracle.LanczosOracle()
+    W = rng.normal(size=3 * N)
+    u, _ = s.sqrtMdotW_with_noise(W)
+    ref, it = lz.run(lambda v: oracle.mdot(pos, eta, a, F=v, wall=True, sys_sizes=sizes)[0], W, TOL)
+    assert abs(s.lastLanczosIterations() - it) <= 1
+    # FP32 pair terms (6e-8 each) add to the tolerance
+    assert np.linalg.norm(u.ravel() - ref) <= (2 * TOL if precision == "fp64" else 4 * TOL) * np.linalg.norm(ref)
