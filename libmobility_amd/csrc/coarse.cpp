@@ -6,9 +6,28 @@
 #include <chrono>
 #include <cmath>
 
+#include "cell_sort.hpp"
 #include "kernels.hpp"
 
 namespace lm {
+
+// First cell edge for about ppc particles per cell, and the cells per axis (the
+// total is returned) of an edge; too many cells: the next edge is kCoarser times
+// longer.
+static constexpr double kCoarser = 1.03;
+static double coarse_side(const double ext[3], int64_t N, int ppc) {
+  double vol = 1.0;
+  for (int k = 0; k < 3; ++k) vol *= std::max(ext[k], 1.0);
+  return std::cbrt(vol / std::max(1.0, (double)N / (double)std::max(ppc, 1)));
+}
+static int64_t coarse_shape(const double ext[3], double side, int g[3]) {
+  int64_t total = 1;
+  for (int k = 0; k < 3; ++k) {
+    g[k] = (int)std::max<long long>(1, std::llround(std::max(ext[k], 1.0) / side));
+    total *= g[k];
+  }
+  return total;
+}
 
 void coarse_cells(const double* xyz, int64_t stride, int64_t N, int ppc, CoarseCells& out,
                   int64_t max_dim) {
@@ -21,20 +40,11 @@ void coarse_cells(const double* xyz, int64_t stride, int64_t N, int ppc, CoarseC
       lo[k] = std::min(lo[k], x);
       hi[k] = std::max(hi[k], x);
     }
-  double vol = 1.0;
-  for (int k = 0; k < 3; ++k) {
-    ext[k] = hi[k] - lo[k];
-    vol *= std::max(ext[k], 1.0);
-  }
-  const double want = std::max(1.0, (double)N / (double)std::max(ppc, 1));
-  double side = std::cbrt(vol / want);
+  for (int k = 0; k < 3; ++k) ext[k] = hi[k] - lo[k];
+  double side = coarse_side(ext, N, ppc);
   std::vector<int64_t> count;
   for (;;) {
-    int64_t total = 1;
-    for (int k = 0; k < 3; ++k) {
-      out.g[k] = (int)std::max<long long>(1, std::llround(std::max(ext[k], 1.0) / side));
-      total *= out.g[k];
-    }
+    const int64_t total = coarse_shape(ext, side, out.g);
     out.cell_of.assign(N, 0);
     for (int64_t i = 0; i < N; ++i) {
       int q[3];
@@ -52,7 +62,7 @@ void coarse_cells(const double* xyz, int64_t stride, int64_t N, int ppc, CoarseC
     int C = 0;
     for (int64_t c = 0; c < total; ++c) C += count[c] > 0;
     if (3 * (int64_t)C <= max_dim) break;
-    side *= 1.03;  // too many cells: coarser grid
+    side *= kCoarser;
   }
   // compact the non-empty cells in raw order, then a stable counting sort
   std::vector<int> compact(count.size(), -1);
@@ -86,59 +96,124 @@ void SideStream::ensure() {
   LM_HIP(hipEventCreateWithFlags(&done, hipEventDisableTiming));
 }
 
-void CoarseLevel::build(const void* rec64, const void* rec32, const std::vector<int64_t>& off,
-                        const std::vector<int>& wall, int ppc_req, int64_t max_dim,
-                        bool force_fp64, hipStream_t s) {
+// The cells of one system on the device (coarse_cells' rule): perm_, start_,
+// cell_of_ and scale_.  False where a cell holds so many particles that ranking
+// them against each other would cost more than the host's sort.
+bool CoarseLevel::device_cells(const double4* rec, int64_t N, const double* box, int ppc,
+                               int64_t max_dim, hipStream_t s) {
+  CellGrid grid{};
+  for (int k = 0; k < 3; ++k) {
+    grid.lo[k] = box[k];
+    grid.ext[k] = box[3 + k] - box[k];
+  }
+  scan_host_.reserve(2 * sizeof(int), hipHostMallocMapped | hipHostMallocCoherent);
+  raw_.reserve(sizeof(int) * N);
+  double side = coarse_side(grid.ext, N, ppc);
+  for (;;) {
+    const int64_t total = coarse_shape(grid.ext, side, grid.g);
+    if (total > INT32_MAX) return false;
+    count_.reserve(sizeof(int) * total);
+    compact_.reserve(sizeof(int) * total);
+    start_.reserve(sizeof(int) * (std::min<int64_t>(total, N) + 1));
+    launch_cell_count(rec, N, grid, raw_.as<int>(), count_.as<int>(), (int)total, s);
+    launch_cell_scan(CellScan{count_.as<int>(), (int)total, nullptr, compact_.as<int>(),
+                              start_.as<int>(), scan_host_.device_as<int>()}, s);
+    LM_HIP(hipStreamSynchronize(s));
+    if (3 * (int64_t)scan_host_.as<int>()[0] <= max_dim) break;
+    side *= kCoarser;
+  }
+  if (scan_host_.as<int>()[1] > kCellRankMax) return false;
+  const int C = scan_host_.as<int>()[0];
+  list_.reserve(sizeof(int) * N);
+  perm_.reserve(sizeof(int) * N);
+  cell_of_.reserve(sizeof(int) * N);
+  scale_.reserve(sizeof(double) * C);
+  launch_cell_fill32(raw_.as<int>(), N, compact_.as<int>(), start_.as<int>(), count_.as<int>(),
+                     list_.as<int>(), s);
+  launch_cell_order(raw_.as<int>(), N, compact_.as<int>(), start_.as<int>(), C, list_.as<int>(),
+                    perm_.as<int>(), cell_of_.as<int>(), scale_.as<double>(), s);
+  cells_.C = C;
+  for (int k = 0; k < 3; ++k) cells_.g[k] = grid.g[k];
+  return true;
+}
+
+const CoarseCells& CoarseLevel::host_cells(hipStream_t s) const {
+  if (!host_cell_of_) {
+    cells_.cell_of.resize(N_);
+    LM_HIP(hipMemcpyAsync(cells_.cell_of.data(), cell_of_.as<int>(), sizeof(int) * N_,
+                          hipMemcpyDeviceToHost, s));
+    LM_HIP(hipStreamSynchronize(s));
+    host_cell_of_ = true;
+  }
+  return cells_;
+}
+
+void CoarseLevel::build(const void* rec64, const void* rec32, const double* box,
+                        const std::vector<int64_t>& off, const std::vector<int>& wall, int ppc_req,
+                        int64_t max_dim, bool force_fp64, hipStream_t s) {
   const auto t_start = std::chrono::steady_clock::now();
   const int nsys = (int)off.size() - 1;
   const int64_t N = off[nsys];
   if (nsys < 1 || N <= 0) throw Error("[libmobility_amd] coarse level: no particles");
   if (N > INT32_MAX) throw Error("[libmobility_amd] coarse level: too many particles");
-  std::vector<double> h((size_t)4 * N);
-  LM_HIP(hipMemcpyAsync(h.data(), rec64, sizeof(double) * 4 * N, hipMemcpyDeviceToHost, s));
-  LM_HIP(hipStreamSynchronize(s));
-  // cells of every system, concatenated; a system's particles (and so its
-  // sorted list) occupy [off[s], off[s+1])
-  cells_.cell_of.assign(N, 0);
-  cells_.perm.assign(N, 0);
-  cells_.start.clear();
-  sys_.assign(nsys, CoarseSys{0, 0, 0, 0, 0, 0});
+  cells_.C = 0;  // nothing is built until the end of this
+  N_ = N;
+  const bool on_device = nsys == 1 && box != nullptr &&
+                         device_cells(static_cast<const double4*>(rec64), N, box, ppc_req, max_dim, s);
   int C = 0;
   int64_t moff = 0, doff = 0;
-  bool have_grid = false;
-  for (int q = 0; q < nsys; ++q) {
-    const int64_t n_q = off[q + 1] - off[q];
-    CoarseSys& S = sys_[q];
-    S.moff = moff;
-    S.doff = doff;
-    S.c0 = C;
-    S.wall = wall[q];
-    if (n_q == 0) continue;
-    CoarseCells cq;
-    coarse_cells(h.data() + 4 * off[q], 4, n_q, ppc_req, cq, max_dim);
-    for (int64_t i = 0; i < n_q; ++i) {
-      cells_.cell_of[off[q] + i] = C + cq.cell_of[i];
-      cells_.perm[off[q] + i] = (int)(off[q] + cq.perm[i]);
-    }
-    for (int c = 0; c < cq.C; ++c) cells_.start.push_back((int)(off[q] + cq.start[c]));
-    if (!have_grid) {
-      for (int k = 0; k < 3; ++k) cells_.g[k] = cq.g[k];
-      have_grid = true;
-    }
-    S.C = cq.C;
-    S.n = (3 * cq.C + kCoarseTile - 1) / kCoarseTile * kCoarseTile;
+  sys_.assign(nsys, CoarseSys{0, 0, 0, 0, 0, 0});
+  auto add_block = [&](CoarseSys& S, int c) {
+    S.C = c;
+    S.n = (3 * c + kCoarseTile - 1) / kCoarseTile * kCoarseTile;
     moff += (int64_t)S.n * S.n;
     doff += (int64_t)(S.n / kCoarseTile) * kCoarseTile * kCoarseTile;
-    C += cq.C;
+    C += c;
+  };
+  std::vector<double> scale;
+  if (on_device) {
+    sys_[0].wall = wall[0];
+    add_block(sys_[0], cells_.C);
+    host_cell_of_ = false;
+  } else {
+    std::vector<double> h((size_t)4 * N);
+    LM_HIP(hipMemcpyAsync(h.data(), rec64, sizeof(double) * 4 * N, hipMemcpyDeviceToHost, s));
+    LM_HIP(hipStreamSynchronize(s));
+    // cells of every system, concatenated; a system's particles (and so its
+    // sorted list) occupy [off[s], off[s+1])
+    cells_.cell_of.assign(N, 0);
+    cells_.perm.assign(N, 0);
+    cells_.start.clear();
+    host_cell_of_ = true;
+    bool have_grid = false;
+    for (int q = 0; q < nsys; ++q) {
+      const int64_t n_q = off[q + 1] - off[q];
+      CoarseSys& S = sys_[q];
+      S.moff = moff;
+      S.doff = doff;
+      S.c0 = C;
+      S.wall = wall[q];
+      if (n_q == 0) continue;
+      CoarseCells cq;
+      coarse_cells(h.data() + 4 * off[q], 4, n_q, ppc_req, cq, max_dim);
+      for (int64_t i = 0; i < n_q; ++i) {
+        cells_.cell_of[off[q] + i] = C + cq.cell_of[i];
+        cells_.perm[off[q] + i] = (int)(off[q] + cq.perm[i]);
+      }
+      for (int c = 0; c < cq.C; ++c) cells_.start.push_back((int)(off[q] + cq.start[c]));
+      if (!have_grid) {
+        for (int k = 0; k < 3; ++k) cells_.g[k] = cq.g[k];
+        have_grid = true;
+      }
+      add_block(S, cq.C);
+    }
+    cells_.start.push_back((int)N);
+    scale.resize(C);
+    for (int c = 0; c < C; ++c)
+      scale[c] = 1.0 / std::sqrt((double)(cells_.start[c + 1] - cells_.start[c]));
   }
-  cells_.start.push_back((int)N);
-  cells_.C = C;
   max_row_ = 0;
   for (const CoarseSys& S : sys_) max_row_ = std::max(max_row_, 3 * S.C);
-  N_ = N;
-  std::vector<double> scale(C);
-  for (int c = 0; c < C; ++c)
-    scale[c] = 1.0 / std::sqrt((double)(cells_.start[c + 1] - cells_.start[c]));
   std::vector<int> row_sys(3 * (size_t)C);
   std::vector<int64_t> pair_off(nsys + 1, 0);
   std::vector<int> small, large;
@@ -157,10 +232,12 @@ void CoarseLevel::build(const void* rec64, const void* rec32, const std::vector<
     b.reserve(bytes);
     if (bytes) LM_HIP(hipMemcpyAsync(b.as<void>(), src, bytes, hipMemcpyHostToDevice, s));
   };
-  upload(perm_, cells_.perm.data(), sizeof(int) * N);
-  upload(cell_of_, cells_.cell_of.data(), sizeof(int) * N);
-  upload(start_, cells_.start.data(), sizeof(int) * (C + 1));
-  upload(scale_, scale.data(), sizeof(double) * C);
+  if (!on_device) {
+    upload(perm_, cells_.perm.data(), sizeof(int) * N);
+    upload(cell_of_, cells_.cell_of.data(), sizeof(int) * N);
+    upload(start_, cells_.start.data(), sizeof(int) * (C + 1));
+    upload(scale_, scale.data(), sizeof(double) * C);
+  }
   upload(sys_dev_, sys_.data(), sizeof(CoarseSys) * nsys);
   upload(row_sys_, row_sys.data(), sizeof(int) * row_sys.size());
   upload(pair_off_, pair_off.data(), sizeof(int64_t) * (nsys + 1));
@@ -199,6 +276,7 @@ void CoarseLevel::build(const void* rec64, const void* rec32, const std::vector<
     if (info == 0) break;
   }
   if (info != 0) throw Error("[libmobility_amd] coarse level: the coarse matrix is not positive definite");
+  cells_.C = C;
   build_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t_start)
                  .count();
 }

@@ -115,11 +115,14 @@ class CoarseLevel {
 
   // rec64 / rec32: the solver's position records; off[0..nsys] the systems'
   // particle offsets, wall[s] 1 for a single-wall system.  Every system gets
-  // its own cells and coarse block.
+  // its own cells and coarse block.  box: corners lo, hi of the records of a
+  // single system, whose cells are then found on the device (nullptr: all cells
+  // on the host).
   // fp64: the coarse matrix from FP64 pair terms (otherwise FP32, and FP64
   // only when the FP32 one turns out indefinite)
-  void build(const void* rec64, const void* rec32, const std::vector<int64_t>& off,
-             const std::vector<int>& wall, int ppc, int64_t max_dim, bool fp64, hipStream_t s);
+  void build(const void* rec64, const void* rec32, const double* box,
+             const std::vector<int64_t>& off, const std::vector<int>& wall, int ppc,
+             int64_t max_dim, bool fp64, hipStream_t s);
   // out = Gc in (kG), Gc^T in (kGt) or Gc^{-1} in (kGinv); vectors of length
   // n >= 3N whose entries past 3N pass through; the particles' blocks `before`
   // or `after` it in the same launches.  in may equal out.
@@ -129,9 +132,9 @@ class CoarseLevel {
   int cells() const { return cells_.C; }
   int dim() const { return 3 * cells_.C; }
   int systems() const { return (int)sys_.size(); }
-  // global cells (cell_of, perm, start over all systems; g of the first
-  // system with particles)
-  const CoarseCells& host_cells() const { return cells_; }
+  // global cells (cell_of over all systems; g of the first system with
+  // particles)
+  const CoarseCells& host_cells(hipStream_t s) const;
   // L and X = L^{-1} of system s's block (3C_s x 3C_s row-major, host)
   void factors(int s, double* L, double* X, hipStream_t st) const;
   int system_cells(int s) const { return sys_.at(s).C; }
@@ -150,7 +153,12 @@ class CoarseLevel {
 
  private:
   bool fp64_pairs_ = false;
-  CoarseCells cells_;
+  mutable CoarseCells cells_;
+  mutable bool host_cell_of_ = true;  // cells_.cell_of holds the last build's
+  bool device_cells(const double4* rec, int64_t N, const double* box, int ppc, int64_t max_dim,
+                    hipStream_t s);
+  HostBuf scan_host_;
+  DevBuf raw_, count_, compact_, list_;
   std::vector<CoarseSys> sys_;
   int64_t N_ = 0;
   int max_row_ = 0;  // largest 3 C_s

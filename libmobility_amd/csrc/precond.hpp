@@ -46,6 +46,8 @@ struct KnnSys {
   int g[3];
   int64_t cell0;
 };
+// Grid of a system of n particles in the box [lo, hi]; the number of its cells.
+int64_t knn_shape(const double lo[3], const double hi[3], int64_t n, KnnSys& S);
 // Host side: grids of all systems (about 8 particles per cell), each
 // particle's local cell id, the particles sorted by (system, cell, index)
 // and the cells' first positions in that order (total cells + 1 entries).

@@ -154,6 +154,23 @@ void launch_knn_cells(const double4* rec, const int64_t* sys_off, int nsys, cons
   LM_HIP(hipGetLastError());
 }
 
+int64_t knn_shape(const double lo[3], const double hi[3], int64_t n, KnnSys& S) {
+  double ext[3], vol = 1.0;
+  for (int k = 0; k < 3; ++k) {
+    ext[k] = hi[k] - lo[k];
+    vol *= std::max(ext[k], 1.0);
+  }
+  const double side = std::cbrt(vol / std::max(1.0, (double)n / 8.0));
+  int64_t ncell = 1;
+  for (int k = 0; k < 3; ++k) {
+    S.g[k] = (int)std::max<long long>(1, std::min<long long>(1024, std::llround(std::max(ext[k], 1.0) / side)));
+    S.lo[k] = lo[k];
+    S.edge[k] = ext[k] > 0.0 ? ext[k] / S.g[k] : 1.0;
+    ncell *= S.g[k];
+  }
+  return ncell;
+}
+
 void knn_grid(const double* xyz4, const int64_t* sys_off, int nsys, std::vector<KnnSys>& sys,
               std::vector<int>& cell_of, std::vector<int>& perm, std::vector<int64_t>& start) {
   const int64_t N = sys_off[nsys];
@@ -166,7 +183,7 @@ void knn_grid(const double* xyz4, const int64_t* sys_off, int nsys, std::vector<
     const int64_t a = sys_off[q], b = sys_off[q + 1], n = b - a;
     KnnSys& S = sys[q];
     S.cell0 = cells;
-    double lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0}, ext[3];
+    double lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};
     if (n > 0)
       for (int k = 0; k < 3; ++k) lo[k] = hi[k] = xyz4[4 * a + k];
     for (int64_t i = a; i < b; ++i)
@@ -174,25 +191,13 @@ void knn_grid(const double* xyz4, const int64_t* sys_off, int nsys, std::vector<
         lo[k] = std::min(lo[k], xyz4[4 * i + k]);
         hi[k] = std::max(hi[k], xyz4[4 * i + k]);
       }
-    double vol = 1.0;
-    for (int k = 0; k < 3; ++k) {
-      ext[k] = hi[k] - lo[k];
-      vol *= std::max(ext[k], 1.0);
-    }
-    const double side = std::cbrt(vol / std::max(1.0, (double)n / 8.0));
-    int64_t ncell = 1;
-    for (int k = 0; k < 3; ++k) {
-      S.g[k] = (int)std::max<long long>(1, std::min<long long>(1024, std::llround(std::max(ext[k], 1.0) / side)));
-      S.lo[k] = lo[k];
-      S.edge[k] = ext[k] > 0.0 ? ext[k] / S.g[k] : 1.0;
-      ncell *= S.g[k];
-    }
+    const int64_t ncell = knn_shape(lo, hi, n, S);
     std::vector<int64_t> count(ncell + 1, 0);
     for (int64_t i = a; i < b; ++i) {
       int qq[3];
       for (int k = 0; k < 3; ++k) {
         qq[k] = 0;
-        if (ext[k] > 0.0) {
+        if (hi[k] - lo[k] > 0.0) {
           const double f = std::floor((xyz4[4 * i + k] - lo[k]) / S.edge[k]);
           qq[k] = (int)std::min<double>(S.g[k] - 1, std::max(0.0, f));
         }

@@ -18,6 +18,8 @@
 #include <cstring>
 #include <string>
 
+#include "cell_sort.hpp"
+
 namespace lm {
 
 
@@ -1982,6 +1984,20 @@ void NBodySolver::lastLanczosIterationsMulti(int* out, int nrhs) const {
 
 // ---- learned preconditioner ------------------------------------------------------
 
+// Corners lo, hi of the box of the current records (one system's).
+const double* NBodySolver::record_box() {
+  box_host_.reserve(sizeof(double) * 6 * kBoxBlocks, hipHostMallocMapped | hipHostMallocCoherent);
+  launch_record_box(rec64_.as<double4>(), N_, box_host_.device_as<double>(), stream_);
+  LM_HIP(hipStreamSynchronize(stream_));
+  const double* b = box_host_.as<double>();
+  for (int c = 0; c < 6; ++c) {
+    box_[c] = b[c];
+    for (int k = 1; k < kBoxBlocks; ++k)
+      box_[c] = c < 3 ? std::min(box_[c], b[6 * k + c]) : std::max(box_[c], b[6 * k + c]);
+  }
+  return box_;
+}
+
 void NBodySolver::ensure_knn() {
   require_positions("[Mobility] Positions have 0 particles. Did you call setPositions?");
   ensure_records();
@@ -1989,21 +2005,46 @@ void NBodySolver::ensure_knn() {
   pc_feat_.reserve(sizeof(float) * N_ * kPrecondIn);
   pc_nbr_.reserve(sizeof(int) * N_ * kPrecondK);
   const int nsys = (int)sys_off_host_.size() - 1;
-  // cell grid on the host (deterministic), neighbour search on the device
-  knn_xyz_.resize((size_t)4 * N_);
-  LM_HIP(hipMemcpyAsync(knn_xyz_.data(), rec64_.as<void>(), sizeof(double) * 4 * N_,
-                        hipMemcpyDeviceToHost, stream_));
-  LM_HIP(hipStreamSynchronize(stream_));
-  knn_grid(knn_xyz_.data(), sys_off_host_.data(), nsys, knn_sys_host_, knn_cell_host_,
-           knn_perm_host_, knn_start_host_);
   auto upload = [&](DevBuf& b, const void* src, size_t bytes) {
     b.reserve(bytes);
     LM_HIP(hipMemcpyAsync(b.as<void>(), src, bytes, hipMemcpyHostToDevice, stream_));
   };
-  upload(knn_sys_, knn_sys_host_.data(), sizeof(KnnSys) * knn_sys_host_.size());
-  upload(knn_cell_, knn_cell_host_.data(), sizeof(int) * N_);
-  upload(knn_perm_, knn_perm_host_.data(), sizeof(int) * N_);
-  upload(knn_start_, knn_start_host_.data(), sizeof(int64_t) * knn_start_host_.size());
+  if (nsys == 1) {
+    knn_sys_host_.assign(1, KnnSys{});
+    CellGrid grid{};
+    const double* box = record_box();
+    const int64_t ncell = knn_shape(box, box + 3, N_, knn_sys_host_[0]);
+    for (int k = 0; k < 3; ++k) {
+      grid.lo[k] = box[k];
+      grid.ext[k] = box[3 + k] - box[k];
+      grid.edge[k] = knn_sys_host_[0].edge[k];
+      grid.g[k] = knn_sys_host_[0].g[k];
+    }
+    grid.by_edge = 1;
+    knn_cell_.reserve(sizeof(int) * N_);
+    knn_perm_.reserve(sizeof(int) * N_);
+    knn_count_.reserve(sizeof(int) * ncell);
+    knn_start_.reserve(sizeof(int64_t) * (ncell + 1));
+    upload(knn_sys_, knn_sys_host_.data(), sizeof(KnnSys));
+    launch_cell_count(rec64_.as<double4>(), N_, grid, knn_cell_.as<int>(), knn_count_.as<int>(),
+                      (int)ncell, stream_);
+    launch_cell_scan(CellScan{knn_count_.as<int>(), (int)ncell, knn_start_.as<int64_t>(), nullptr,
+                              nullptr, nullptr}, stream_);
+    launch_cell_fill64(knn_cell_.as<int>(), N_, knn_start_.as<int64_t>(), knn_count_.as<int>(),
+                       knn_perm_.as<int>(), stream_);
+  } else {
+    // small systems: grids on the host, neighbour search on the device
+    knn_xyz_.resize((size_t)4 * N_);
+    LM_HIP(hipMemcpyAsync(knn_xyz_.data(), rec64_.as<void>(), sizeof(double) * 4 * N_,
+                          hipMemcpyDeviceToHost, stream_));
+    LM_HIP(hipStreamSynchronize(stream_));
+    knn_grid(knn_xyz_.data(), sys_off_host_.data(), nsys, knn_sys_host_, knn_cell_host_,
+             knn_perm_host_, knn_start_host_);
+    upload(knn_sys_, knn_sys_host_.data(), sizeof(KnnSys) * knn_sys_host_.size());
+    upload(knn_cell_, knn_cell_host_.data(), sizeof(int) * N_);
+    upload(knn_perm_, knn_perm_host_.data(), sizeof(int) * N_);
+    upload(knn_start_, knn_start_host_.data(), sizeof(int64_t) * knn_start_host_.size());
+  }
   launch_knn_cells(rec64_.as<double4>(), sys_off_.as<int64_t>(), nsys, knn_sys_.as<KnnSys>(),
                    knn_cell_.as<int>(), knn_perm_.as<int>(), knn_start_.as<int64_t>(), N_,
                    kinds_dev(), wall_ ? 1 : 0, pc_feat_.as<float>(), pc_nbr_.as<int>(), stream_);
@@ -2077,8 +2118,9 @@ void NBodySolver::ensure_coarse() {
   std::vector<int> wall(nsys);
   for (int q = 0; q < nsys; ++q)
     wall[q] = q < (int)sys_kind_host_.size() ? (sys_kind_host_[q] != 0) : (wall_ ? 1 : 0);
-  coarse_.build(rec64_.as<void>(), rec32_.as<void>(), sys_off_host_, wall, coarse_ppc_,
-                coarse_max_dim_, coarse_fp64_, stream_);
+  coarse_.layout = 0;  // the buffers change from here on
+  coarse_.build(rec64_.as<void>(), rec32_.as<void>(), nsys == 1 ? record_box() : nullptr,
+                sys_off_host_, wall, coarse_ppc_, coarse_max_dim_, coarse_fp64_, stream_);
   coarse_.layout = layout_id_;
   coarse_.structure = struct_id_;
   coarse_.a = a_;
@@ -2124,7 +2166,7 @@ void NBodySolver::pre_inverse(const double* y, double* out, int64_t n) {
 }
 
 int NBodySolver::coarseCells(int* cell_of, int* grid) const {
-  const CoarseCells& c = coarse_.host_cells();
+  const CoarseCells& c = coarse_.host_cells(stream_);
   if (c.C == 0) throw Error("[libmobility_amd] no coarse level has been built");
   if (cell_of) std::copy(c.cell_of.begin(), c.cell_of.end(), cell_of);
   if (grid)

@@ -484,7 +484,10 @@ class NBodySolver {
   std::vector<KnnSys> knn_sys_host_;
   std::vector<int> knn_cell_host_, knn_perm_host_;
   std::vector<int64_t> knn_start_host_;
-  DevBuf knn_sys_, knn_cell_, knn_perm_, knn_start_;
+  DevBuf knn_sys_, knn_cell_, knn_perm_, knn_start_, knn_count_;
+  HostBuf box_host_;
+  double box_[6];
+  const double* record_box();
   uint64_t knn_layout_ = 0, pc_layout_ = 0, pc_struct_ = 0, pc_version_ = 0;
   double pc_a_ = 0.0;
   int pc_refresh_ = 1;
