@@ -658,18 +658,19 @@ __global__ __launch_bounds__(kPairThreads) void k_pair_sym(SymArgs a) {
 
 // Products of plain Lanczos over small open systems: the launch first finishes
 // the step before (lanczos_head.hpp), in every workgroup, and reads the forces
-// from LDS.  1024 particles, FP64, a step and a product: 17.8 us in two launches
-// (this and the chunk sums), 20.4 as product and one-workgroup step.
-template <class R, int BLK>
+// from LDS.  1024 particles, translational, FP64, a step and a product: 17.8 us
+// in two launches (this and the chunk sums), 20.4 as product and one-workgroup
+// step.  All four blocks:
+template <class R>
 __global__ __launch_bounds__(kPairThreads) void k_pair_head(
     const PairItem* __restrict__ items, const typename Rec<R>::T* __restrict__ pos,
     double* __restrict__ U, double* __restrict__ W, int64_t slab, const int* stop, double t0,
     double rt0, double r0, LanczosHead h) {
   using R4 = typename Rec<R>::T;
-  constexpr bool kNeedT = (BLK & (kUT | kWT)) != 0;
+  constexpr int BLK = kUF | kUT | kWT | kWF;
   __shared__ R4 s_pos[kPairThreads];
   __shared__ R4 s_f[kPairThreads];
-  __shared__ R4 s_t[kNeedT ? kPairThreads : 1];
+  __shared__ R4 s_t[kPairThreads];
   __shared__ double s_v[kLanczosHeadMax];
   __shared__ double sh[2][16];
   __shared__ int s_stop;
@@ -679,6 +680,98 @@ __global__ __launch_bounds__(kPairThreads) void k_pair_head(
   lanczos_head(h, s_v, sh, blockIdx.x == 0);
   if (s_stop != 0) return;  // read after the barriers of the head
   pair_item<R, false, BLK, 1>(it, pos, s_v, s_v + slab, U, W, slab, t0, rt0, r0, s_pos, s_f, s_t);
+}
+
+// The same for the translational block alone, where one item's 256 targets x 64
+// sources leave a wave 64 pairs in series on a quarter of the chip's CUs: a
+// workgroup takes 64 targets, its waves the coefficients of 16 sources each, and
+// three of them then add one component each, source by source in k_pair's order
+// (the same bits).  1024 particles, FP64: 13.8 -> 10.8 us.
+template <class R>
+__global__ __launch_bounds__(kPairThreads) void k_pair_head_uf(
+    const PairItem* __restrict__ items, const typename Rec<R>::T* __restrict__ pos,
+    double* __restrict__ U, int64_t slab, const int* stop, double t0, LanczosHead h) {
+  using R4 = typename Rec<R>::T;
+  __shared__ R s_p[3][64], s_f[3][64];
+  __shared__ R s_fuf[64][64], s_s[64][64];  // per source and target
+  __shared__ double s_v[kLanczosHeadMax];
+  __shared__ double sh[2][16];
+  __shared__ int s_stop;
+  if (threadIdx.x == 0) s_stop = stop != nullptr ? *(volatile const int*)stop : 0;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const PairItem it = items[blockIdx.x >> 2];
+  const int loc = 64 * (int)(blockIdx.x & 3) + lane;
+  const R4 pi = loc < it.ntgt ? pos[it.tgt0 + loc] : far_record<R4>();
+  // sources of the first 64, in flight while the step ends
+  R4 pj = it.src0 + lane < it.src1 ? pos[it.src0 + lane] : far_record<R4>();
+  lanczos_head(h, s_v, sh, blockIdx.x == 0);
+  if (s_stop != 0 || 64 * (int)(blockIdx.x & 3) >= it.ntgt) return;  // the whole workgroup
+  const R xi = wave == 0 ? pi.x : (wave == 1 ? pi.y : pi.z);
+  R acc = R(0);
+  double acc64 = 0.0;
+  for (int64_t base = it.src0; base < it.src1; base += 64) {
+    const int64_t j = base + lane;
+    const int cnt = (int)min((int64_t)64, it.src1 - base);
+    if (base > it.src0) {
+      __syncthreads();  // the block before is done with the LDS
+      if (j < it.src1) pj = pos[j];
+    }
+    if (wave == 0) {
+      s_p[0][lane] = pj.x;
+      s_p[1][lane] = pj.y;
+      s_p[2][lane] = pj.z;
+#pragma unroll
+      for (int c = 0; c < 3; ++c) s_f[c][lane] = j < it.src1 ? R(s_v[3 * j + c]) : R(0);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int s = 16 * wave; s < 16 * wave + 16; s += 4) {
+      R dx[4], dy[4], dz[4], r2[4], ir[4];
+      RpyCoef<R> cf[4];
+      NearTestCmp<R> near;
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int q = s + g < cnt ? s + g : cnt - 1;
+        dx[g] = pi.x - s_p[0][q];
+        dy[g] = pi.y - s_p[1][q];
+        dz[g] = pi.z - s_p[2][q];
+        r2[g] = dx[g] * dx[g] + dy[g] * dy[g] + dz[g] * dz[g];
+        ir[g] = lm_rsqrt(r2[g]);
+        cf[g] = RpyCoef<R>{};
+        rpy_far_uf34<R>(ir[g], cf[g]);
+        near.add(r2[g]);
+      }
+      if (__builtin_expect(near.hit(), 0)) {
+        lm_rare_path();
+#pragma unroll
+        for (int g = 0; g < 4; ++g) rpy_near_select_uf34<R>(r2[g], ir[g], cf[g]);
+      }
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int q = s + g < cnt ? s + g : cnt - 1;
+        s_fuf[s + g][lane] = cf[g].fuf;
+        s_s[s + g][lane] =
+            cf[g].guf * (dx[g] * s_f[0][q] + dy[g] * s_f[1][q] + dz[g] * s_f[2][q]);
+      }
+    }
+    __syncthreads();
+    if (wave < 3) {
+#pragma unroll 8
+      for (int s = 0; s < cnt; ++s)
+        acc = lm_fma(s_s[s][lane], xi - s_p[wave][s], lm_fma(s_fuf[s][lane], s_f[wave][s], acc));
+      if constexpr (std::is_same<R, float>::value) {
+        // FP64 sums over tiles of kPairThreads sources, as in pair_item
+        if ((base - it.src0) % kPairThreads == kPairThreads - 64 || base + 64 >= it.src1) {
+          acc64 += acc;
+          acc = R(0);
+        }
+      }
+    }
+  }
+  if constexpr (std::is_same<R, double>::value) acc64 = acc;
+  if (wave < 3 && loc < it.ntgt)
+    U[(int64_t)it.chunk * slab + 3 * (it.tgt0 + loc) + wave] = 0.75 * t0 * acc64;
 }
 
 // ---- several force vectors per pass (translational block) ----------------------
@@ -892,11 +985,15 @@ static void launch_pair_kind(const PairArgs& a, hipStream_t s) {
   }
 }
 
-template <class R, int BLK>
+template <class R>
 static void launch_pair_head(const PairArgs& a, hipStream_t s) {
-  hipLaunchKernelGGL((k_pair_head<R, BLK>), dim3(a.nitems), dim3(kPairThreads), 0, s, a.items,
-                     static_cast<const typename Rec<R>::T*>(a.pos), a.U, a.W, a.slab, a.stop, a.t0,
-                     a.rt0, a.r0, a.head);
+  const auto* pos = static_cast<const typename Rec<R>::T*>(a.pos);
+  if (a.blocks == kUF)
+    hipLaunchKernelGGL(k_pair_head_uf<R>, dim3(4 * a.nitems), dim3(kPairThreads), 0, s, a.items,
+                       pos, a.U, a.slab, a.stop, a.t0, a.head);
+  else
+    hipLaunchKernelGGL((k_pair_head<R>), dim3(a.nitems), dim3(kPairThreads), 0, s, a.items, pos, a.U,
+                       a.W, a.slab, a.stop, a.t0, a.rt0, a.r0, a.head);
   LM_HIP(hipGetLastError());
 }
 
@@ -909,9 +1006,9 @@ void launch_pair(const PairArgs& a, hipStream_t s) {
         a.head.n != a.slab * (a.blocks == kAll ? 2 : 1))
       throw Error("[libmobility_amd] this product cannot finish a Lanczos step");
     if (a.fp32)
-      a.blocks == kUF ? launch_pair_head<float, kUF>(a, s) : launch_pair_head<float, kAll>(a, s);
+      launch_pair_head<float>(a, s);
     else
-      a.blocks == kUF ? launch_pair_head<double, kUF>(a, s) : launch_pair_head<double, kAll>(a, s);
+      launch_pair_head<double>(a, s);
     return;
   }
   if (a.fp32)
