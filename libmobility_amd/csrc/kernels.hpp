@@ -241,8 +241,9 @@ void launch_chunk_reduce(const double* part, int nchunks, int64_t n, double* out
 // setPositions: per-system bounding boxes (6 doubles each: min xyz, max xyz)
 // of the wall-shifted positions.
 // kinds[s] (0 open, 1 wall) selects per system; nullptr: all systems `wall`.
-void launch_system_bbox(const double* pos, const int64_t* sys_off, int nsys, double wall_shift,
-                        const int* kinds, int wall, double* bbox, hipStream_t s,
+// `largest`: particles of the largest system.
+void launch_system_bbox(const double* pos, const int64_t* sys_off, int nsys, int64_t largest,
+                        double wall_shift, const int* kinds, int wall, double* bbox, hipStream_t s,
                         double* host = nullptr);
 // Records for the pair kernels; `shifted` receives the wall-shifted AoS copy.
 void launch_make_records(const double* pos, int64_t N, const int64_t* sys_off, int nsys,

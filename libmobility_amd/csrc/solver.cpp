@@ -214,7 +214,7 @@ void NBodySolver::setPositions(const double* pos, int64_t n3, bool dev) {
     const double shift = wall_height_;
     if (any_wall) {
       bbox_host_.reserve(sizeof(double) * 6 * nsys, hipHostMallocMapped | hipHostMallocCoherent);
-      launch_system_bbox(src, sys_off_.as<int64_t>(), nsys, shift, kinds_d, wall_ ? 1 : 0,
+      launch_system_bbox(src, sys_off_.as<int64_t>(), nsys, largest, shift, kinds_d, wall_ ? 1 : 0,
                          bbox_.as<double>(), stream_, bbox_host_.device_as<double>());
       LM_HIP(hipStreamSynchronize(stream_));
       const double* bb = bbox_host_.as<double>();
@@ -226,8 +226,8 @@ void NBodySolver::setPositions(const double* pos, int64_t n3, bool dev) {
             "[Mobility] The center of a particle has fallen below the wall. Check your "
             "configuration and forces to ensure particle centers stay above the wall.");
     } else if (!place) {
-      launch_system_bbox(src, sys_off_.as<int64_t>(), nsys, shift, kinds_d, 0, bbox_.as<double>(),
-                         stream_);
+      launch_system_bbox(src, sys_off_.as<int64_t>(), nsys, largest, shift, kinds_d, 0,
+                         bbox_.as<double>(), stream_);
     }
     shifted_.reserve(sizeof(double) * n3);
     rec64_.reserve(sizeof(double) * 4 * N);
@@ -1105,7 +1105,7 @@ void NBodySolver::pair_product(const void* rec64, const void* rec32, const doubl
 void NBodySolver::ensure_records() {
   if (N_ <= 0 || rec_a_ == a_) return;
   const int nsys = (int)sys_off_host_.size() - 1;
-  launch_system_bbox(shifted_.as<double>(), sys_off_.as<int64_t>(), nsys, 0.0, kinds_dev(),
+  launch_system_bbox(shifted_.as<double>(), sys_off_.as<int64_t>(), nsys, N_, 0.0, kinds_dev(),
                      wall_ ? 1 : 0, bbox_.as<double>(), stream_);
   launch_make_records(shifted_.as<double>(), N_, sys_off_.as<int64_t>(), nsys, bbox_.as<double>(),
                       kinds_dev(), wall_ ? 1 : 0, 0.0, a_, nullptr, rec64_.as<void>(),
@@ -2270,7 +2270,7 @@ void NBodySolver::divM_dev(double* U, double* W, double prefactor, const double*
     launch_zero_open_systems(noise, N, sys_off_.as<int64_t>(), nsys, kinds_dev(), stream_);
   // q + (delta/2) W, then M(q + delta/2 W) W  (random_finite_differences.h:47-49)
   launch_axpy_to(rfd_pos_.as<double>(), shifted_.as<double>(), noise, 0.5 * delta, n3, stream_);
-  launch_system_bbox(rfd_pos_.as<double>(), sys_off_.as<int64_t>(), nsys, 0.0, kinds_dev(),
+  launch_system_bbox(rfd_pos_.as<double>(), sys_off_.as<int64_t>(), nsys, N_, 0.0, kinds_dev(),
                      wall_ ? 1 : 0, bbox_.as<double>(), stream_);
   launch_make_records(rfd_pos_.as<double>(), N, sys_off_.as<int64_t>(), nsys, bbox_.as<double>(),
                       kinds_dev(), wall_ ? 1 : 0, 0.0, a_, nullptr, rfd_rec64_.as<void>(),
@@ -2279,7 +2279,7 @@ void NBodySolver::divM_dev(double* U, double* W, double prefactor, const double*
                angular_ ? rfd_wp_.as<double>() : nullptr, drift_prec_);
   // q - (delta/2) W  (:50-52)
   launch_axpy_to(rfd_pos_.as<double>(), shifted_.as<double>(), noise, -0.5 * delta, n3, stream_);
-  launch_system_bbox(rfd_pos_.as<double>(), sys_off_.as<int64_t>(), nsys, 0.0, kinds_dev(),
+  launch_system_bbox(rfd_pos_.as<double>(), sys_off_.as<int64_t>(), nsys, N_, 0.0, kinds_dev(),
                      wall_ ? 1 : 0, bbox_.as<double>(), stream_);
   launch_make_records(rfd_pos_.as<double>(), N, sys_off_.as<int64_t>(), nsys, bbox_.as<double>(),
                       kinds_dev(), wall_ ? 1 : 0, 0.0, a_, nullptr, rfd_rec64_.as<void>(),
