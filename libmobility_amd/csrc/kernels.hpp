@@ -204,6 +204,7 @@ struct SymArgs {
   // finished Lanczos solve no longer needs; nullptr: never)
   const int* stop;
   double t0, rt0, r0;
+  int fine;  // launch_pair_sym: FP32 sums of at most 64 sources (0: 256)
 };
 // The open translational block in FP32, and (open blocks) the order of
 // operations that plain Lanczos products keep; 4 waves per workgroup.

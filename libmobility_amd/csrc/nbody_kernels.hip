@@ -295,6 +295,15 @@ __device__ inline void sym_item(const SymItem& it, const SymArgs& a, typename Re
     acc[t] = {R(0), R(0), R(0)};
     acc64[t] = {0.0, 0.0, 0.0};
   }
+  auto flush = [&]() {
+#pragma unroll
+    for (int t = 0; t < TPL; ++t) {
+      acc64[t].x += acc[t].x;
+      acc64[t].y += acc[t].y;
+      acc64[t].z += acc[t].z;
+      acc[t] = {R(0), R(0), R(0)};
+    }
+  };
 
   for (int o = it.o0; o < it.o1; ++o) {
     if (2 * o == S.ntiles && 2 * it.tile >= S.ntiles) continue;  // met from the other side
@@ -395,6 +404,10 @@ __device__ inline void sym_item(const SymItem& it, const SymArgs& a, typename Re
         s_red[(wave * 3 + 0) * kPairThreads + blk * 64 + lane] = lane_rol1(sa.x);
         s_red[(wave * 3 + 1) * kPairThreads + blk * 64 + lane] = lane_rol1(sa.y);
         s_red[(wave * 3 + 2) * kPairThreads + blk * 64 + lane] = lane_rol1(sa.z);
+        // With 2 or 4 targets per lane a source's FP32 sum has 128 or 256 terms;
+        // the targets' sums then go to FP64 every 64 sources instead of every
+        // 256, so that the error is no larger than with 1 per lane.
+        if (std::is_same<R, float>::value && TPL > 1 && a.fine != 0) flush();
       }
       __syncthreads();
       if (j < N) {
@@ -409,15 +422,7 @@ __device__ inline void sym_item(const SymItem& it, const SymArgs& a, typename Re
         So[3 * j + 1] = t0s * vy;
         So[3 * j + 2] = t0s * vz;
       }
-      if constexpr (std::is_same<R, float>::value) {
-#pragma unroll
-        for (int t = 0; t < TPL; ++t) {
-          acc64[t].x += acc[t].x;
-          acc64[t].y += acc[t].y;
-          acc64[t].z += acc[t].z;
-          acc[t] = {R(0), R(0), R(0)};
-        }
-      }
+      if (std::is_same<R, float>::value && (TPL == 1 || a.fine == 0)) flush();
     }
   }
   if constexpr (std::is_same<R, double>::value) {

@@ -682,6 +682,7 @@ void NBodySolver::run_sym(const SymShape& sh, int blocks, bool fp32, const void*
     a.t0 = t0_;
     a.rt0 = rt0_;
     a.r0 = r0_;
+    a.fine = keep_order_ ? 0 : 1;
     if (sh.keep)
       launch_pair_sym(a, stream_);
     else

@@ -115,6 +115,12 @@ struct SymParticle {
 };
 
 template <class R>
+__device__ inline void add3(Vec3<R>& d, const Vec3<R>& s) {
+  d.x += s.x;
+  d.y += s.y;
+  d.z += s.z;
+}
+template <class R>
 __device__ inline void add_to(Vec3<double>& d, Vec3<R>& s) {
   d.x += s.x;
   d.y += s.y;
@@ -135,6 +141,9 @@ __device__ inline void sym_steps(const SymStage<R, SymForm<BLK>::nrec, NW>& st, 
                                  Vec3<R>& su, Vec3<R>& sw) {
   using Fm = SymForm<BLK>;
   const Vec3<R> zero = {R(0), R(0), R(0)};
+  // FP32, several targets per lane: a step's terms of a source are added up before
+  // they go to its running sum, which so has 64 terms as with one target.
+  constexpr bool kOwn = std::is_same<R, float>::value && TPL > 1 && !DIAG;
   if constexpr (!WALL && BLK == kUF) {
     // the open translational block: overlap test over the step's pairs, and in
     // FP32 the fences of sym_item (nbody_kernels.hip)
@@ -168,10 +177,12 @@ __device__ inline void sym_steps(const SymStage<R, SymForm<BLK>::nrec, NW>& st, 
 #pragma unroll
         for (int t = 0; t < TPL; ++t) rpy_near_select_uf34<R>(r2[t], ir[t], cf[t]);
       }
+      Vec3<R> cu = zero, cw = zero;
 #pragma unroll
       for (int t = 0; t < TPL; ++t)
         open_unit<R, BLK, !DIAG>(dx[t], dy[t], dz[t], cf[t], fg, zero, me[t].f, zero, u[t], w[t],
-                                 su, sw);
+                                 kOwn ? cu : su, kOwn ? cw : sw);
+      if constexpr (kOwn) add3(su, cu);
     }
   } else {
 #pragma unroll 1
@@ -184,12 +195,18 @@ __device__ inline void sym_steps(const SymStage<R, SymForm<BLK>::nrec, NW>& st, 
         rol1(su);
         if (Fm::angular) rol1(sw);
       }
+      Vec3<R> cu = zero, cw = zero;
 #pragma unroll
       for (int t = 0; t < TPL; ++t) {
         PairGeo<R> g;
         pair_distances<R, WALL>(me[t].p.x, me[t].p.y, me[t].p.z, pj.x, pj.y, pj.z, g);
         pair_inverses<R, WALL>(g);
-        pair_unit<R, WALL, BLK, !DIAG>(g, pj.z, fj, tj, me[t].f, me[t].t, u[t], w[t], su, sw);
+        pair_unit<R, WALL, BLK, !DIAG>(g, pj.z, fj, tj, me[t].f, me[t].t, u[t], w[t],
+                                       kOwn ? cu : su, kOwn ? cw : sw);
+      }
+      if constexpr (kOwn) {
+        add3(su, cu);
+        if (Fm::angular) add3(sw, cw);
       }
     }
   }
@@ -252,6 +269,14 @@ __device__ inline void sym_unit_item(const SymItem& it, const SymSys& S, const S
         const int blk = NW == 1 ? 0 : (wave + p) & (NW - 1);
         su = sw = zero;
         sym_steps<R, WALL, BLK, TPL, NW, DIAG>(lds.st, blk * 128 + lane, me, u, w, su, sw);
+        if constexpr (std::is_same<R, float>::value) {
+          // FP32 sums over 64 sources at most
+#pragma unroll
+          for (int t = 0; t < TPL; ++t) {
+            add_to(u64[t], u[t]);
+            if (Fm::angular) add_to(w64[t], w[t]);
+          }
+        }
         if (!DIAG) {
           // lane l holds source l - 1 after 64 steps: one more move
           rol1(su);
@@ -277,13 +302,6 @@ __device__ inline void sym_unit_item(const SymItem& it, const SymSys& S, const S
         const int64_t row = (int64_t)(o - a.obase) * a.n3 + 3 * j;
         put3(a.slab_s + row, us * (double)bj, v[0], v[1], v[2]);
         if (Fm::angular) put3(a.slab_sw + row, ws * (double)bj, v[3], v[4], v[5]);
-      }
-      if constexpr (std::is_same<R, float>::value) {
-#pragma unroll
-        for (int t = 0; t < TPL; ++t) {
-          add_to(u64[t], u[t]);
-          if (Fm::angular) add_to(w64[t], w[t]);
-        }
       }
     }
   }
