@@ -36,7 +36,7 @@ NBodySolver::NBodySolver(int px, int py, int pz) {
 }
 
 NBodySolver::~NBodySolver() {
-  if (pos_host_busy_) (void)hipStreamSynchronize(pos_host_stream_);
+  if (pos_pending_) (void)hipStreamSynchronize(nullptr);
   if (chk_stream_) (void)hipStreamSynchronize(chk_stream_);
   for (auto& e : lz_ev_)
     if (e) (void)hipEventDestroy(e);
@@ -188,7 +188,7 @@ void NBodySolver::setPositions(const double* pos, int64_t n3, bool dev) {
     if (!dev) {
       staged = (size_t)n3 * sizeof(double) <= kStageBytes;
       if (staged) {
-        pos_host_wait();  // kernels of the call before may still read the buffer
+        pos_wait();  // kernels of the call before may still read the buffer
         src = stage_in(kStagePos, pos, n3);
         if (!place) {  // read more than once
           st_pos_.reserve(sizeof(double) * n3);
@@ -260,26 +260,31 @@ void NBodySolver::setPositions(const double* pos, int64_t n3, bool dev) {
     throw Error(
         "[Mobility] Invalid batch parameters for NBody. If in doubt, use the defaults.");
   // The caller's array may change after the return: positions that a transfer
-  // still reads are waited for, those in our own buffer are not.
-  if (staged) {
-    pos_host_stream_ = stream_;
-    pos_host_busy_ = true;
-  } else if (!dev) {
+  // still reads are waited for, those in our own buffer are not.  On the default
+  // stream, which always exists, the records are not waited for either; a change
+  // of the stream does it.
+  if (stream_ == nullptr && (staged || (dev && wall_)))
+    pos_pending_ = true;
+  else if (!dev || wall_)
     LM_HIP(hipStreamSynchronize(stream_));
-  }
 }
 
-void NBodySolver::pos_host_wait() {
-  if (!pos_host_busy_) return;
-  LM_HIP(hipStreamSynchronize(pos_host_stream_));
-  pos_host_busy_ = false;
+void NBodySolver::pos_wait() {
+  if (!pos_pending_) return;
+  // also while another stream (setStream's) is being captured
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  LM_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+  const hipError_t e = hipStreamSynchronize(nullptr);
+  LM_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+  LM_HIP(e);
+  pos_pending_ = false;
 }
 
 // One part of the mapped host buffer for n values, host and device address.  A
 // larger buffer replaces the old one once no kernel reads it.
 double* NBodySolver::stage_out(StagePart part, int64_t n, const double** host) {
   if (n > stage_cap_) {
-    pos_host_wait();
+    pos_wait();
     const int64_t cap = std::max<int64_t>(n, std::min<int64_t>(2 * stage_cap_, kStageBytes / 8));
     stage_cap_ = 0;
     stage_.reserve(sizeof(double) * kStageParts * cap, hipHostMallocMapped | hipHostMallocCoherent);
@@ -297,7 +302,7 @@ const double* NBodySolver::stage_in(StagePart part, const double* x, int64_t n) 
 }
 
 void NBodySolver::setStream(hipStream_t s) {
-  if (s != stream_) pos_host_wait();  // work on the new stream uses the records
+  if (s != stream_) pos_wait();  // work on the new stream uses the records
   stream_ = s;
 }
 

@@ -344,9 +344,8 @@ class NBodySolver {
   int64_t stage_cap_ = 0;  // values per part of stage_
   double* stage_out(StagePart part, int64_t n, const double** host);
   const double* stage_in(StagePart part, const double* x, int64_t n);
-  hipStream_t pos_host_stream_ = nullptr;  // of the kernels that read the positions there
-  bool pos_host_busy_ = false;
-  void pos_host_wait();
+  bool pos_pending_ = false;  // the last positions' kernels, on the default stream
+  void pos_wait();
   std::vector<int64_t> sys_off_dev_;  // what sys_off_ holds
   // Lanczos
   DevBuf V_, w_, coef_, noise_, red_partial_, scalars_, tsq_work_;
