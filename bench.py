@@ -226,17 +226,17 @@ C1_TILING = (1, 16)
 MEASURED_FP32_FLOPS = {
     ("c3", 131072, "symmetric", 4, 64): 7.134e9 * 64,
     ("c3", 131072, "symmetric", 4, 32): 7.00029e9 * 64,
-    ("c2", 65536, "symmetric", 1, 64): 1.25718e10 * 64,
-    ("c4", 816182, "symmetric", 2, 8): 3.19152e9 * 64,
+    ("c2", 65536, "symmetric", 1, 32): 1.0756e10 * 64,
+    ("c4", 816182, "symmetric", 1, 16): 2.719e9 * 64,
 }
 
 MEASURED_TRAFFIC_BYTES = {
     ("c3", 131072, "ordered", 2, 32): (10454.1 * 2.0 + 98304.0) * 1024.0,
     ("c3", 131072, "symmetric", 4, 64): (152410.0 * 2.0 + 394750.0) * 1024.0,
-    ("c3", 131072, "symmetric", 4, 32): (104635.2 * 2.0 + 296448.0) * 1024.0,
+    ("c3", 131072, "symmetric", 4, 32): (106120.0 * 2.0 + 296448.0) * 1024.0,
     ("c3", 131072, "symmetric", 2, 64): (177902.1 * 2.0 + 591360.0) * 1024.0,
-    ("c2", 65536, "symmetric", 1, 64): (130223.0 * 2.0 + 591360.0) * 1024.0,
-    ("c4", 816182, "symmetric", 2, 8): (108844.0 * 2.0 + 165989.0) * 1024.0,
+    ("c2", 65536, "symmetric", 1, 32): (91020.0 * 2.0 + 493060.0) * 1024.0,
+    ("c4", 816182, "symmetric", 1, 16): (124180.0 * 2.0 + 317090.0) * 1024.0,
     ("c1", 1024, "ordered", 1, 16): (173.0 * 2.0 + 384.0) * 1024.0,
 }
 

@@ -100,7 +100,9 @@ int lm_nbody_set_pair_tiling(lm_nbody* h, int targets_per_lane, int source_chunk
  * mobility matrix is symmetric (M_ji = M_ij^T blockwise), so each unordered
  * pair is evaluated once and applied to both particles; the reference
  * evaluates every ordered pair (NbodyRPY.cu:27-97, hydrodynamicKernels.cuh).
- * Auto uses it from N = 16384.  Results agree with the ordered evaluation to
+ * Auto uses it from N = 4096 (single wall), 8192 (open, FP64) or 16384 (open,
+ * FP32, and the products of plain Lanczos over open systems); for ensembles
+ * from 16384 particles in systems of 1500 on average.  Results agree with the ordered evaluation to
  * rounding and are bitwise reproducible. */
 int lm_nbody_set_pair_symmetric(lm_nbody* h, int mode);
 
@@ -116,10 +118,13 @@ int lm_nbody_last_pair_symmetric(lm_nbody* h, int* used);
  * and keeps the fastest for later calls. */
 int lm_nbody_set_autotune(lm_nbody* h, int enable);
 
-/* Extension: tiling used by the last pair-kernel launch. */
+/* Extension: tiling used by the last pair-kernel launch.  Small systems run a
+ * kernel whose lanes hold sources: it reports 4 targets and 1 chunk. */
 int lm_nbody_get_pair_tiling(lm_nbody* h, int* targets_per_lane, int* source_chunks);
 
-/* Extension: order all work of this handle on `stream` (a hipStream_t). */
+/* Extension: order all work of this handle on `stream` (a hipStream_t).  Where
+ * the last set_positions took host arrays on the default stream, this waits for
+ * the kernels that still read them (also while `stream` is being captured). */
 int lm_nbody_set_stream(lm_nbody* h, void* stream);
 
 /* NBody::initialize + Mobility::initialize, mobility.h:99-114 and

@@ -388,8 +388,8 @@ class NBody(_Solver):
 
     def setPairSymmetric(self, mode=-1, memoryBytes=0):
         """Extension: evaluate each unordered pair once for a single open or
-        single-wall system (-1 auto, 0 off, 1 on); memoryBytes bounds its
-        partial sums (0 = 4 GiB; the work is split into passes that fit)."""
+        single-wall system or an ensemble (-1 auto: by size and kind, 0 off,
+        1 on); memoryBytes bounds its partial sums (0 = 4 GiB; the work is split into passes that fit)."""
         _ffi.check(self._lib.lm_nbody_set_pair_symmetric(self._h, int(mode)))
         _ffi.check(self._lib.lm_nbody_set_pair_symmetric_memory(self._h, int(memoryBytes)))
 
