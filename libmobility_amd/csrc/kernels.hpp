@@ -245,7 +245,7 @@ void launch_chunk_reduce(const double* part, int nchunks, int64_t n, double* out
 // `largest`: particles of the largest system.
 void launch_system_bbox(const double* pos, const int64_t* sys_off, int nsys, int64_t largest,
                         double wall_shift, const int* kinds, int wall, double* bbox, hipStream_t s,
-                        double* host = nullptr);
+                        double* host = nullptr, double* own = nullptr);
 // Records for the pair kernels; `shifted` receives the wall-shifted AoS copy.
 void launch_make_records(const double* pos, int64_t N, const int64_t* sys_off, int nsys,
                          const double* bbox, const int* kinds, int wall, double wall_shift,

@@ -1211,12 +1211,15 @@ struct BoxSum {
 // particles.  With 256 threads and one particle in flight 2999 particles took
 // 4.9 us, 65536 74, 131072 142; now 3.9, 22, 39.  host (may be null): a copy of
 // bbox in mapped host memory, where reading it takes no transfer of its own.
+// own (may be null): a copy of the positions, so that a wait for the boxes is
+// also one for the last read of the caller's array.
 template <int NT>
 __global__ __launch_bounds__(NT) void k_system_bbox(const double* __restrict__ pos,
                                                    const int64_t* __restrict__ off,
                                                    double wall_shift_in,
                                                    const int* __restrict__ kinds, int wall,
-                                                   double* __restrict__ bbox, double* host) {
+                                                   double* __restrict__ bbox, double* host,
+                                                   double* __restrict__ own) {
   __shared__ double sh[6][NT / 64];
   const int s = blockIdx.x;
   const int64_t b = off[s], e = off[s + 1];
@@ -1233,6 +1236,12 @@ __global__ __launch_bounds__(NT) void k_system_bbox(const double* __restrict__ p
     }
 #pragma unroll
     for (int q = 0; q < kQ; ++q) box.add(p[q][0], p[q][1], p[q][2] - wall_shift);
+    if (own != nullptr)
+#pragma unroll
+      for (int q = 0; q < kQ; ++q)
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+          if (i0 + q * NT < e) own[3 * (i0 + q * NT) + c] = p[q][c];
   }
   box.reduce(sh);
   if (threadIdx.x < 6) {
@@ -1243,14 +1252,14 @@ __global__ __launch_bounds__(NT) void k_system_bbox(const double* __restrict__ p
 
 void launch_system_bbox(const double* pos, const int64_t* sys_off, int nsys, int64_t largest,
                         double wall_shift, const int* kinds, int wall, double* bbox, hipStream_t s,
-                        double* host) {
+                        double* host, double* own) {
   if (nsys <= 0) return;
   if (largest > 4096)
     hipLaunchKernelGGL(k_system_bbox<1024>, dim3(nsys), dim3(1024), 0, s, pos, sys_off, wall_shift,
-                       kinds, wall, bbox, host);
+                       kinds, wall, bbox, host, own);
   else
     hipLaunchKernelGGL(k_system_bbox<256>, dim3(nsys), dim3(256), 0, s, pos, sys_off, wall_shift,
-                       kinds, wall, bbox, host);
+                       kinds, wall, bbox, host, own);
   LM_HIP(hipGetLastError());
 }
 

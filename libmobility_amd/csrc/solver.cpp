@@ -179,7 +179,12 @@ void NBodySolver::setPositions(const double* pos, int64_t n3, bool dev) {
   }
   bool any_wall = false, any_open = false;
   for (int k : kinds) (k ? any_wall : any_open) = true;
-  bool staged = false;  // the positions are in our pinned buffer
+  // Records are made from our own memory: the positions are in the mapped buffer,
+  // or the kernel of the boxes copies them (the caller's array may change after
+  // the return, on any stream; above this size waiting costs less than the copy).
+  bool staged = false;
+  const bool own = dev && wall_ && any_wall && stream_ == nullptr &&
+                   (size_t)n3 * sizeof(double) <= kStageBytes;
   if (N > 0) {
     const double* src = pos;
     int64_t largest = 0;
@@ -214,8 +219,11 @@ void NBodySolver::setPositions(const double* pos, int64_t n3, bool dev) {
     const double shift = wall_height_;
     if (any_wall) {
       bbox_host_.reserve(sizeof(double) * 6 * nsys, hipHostMallocMapped | hipHostMallocCoherent);
+      if (own) st_pos_.reserve(sizeof(double) * n3);
       launch_system_bbox(src, sys_off_.as<int64_t>(), nsys, largest, shift, kinds_d, wall_ ? 1 : 0,
-                         bbox_.as<double>(), stream_, bbox_host_.device_as<double>());
+                         bbox_.as<double>(), stream_, bbox_host_.device_as<double>(),
+                         own ? st_pos_.as<double>() : nullptr);
+      if (own) src = st_pos_.as<double>();
       LM_HIP(hipStreamSynchronize(stream_));
       const double* bb = bbox_host_.as<double>();
       double minz = 1e300;
@@ -259,11 +267,11 @@ void NBodySolver::setPositions(const double* pos, int64_t n3, bool dev) {
   if (!valid)
     throw Error(
         "[Mobility] Invalid batch parameters for NBody. If in doubt, use the defaults.");
-  // The caller's array may change after the return: positions that a transfer
-  // still reads are waited for, those in our own buffer are not.  On the default
-  // stream, which always exists, the records are not waited for either; a change
-  // of the stream does it.
-  if (stream_ == nullptr && (staged || (dev && wall_)))
+  // The caller's array may change after the return: positions that a transfer or
+  // a kernel still reads are waited for, those in our own memory are not.  On the
+  // default stream, which always exists, the records are not waited for either; a
+  // change of the stream does it.
+  if (stream_ == nullptr && (staged || own))
     pos_pending_ = true;
   else if (!dev || wall_)
     LM_HIP(hipStreamSynchronize(stream_));

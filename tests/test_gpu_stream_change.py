@@ -80,3 +80,25 @@ def test_captured_product_after_host_positions(wall):
         torch.cuda.synchronize()
         ref, _ = oracle.mdot(pos, ETA, A, F=F.cpu().numpy(), wall=wall)
         assert np.linalg.norm(U.cpu().numpy().ravel() - ref) <= 1e-12 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("n", [1, 255, 257, 4097, 16384, 16385])
+def test_positions_overwritten_on_another_stream(n):
+    """Above a wall setPositions has read the caller's tensor when it returns."""
+    import torch
+    s = _solver(True)
+    rng = np.random.default_rng(n)
+    pos = rng.uniform(0, 3.0 * A * n ** (1 / 3), (n, 3))
+    pos[:, 2] += A
+    F = rng.standard_normal((n, 3))
+    ref, _ = oracle.mdot(pos, ETA, A, F=F, wall=True)
+    other = torch.cuda.Stream()
+    for _ in range(3):
+        tensor = torch.as_tensor(pos, device="cuda")
+        torch.cuda.synchronize()
+        s.setPositions(tensor)
+        with torch.cuda.stream(other):
+            tensor.fill_(float("nan"))
+        U, _ = s.Mdot(torch.as_tensor(F, device="cuda"))
+        torch.cuda.synchronize()
+        assert np.linalg.norm(U.cpu().numpy().ravel() - ref) <= 1e-12 * np.linalg.norm(ref)
