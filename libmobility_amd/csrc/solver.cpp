@@ -994,25 +994,20 @@ void NBodySolver::build_active_items(const int* act) {
   seg_items_.count = count;
 }
 
-// Tiling: user override, else the autotuned choice, else the default rule.
-void NBodySolver::choose_tiling(int blocks, bool fp32, const double* F, const double* T,
-                                double* U, double* W, const void* rec, int& tpl, int& nch) {
-  const bool tpl4_ok = kind_code() == 0 && blocks == kUF;
-  if (tile_tpl_ != 0 || tile_nch_ != 0) {
-    tpl = tile_tpl_ != 0 ? tile_tpl_ : 1;
-    if (tpl == 4 && !tpl4_ok) tpl = 2;
-    nch = tile_nch_;
-    return;
-  }
+// Tiling of the ordered kernel without the autotuner, which may choose another one
+// where this returns true: user override, else the algorithm, else the default rule.
+bool NBodySolver::rule_tiling(int blocks, int& tpl, int& nch) const {
   tpl = 1;
   nch = 0;
-  if (algorithm_ == kNaive) {
-    nch = 1;
-    return;
+  if (tile_tpl_ != 0 || tile_nch_ != 0) {
+    tpl = tile_tpl_ != 0 ? tile_tpl_ : 1;
+    if (tpl == 4 && !(kind_code() == 0 && blocks == kUF)) tpl = 2;
+    nch = tile_nch_;
+    return false;
   }
-  if (algorithm_ == kBlock) {
-    nch = 32;
-    return;
+  if (algorithm_ == kNaive || algorithm_ == kBlock) {
+    nch = algorithm_ == kNaive ? 1 : 32;
+    return false;
   }
   // Measured on MI355X: two targets per lane pay off once the system is
   // large enough to keep every CU busy with 512-target tiles.
@@ -1020,6 +1015,14 @@ void NBodySolver::choose_tiling(int blocks, bool fp32, const double* F, const do
   for (size_t s = 0; s + 1 < sys_off_host_.size(); ++s)
     maxn = std::max(maxn, sys_off_host_[s + 1] - sys_off_host_[s]);
   if (maxn >= 16384) tpl = 2;
+  return true;
+}
+
+// The same with the autotuned choice.
+void NBodySolver::choose_tiling(int blocks, bool fp32, const double* F, const double* T,
+                                double* U, double* W, const void* rec, int& tpl, int& nch) {
+  const bool tpl4_ok = kind_code() == 0 && blocks == kUF;
+  if (!rule_tiling(blocks, tpl, nch)) return;
   if (!autotune_) return;
   const int nsys = (int)sys_off_host_.size() - 1;
   const auto key = std::make_tuple(N_, nsys, kind_code() + 4 * (use_persistent() ? 1 : 0),
@@ -1511,10 +1514,11 @@ bool NBodySolver::wide_step_route() {
 // ordered pair kernel over open systems, one target per lane, chunk slabs (which
 // keep w apart from what the launch writes).
 bool NBodySolver::head_route() const {
-  if (kind_code() != 0 || use_persistent() || autotune_ || tile_tpl_ > 1 || algorithm_ == kNaive ||
-      pair_active_ != nullptr || sym_mode_ == 1)
+  if (kind_code() != 0 || use_persistent() || autotune_ || pair_active_ != nullptr || sym_mode_ == 1)
     return false;
-  return resolve_nch(1, algorithm_ == kBlock ? 32 : tile_nch_) > 1;
+  int tpl, nch;
+  rule_tiling(angular_ ? kUF | kUT | kWT | kWF : kUF, tpl, nch);
+  return tpl == 1 && resolve_nch(tpl, nch) > 1;
 }
 
 // w = M v ; torques are stored after the forces (MobilityInterface.h:164-176).

@@ -228,6 +228,7 @@ class NBodySolver {
   void ensure_records();
   void build_systems(int64_t N, std::vector<int64_t>& off, bool& valid) const;
   void ensure_items(int tpl, int nch_hint);
+  bool rule_tiling(int blocks, int& tpl, int& nch) const;
   void choose_tiling(int blocks, bool fp32, const double* F, const double* T, double* U,
                      double* W, const void* rec, int& tpl, int& nch);
   void launch_pair_items(const PairItem* list, int count, int tpl, int nch, int blocks, bool fp32,

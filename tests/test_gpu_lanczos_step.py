@@ -64,3 +64,39 @@ def test_one_recurrence_over_systems_vs_oracle(sizes, precision):
     assert abs(s.lastLanczosIterations() - it) <= 1
     # FP32 pair terms (6e-8 each) add to the tolerance
     assert np.linalg.norm(u.ravel() - ref) <= (2 * TOL if precision == "fp64" else 4 * TOL) * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("angular,N", [(False, 65), (False, 1365), (False, 1366),
+                                       (True, 65), (True, 682), (True, 683)])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("params,tiling", [
+    ({}, (0, 0)), ({"algorithm": "block"}, (0, 0)), ({"algorithm": "block"}, (1, 1)),
+    ({"algorithm": "block"}, (0, 1)), ({"algorithm": "naive"}, (1, 0)), ({}, (1, 1)), ({}, (1, 3))])
+def test_open_step_lengths_vs_oracle(angular, N, precision, params, tiling):
+    """Open systems, where the product finishes the step before it up to 4096
+    entries: not with one source chunk, whichever of the tiling and the
+    algorithm asks for it."""
+    from libmobility_amd import NBody
+    rng = np.random.default_rng(N)
+    eta, a = 1 / (6 * np.pi), 1.0
+    # dilute: the solve converges before orthogonality is lost (as above; a product
+    # perturbed by 1e-7 moves the oracle's own result by 3e-7 at most)
+    pos = rng.uniform(0, 25.0 * N ** (1 / 3), (N, 3))
+    s = NBody("open", "open", "open")
+    s.setParameters(**params)
+    s.setPairPrecision(precision)
+    s.setPairTiling(*tiling)
+    s.initialize(viscosity=eta, hydrodynamicRadius=a, includeAngular=angular, tolerance=TOL)
+    s.setPositions(pos)
+
+    def product(v):
+        F, T = (v[:3 * N], v[3 * N:]) if angular else (v, None)
+        U, W = oracle.mdot(pos, eta, a, F=F, T=T, angular=angular)
+        return np.concatenate([U, W]) if angular else U
+
+    W = rng.normal(size=(6 if angular else 3) * N)
+    u, w = s.sqrtMdotW_with_noise(W)
+    got = np.concatenate([u.ravel(), w.ravel()]) if angular else u.ravel()
+    ref, it = oracle.LanczosOracle().run(product, W, TOL)
+    assert abs(s.lastLanczosIterations() - it) <= 1
+    assert np.linalg.norm(got - ref) <= (2 * TOL if precision == "fp64" else 4 * TOL) * np.linalg.norm(ref)
