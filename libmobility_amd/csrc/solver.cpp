@@ -159,6 +159,7 @@ void NBodySolver::setPositions(const double* pos, int64_t n3, bool dev) {
     throw Error(
         "[libMobility] The input arrays for positions, forces, and torques must each have "
         "total size 3*N.");
+  if (pos == nullptr && n3 > 0) throw Error("[libmobility_amd] setPositions needs a positions array");
   const int64_t N = n3 / 3;
   std::vector<int64_t> off;
   bool valid = true;
@@ -1075,6 +1076,10 @@ void NBodySolver::choose_tiling(int blocks, bool fp32, const double* F, const do
   nch = best_nch;
 }
 
+static void require_linear(const double* U) {
+  if (!U) throw Error("[libmobility_amd] Mdot needs a linear output array");
+}
+
 // U (3N) and, when angular, W (3N) are overwritten (NbodyRPY.cu:91-96).
 void NBodySolver::pair_product(const void* rec64, const void* rec32, const double* F,
                                const double* T, double* U, double* W, int prec) {
@@ -1083,7 +1088,7 @@ void NBodySolver::pair_product(const void* rec64, const void* rec32, const doubl
   if (F) blocks |= kUF | (angular_ ? kWF : 0);
   if (T && angular_) blocks |= kUT | kWT;
   const int64_t n3 = 3 * N_;
-  if (!U) throw Error("[libmobility_amd] Mdot needs a linear output array");
+  require_linear(U);
   if (blocks == 0) {
     launch_zero(U, n3, stream_);
     if (angular_ && W) launch_zero(W, n3, stream_);
@@ -1148,6 +1153,7 @@ void NBodySolver::Mdot(const double* F, int64_t nF, const double* T, int64_t nT,
         "The solver was configured without including angular velocities. Set includeAngular "
         "to true when initializing if you want to use torques");
   require_positions("[Mobility] Positions have 0 particles. Did you call setPositions?");
+  require_linear(U);
   const double* f = nF > 0 ? F : nullptr;
   const double* t = nT > 0 ? T : nullptr;
   if (dev) {
