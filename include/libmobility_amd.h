@@ -123,8 +123,8 @@ int lm_nbody_set_autotune(lm_nbody* h, int enable);
 int lm_nbody_get_pair_tiling(lm_nbody* h, int* targets_per_lane, int* source_chunks);
 
 /* Extension: order all work of this handle on `stream` (a hipStream_t).  Where
- * the last set_positions, from host arrays or above a wall, was on the default
- * stream, this waits for the kernels that still read the solver's copy of them (also while `stream` is being captured). */
+ * the last set_positions was on the default stream, also one that ended with an
+ * error, this waits for its kernels (also while `stream` is being captured). */
 int lm_nbody_set_stream(lm_nbody* h, void* stream);
 
 /* NBody::initialize + Mobility::initialize, mobility.h:99-114 and

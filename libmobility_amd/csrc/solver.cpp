@@ -36,7 +36,10 @@ NBodySolver::NBodySolver(int px, int py, int pz) {
 }
 
 NBodySolver::~NBodySolver() {
-  if (pos_pending_) (void)hipStreamSynchronize(nullptr);
+  try {
+    pos_wait();
+  } catch (const Error&) {  // the buffers go all the same
+  }
   if (chk_stream_) (void)hipStreamSynchronize(chk_stream_);
   for (auto& e : lz_ev_)
     if (e) (void)hipEventDestroy(e);
@@ -196,6 +199,12 @@ void NBodySolver::setPositions(const double* pos, int64_t n3, bool dev) {
       if (staged) {
         pos_wait();  // kernels of the call before may still read the buffer
         src = stage_in(kStagePos, pos, n3);
+      }
+    }
+    // from the first launch on, whatever ends this call
+    pos_pending_ |= stream_ == nullptr;
+    if (!dev) {
+      if (staged) {
         if (!place) {  // read more than once
           st_pos_.reserve(sizeof(double) * n3);
           launch_copy2(src, st_pos_.as<double>(), nullptr, nullptr, n3, stream_);
@@ -265,17 +274,15 @@ void NBodySolver::setPositions(const double* pos, int64_t n3, bool dev) {
     ++struct_id_;
     items_tpl_ = -1;
   }
-  if (!valid)
-    throw Error(
-        "[Mobility] Invalid batch parameters for NBody. If in doubt, use the defaults.");
   // The caller's array may change after the return: positions that a transfer or
   // a kernel still reads are waited for, those in our own memory are not.  On the
   // default stream, which always exists, the records are not waited for either; a
   // change of the stream does it.
-  if (stream_ == nullptr && (staged || own))
-    pos_pending_ = true;
-  else if (!dev || wall_)
+  if ((!dev || wall_) && !(stream_ == nullptr && (staged || own)))
     LM_HIP(hipStreamSynchronize(stream_));
+  if (!valid)
+    throw Error(
+        "[Mobility] Invalid batch parameters for NBody. If in doubt, use the defaults.");
 }
 
 void NBodySolver::pos_wait() {

@@ -345,7 +345,7 @@ class NBodySolver {
   int64_t stage_cap_ = 0;  // values per part of stage_
   double* stage_out(StagePart part, int64_t n, const double** host);
   const double* stage_in(StagePart part, const double* x, int64_t n);
-  bool pos_pending_ = false;  // the last positions' kernels, on the default stream
+  bool pos_pending_ = false;  // kernels of setPositions on the default stream since pos_wait
   void pos_wait();
   std::vector<int64_t> sys_off_dev_;  // what sys_off_ holds
   // Lanczos

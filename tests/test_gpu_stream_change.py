@@ -102,3 +102,46 @@ def test_positions_overwritten_on_another_stream(n):
         U, _ = s.Mdot(torch.as_tensor(F, device="cuda"))
         torch.cuda.synchronize()
         assert np.linalg.norm(U.cpu().numpy().ravel() - ref) <= 1e-12 * np.linalg.norm(ref)
+
+
+def _occupy_default_stream():
+    """Some tens of milliseconds of work queued on the default stream."""
+    import torch
+    x = torch.full((8192, 8192), 1e-4, dtype=torch.float64, device="cuda")
+    torch.cuda.synchronize()
+    for _ in range(3):
+        x = x @ x
+    return x
+
+
+@pytest.mark.parametrize("wall", [False, True])
+@pytest.mark.parametrize("host", [True, False])
+@pytest.mark.parametrize("valid", [True, False])
+def test_product_on_another_stream_behind_other_work(wall, host, valid):
+    """The records of a busy default stream: a product on another stream has those
+    of the last positions, also where setPositions refused the batch parameters
+    (which leaves one system of all particles)."""
+    import torch
+    from libmobility_amd import NBody
+    s = NBody("open", "open", "single_wall" if wall else "open")
+    s.setParameters(**({"wallHeight": 0.0} if wall else {}))
+    s.initialize(viscosity=ETA, hydrodynamicRadius=A)
+    F = torch.randn((N, 3), dtype=torch.float64, device="cuda")
+    s.setPositions(_positions(0))
+    if not valid:
+        s.setParameters(Nbatch=2, NperBatch=N, **({"wallHeight": 0.0} if wall else {}))
+    # several streams: some may share the default stream's hardware queue
+    for step, other in enumerate([torch.cuda.Stream() for _ in range(4)], 1):
+        s.Mdot(F)  # back on the default stream, where host arrays then stay
+        pos = _positions(step)
+        given = pos if host else torch.as_tensor(pos, device="cuda")
+        _occupy_default_stream()
+        if valid:
+            s.setPositions(given)
+        else:
+            with pytest.raises(RuntimeError, match="Invalid batch parameters"):
+                s.setPositions(given)
+        with torch.cuda.stream(other):
+            U, _ = s.Mdot(F)
+        ref, _ = oracle.mdot(pos, ETA, A, F=F.cpu().numpy(), wall=wall)
+        assert np.linalg.norm(U.cpu().numpy().ravel() - ref) <= 1e-12 * np.linalg.norm(ref)
