@@ -223,7 +223,7 @@ void NBodySolver::setPositions(const double* pos, int64_t n3, bool dev) {
       sys_off_.reserve(sizeof(int64_t) * off.size());
       LM_HIP(hipMemcpyAsync(sys_off_.as<int64_t>(), off.data(), sizeof(int64_t) * off.size(),
                             hipMemcpyHostToDevice, stream_));
-      sys_off_dev_ = off;
+      if (!capturing()) sys_off_dev_ = off;
     }
     bbox_.reserve(sizeof(double) * 6 * nsys);
     const double shift = wall_height_;
@@ -315,6 +315,21 @@ const double* NBodySolver::stage_in(StagePart part, const double* x, int64_t n) 
   double* dev = stage_out(part, n, &host);
   std::copy(x, x + n, const_cast<double*>(host));
   return dev;
+}
+
+// Whether the stream is being captured: what is launched then has not run when the
+// call returns, and what a kernel or a copy prepares for later calls is not there.
+bool NBodySolver::capturing() const {
+  if (stream_ == nullptr) return false;  // cannot be captured
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  LM_HIP(hipStreamIsCapturing(stream_, &st));
+  return st != hipStreamCaptureStatusNone;
+}
+
+void NBodySolver::refuse_capture() const {
+  if (capturing())
+    throw Error("[libmobility_amd] this call cannot be captured: run it once before, or use "
+                "lm_nbody_mdot_noalloc");
 }
 
 void NBodySolver::setStream(hipStream_t s) {
@@ -512,6 +527,8 @@ void NBodySolver::ensure_sym_plan(const SymShape& sh, bool ang) {
   if (plan.N == N_ && plan.structure == struct_id_ && plan.tpl == tpl && plan.waves == sh.waves &&
       plan.nchunks == nch && plan.per == sh.per[0] && plan.ang == (ang ? 1 : 0) && plan.budget == sym_budget_)
     return;
+  refuse_capture();
+  plan.N = -1;
   const int nsys = (int)sys_off_host_.size() - 1;
   const int64_t bt = 64 * (int64_t)sh.waves * tpl;
   std::vector<SymSys> systems(nsys);
@@ -1236,6 +1253,7 @@ void NBodySolver::setLanczosIterationLimit(int limit) {
 }
 
 int NBodySolver::lanczos_run(const double* z, double** result) {
+  refuse_capture();
   const int64_t n = (angular_ ? 6 : 3) * N_;
   ensure_records();
   // The checks run on a second stream, overlapped with the next iterations:

@@ -347,6 +347,8 @@ class NBodySolver {
   const double* stage_in(StagePart part, const double* x, int64_t n);
   bool pos_pending_ = false;  // kernels of setPositions on the default stream since pos_wait
   void pos_wait();
+  bool capturing() const;
+  void refuse_capture() const;
   std::vector<int64_t> sys_off_dev_;  // what sys_off_ holds
   // Lanczos
   DevBuf V_, w_, coef_, noise_, red_partial_, scalars_, tsq_work_;
