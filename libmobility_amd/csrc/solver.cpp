@@ -824,6 +824,13 @@ bool NBodySolver::use_wide() {
          persistent_mode_ == -1 && mean_system_size() <= kWideMaxSize;
 }
 
+// Whether the autotuner, if it is on, has found that kernel to be the fastest.
+bool NBodySolver::tuned_wide(int blocks, bool fp32) const {
+  if (!autotune_) return true;
+  const auto it = tuned_.find(tune_key(blocks, fp32));
+  return it != tuned_.end() && it->second.first == 0;
+}
+
 // Units of kWideTargets targets of one system.  Equal systems of one kind need
 // no list; else the systems with the most work per unit come first.
 void NBodySolver::ensure_wide_plan() {
@@ -1043,15 +1050,23 @@ bool NBodySolver::rule_tiling(int blocks, int& tpl, int& nch) const {
   return true;
 }
 
-// The same with the autotuned choice.
+// What the autotuner keeps its choices by: the products that keep their order run
+// other kernels than the rest.
+NBodySolver::TuneKey NBodySolver::tune_key(int blocks, bool fp32) const {
+  const int nsys = (int)sys_off_host_.size() - 1;
+  return {N_, nsys, kind_code() + 4 * (use_persistent() ? 1 : 0) + 8 * (keep_order_ ? 1 : 0),
+          fp32 ? 1 : 0, blocks};
+}
+
+// The same with the autotuned choice; `wide`: sources across the lanes is a
+// candidate too, and tpl 0 means that it is the fastest.
 void NBodySolver::choose_tiling(int blocks, bool fp32, const double* F, const double* T,
-                                double* U, double* W, const void* rec, int& tpl, int& nch) {
+                                double* U, double* W, const void* rec, bool wide, int& tpl,
+                                int& nch) {
   const bool tpl4_ok = kind_code() == 0 && blocks == kUF;
   if (!rule_tiling(blocks, tpl, nch)) return;
   if (!autotune_) return;
-  const int nsys = (int)sys_off_host_.size() - 1;
-  const auto key = std::make_tuple(N_, nsys, kind_code() + 4 * (use_persistent() ? 1 : 0),
-                                   fp32 ? 1 : 0, blocks);
+  const TuneKey key = tune_key(blocks, fp32);
   auto it = tuned_.find(key);
   if (it != tuned_.end()) {
     tpl = it->second.first;
@@ -1067,34 +1082,40 @@ void NBodySolver::choose_tiling(int blocks, bool fp32, const double* F, const do
   int best_tpl = tpl, best_nch = 0;
   const int tpls[3] = {1, 2, 4};
   const int nchs[6] = {0, 1, 2, 4, 8, 16};
+  auto time_one = [&](auto&& product) {
+    // per-launch time of `reps` back-to-back launches after one untimed
+    auto time_reps = [&](int reps) {
+      product();
+      LM_HIP(hipEventRecord(e0, stream_));
+      for (int r = 0; r < reps; ++r) product();
+      LM_HIP(hipEventRecord(e1, stream_));
+      LM_HIP(hipEventSynchronize(e1));
+      float t = 0.f;
+      LM_HIP(hipEventElapsedTime(&t, e0, e1));
+      return t / reps;
+    };
+    float ms = time_reps(2);
+    // short products: two launches are within the clock's noise
+    if (ms < 0.1f) ms = time_reps(16);
+    if (ms >= best) return false;
+    best = ms;
+    return true;
+  };
   for (int ti = 0; ti < 3; ++ti) {
     if (tpls[ti] == 4 && !tpl4_ok) continue;
     for (int ci = 0; ci < 6; ++ci) {
       ensure_items(tpls[ti], nchs[ci]);
       if (nchs[ci] != 0 && items_nch_ != nchs[ci]) continue;  // clamped duplicate
-      // per-launch time of `reps` back-to-back launches after one untimed
-      auto time_reps = [&](int reps) {
-        launch_main_items(blocks, fp32, rec, F, T, U, W);
-        LM_HIP(hipEventRecord(e0, stream_));
-        for (int r = 0; r < reps; ++r) launch_main_items(blocks, fp32, rec, F, T, U, W);
-        LM_HIP(hipEventRecord(e1, stream_));
-        LM_HIP(hipEventSynchronize(e1));
-        float t = 0.f;
-        LM_HIP(hipEventElapsedTime(&t, e0, e1));
-        return t / reps;
-      };
-      float ms = time_reps(2);
-      // short products: two launches are within the clock's noise
-      if (ms < 0.1f) ms = time_reps(16);
-      if (ms < best) {
-        best = ms;
+      if (time_one([&] { launch_main_items(blocks, fp32, rec, F, T, U, W); })) {
         best_tpl = items_tpl_;
         best_nch = items_nch_;
       }
     }
   }
+  if (wide && time_one([&] { launch_wide(blocks, fp32, rec, F, T, U, W); })) best_tpl = best_nch = 0;
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
+  deferred_nch_ = 0;  // of a candidate
   tuned_[key] = {best_tpl, best_nch};
   tpl = best_tpl;
   nch = best_nch;
@@ -1129,19 +1150,26 @@ void NBodySolver::pair_product(const void* rec64, const void* rec32, const doubl
   if (use_sym(blocks, fp32)) {
     launch_sym(blocks, fp32, rec, F, T, U, W);
     last_sym_ = true;
-  } else if (use_wide()) {
-    launch_wide(blocks, fp32, rec, F, T, U, W);
-    last_wide_ = true;
-  } else if (seg_items_.count > 0) {
-    // per-system Lanczos after some systems converged: their work is dropped
-    launch_pair_items(seg_items_.buf.as<PairItem>(), seg_items_.count, seg_items_.tpl,
-                      seg_items_.nch, blocks, fp32, rec, F, T, U, W);
   } else {
-    int tpl = 1, nch = 0;
-    choose_tiling(blocks, fp32, F, T, U, W, rec, tpl, nch);
-    ensure_items(tpl, nch);
-    if (items_count_ <= 0) throw Error("[libmobility_amd] empty pair work list");
-    launch_main_items(blocks, fp32, rec, F, T, U, W);
+    int tpl = 0, nch = 0;  // tpl 0: sources across the lanes
+    const bool wide = use_wide();
+    // per-system Lanczos after some systems converged: their work is dropped
+    const bool seg = seg_items_.count > 0;
+    if (seg)
+      tpl = wide && tuned_wide(blocks, fp32) ? 0 : 1;
+    else if (!wide || autotune_)
+      choose_tiling(blocks, fp32, F, T, U, W, rec, wide, tpl, nch);
+    if (tpl == 0) {
+      launch_wide(blocks, fp32, rec, F, T, U, W);
+      last_wide_ = true;
+    } else if (seg) {
+      launch_pair_items(seg_items_.buf.as<PairItem>(), seg_items_.count, seg_items_.tpl,
+                        seg_items_.nch, blocks, fp32, rec, F, T, U, W);
+    } else {
+      ensure_items(tpl, nch);
+      if (items_count_ <= 0) throw Error("[libmobility_amd] empty pair work list");
+      launch_main_items(blocks, fp32, rec, F, T, U, W);
+    }
   }
   if (angular_ && W && !ang) launch_zero(W, n3, stream_);
 }
@@ -1534,7 +1562,8 @@ bool NBodySolver::wide_step_route() {
   static_assert(kWideStepMax == kLanczosFusedMaxN, "the vectors of the fused steps");
   if (pre_on() || kind_code() != 1 || pair_active_ != nullptr) return false;
   const bool fp32 = pair_prec_ == kPairFP32;
-  if (use_sym(angular_ ? kUF | kUT | kWT | kWF : kUF, fp32) || !use_wide()) return false;
+  const int blocks = angular_ ? kUF | kUT | kWT | kWF : kUF;
+  if (use_sym(blocks, fp32) || !use_wide() || !tuned_wide(blocks, fp32)) return false;
   last_sym_ = false;
   last_wide_ = true;
   deferred_nch_ = 0;

@@ -230,7 +230,7 @@ class NBodySolver {
   void ensure_items(int tpl, int nch_hint);
   bool rule_tiling(int blocks, int& tpl, int& nch) const;
   void choose_tiling(int blocks, bool fp32, const double* F, const double* T, double* U,
-                     double* W, const void* rec, int& tpl, int& nch);
+                     double* W, const void* rec, bool wide, int& tpl, int& nch);
   void launch_pair_items(const PairItem* list, int count, int tpl, int nch, int blocks, bool fp32,
                          const void* rec, const double* F, const double* T, double* U, double* W);
   void launch_main_items(int blocks, bool fp32, const void* rec, const double* F, const double* T,
@@ -332,7 +332,9 @@ class NBodySolver {
   WideArgs wide_args(int blocks, bool fp32, const void* rec);
   int tile_tpl_ = 0, tile_nch_ = 0;  // user override (0 = auto)
   bool autotune_ = false;
-  std::map<std::tuple<int64_t, int, int, int, int>, std::pair<int, int>> tuned_;
+  using TuneKey = std::tuple<int64_t, int, int, int, int>;
+  TuneKey tune_key(int blocks, bool fp32) const;
+  std::map<TuneKey, std::pair<int, int>> tuned_;  // targets per lane (0: launch_wide), chunks
   // staging for host arrays
   DevBuf st_pos_, st_f_, st_t_, st_u_, st_w_;
   // Host arrays of up to kStageBytes go through mapped host memory, which kernels
@@ -443,6 +445,7 @@ class NBodySolver {
   uint64_t mean_size_struct_ = 0;
   int64_t mean_size_N_ = -1;
   bool use_wide();
+  bool tuned_wide(int blocks, bool fp32) const;
   // Products of a plain Lanczos recurrence over open systems: the summation
   // order stays that of k_pair's chunks (k_pair_sym from kSymKeepN).  There the
   // largest Ritz values converge to rounding within about 15 iterations, the
