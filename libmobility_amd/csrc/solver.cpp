@@ -753,7 +753,9 @@ void NBodySolver::run_sym(const SymShape& sh, int blocks, bool fp32, const void*
 void NBodySolver::launch_sym(int blocks, bool fp32, const void* rec, const double* F,
                              const double* T, double* U, double* W) {
   const int nsys = (int)sys_off_host_.size() - 1;
-  const auto key = std::make_tuple(N_, fp32 ? 1 : 0, kind_code() + 4 * nsys, blocks);
+  // products that keep their order run other kernels, in other shapes
+  const auto key = std::make_tuple(N_, fp32 ? 1 : 0,
+                                   kind_code() + 4 * (keep_order_ ? 1 : 0) + 8 * nsys, blocks);
   double pairs = 0.0;
   for (int s = 0; s < nsys; ++s) {
     const double n = (double)(sys_off_host_[s + 1] - sys_off_host_[s]);

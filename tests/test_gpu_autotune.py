@@ -98,3 +98,40 @@ def test_square_root_with_the_autotuner(wall, angular, sizes, per_system):
         # two square roots that stop near a relative 1e-4 (their estimate is no bound)
         assert np.linalg.norm(y - ref) <= 2e-3 * np.linalg.norm(ref)
         s.Mdot(F, T if angular else None)
+
+
+@pytest.mark.parametrize("root_first", [True, False])
+def test_symmetric_choices_of_roots_and_products_are_apart(root_first):
+    """Plain Lanczos products over open systems run other symmetric kernels than Mdot
+    at the same size: each is timed at its own first use."""
+    import torch
+    N = 17000
+    pos, F, _ = _inputs(N)
+    dpos, dF = (torch.as_tensor(x, device="cuda") for x in (pos, F))
+    z = torch.as_tensor(np.random.default_rng(1).normal(size=3 * N), device="cuda")
+
+    def make():
+        s = _solver(False, False, "fp64", True)
+        s.setPositions(dpos)
+        return s
+
+    def product(s):
+        return s.Mdot(dF)
+
+    def root(s):
+        return s.sqrtMdotW_with_noise(z)
+
+    first, then = (root, product) if root_first else (product, root)
+    s = make()  # kernels loaded, both tuned
+    for call in (product, root, product, root):
+        call(s)
+    again = min(_first(then, [s]) for _ in range(5))
+    new = [make() for _ in range(3)]
+    for t in new:
+        first(t)
+    # ten candidates and more, three products each: thirty products besides
+    one = min(_first(product, [s]) for _ in range(5))
+    assert _first(then, new) > again + 10 * one
+    U, _ = product(new[0])
+    Uo, _ = product(s)
+    assert float((U - Uo).norm()) <= 1e-12 * float(Uo.norm())
