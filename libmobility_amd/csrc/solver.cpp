@@ -549,24 +549,39 @@ void NBodySolver::ensure_sym_plan(const SymShape& sh, bool ang) {
   const double unit = 8.0 * 3.0 * (double)N_ * (ang ? 2.0 : 1.0);  // bytes per slab (U and W)
   const double per_offset = 1.0 + (h > 0 ? (double)nch / h : 0.0);
   const int span = std::max(1, (int)(((double)sym_budget_ / unit - 2.0) / per_offset));
+  // Target slabs of a pass over `width` offsets from oa: the items of the longest ring
+  // of either kind (they may differ in length, in mixed ensembles).
+  const int64_t room = (int64_t)((double)sym_budget_ / unit);
+  int ring[2] = {0, 0};
+  for (const SymSys& S : systems) ring[S.wall ? 1 : 0] = std::max(ring[S.wall ? 1 : 0], S.hmax);
+  auto target_slabs = [&](int oa, int width) {
+    int c = 0;
+    for (int k = 0; k < 2; ++k) {
+      const int ws = std::min(width, ring[k] + 1 - oa);
+      if (ws > 0) c = std::max(c, (ws + sh.per[k] - 1) / sh.per[k]);
+    }
+    return c;
+  };
   std::vector<SymItem> items;
   size_t nitems = 0;
   plan.passes.clear();
   plan.max_slabs = 0;
   int oa = 1;
   do {
-    const int ob = std::min(h + 1, oa + span);
     const bool first = oa == 1;
-    const int width = ob - oa;
+    int width = std::min(h + 1, oa + span) - oa;
+    if (sh.per[0] > 0) {
+      // one offset less takes one or two slabs away
+      for (int64_t over; width > 1 && (over = width + target_slabs(oa, width) + first - room) > 0;)
+        width -= (int)std::min<int64_t>(width - 1, (over + 1) / 2);
+    }
+    const int ob = oa + width;
     SymPass ps;
     ps.item0 = (int)nitems;
     ps.oa = oa;
     ps.ob = ob;
     ps.nch = width > 0 ? std::max(1, std::min(width, (int)(((int64_t)nch * width + h - 1) / h))) : 0;
-    if (sh.per[0] > 0) {
-      const int least = std::min(sh.per[0], sh.per[1]);
-      ps.nch = (width + least - 1) / least;
-    }
+    if (sh.per[0] > 0) ps.nch = target_slabs(oa, width);
     ps.diag = first ? 1 : 0;
     // This system's offsets in the pass and its items per tile.
     auto widths = [&](const SymSys& S, int& ws, int& cs) {

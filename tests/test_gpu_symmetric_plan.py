@@ -70,3 +70,39 @@ def test_ensembles_vs_oracle(sizes, kinds, angular, precision):
         assert np.linalg.norm(U.ravel() - Uo) <= TOL[precision] * np.linalg.norm(Uo)
         if angular:
             assert np.linalg.norm(W.ravel() - Wo) <= TOL[precision] * np.linalg.norm(Wo)
+
+
+@pytest.mark.parametrize("slabs", [70, 20])
+@pytest.mark.parametrize("angular", [False, True])
+def test_partial_sums_of_a_mixed_ensemble_fit_their_memory(slabs, angular):
+    """Open systems have the longest rings and the longest items, the walls' items
+    are shorter: the memory limit holds for what both need."""
+    import torch
+    from libmobility_amd import NBody
+    sizes, walls = [6000] * 11 + [1000] * 8, [False] * 11 + [True] * 8
+    parts = [_cloud(n, w, 7 + k) for k, (n, w) in enumerate(zip(sizes, walls))]
+    pos, F, T = (torch.as_tensor(np.concatenate([p[k] for p in parts]), device="cuda") for k in range(3))
+    if not angular:
+        T = None
+    N = sum(sizes)
+    limit = slabs * 24 * N * (2 if angular else 1)
+    results = []
+    for memory in (limit, 0):
+        s = NBody("open", "open", "single_wall")
+        s.setParameters(wallHeight=0.0)
+        s.setPairSymmetric(1, memoryBytes=memory)
+        s.initialize(viscosity=ETA, hydrodynamicRadius=A, includeAngular=angular)
+        s.setSystems(sizes, ["single_wall" if w else "open" for w in walls])
+        s.setPositions(pos)
+        torch.cuda.synchronize()
+        out = [torch.empty_like(pos) for _ in range(3)]  # the allocator has what Mdot returns
+        del out
+        free = torch.cuda.mem_get_info()[0]
+        results.append(s.Mdot(F, T))
+        taken = free - torch.cuda.mem_get_info()[0]
+        if memory:
+            # besides: 20 bytes per item, at most some 10^5 of them, and page granularity
+            assert taken <= limit + (8 << 20)
+    for got, ref in zip(*results):
+        if ref is not None:
+            assert float((got - ref).norm()) <= 1e-12 * float(ref.norm())
