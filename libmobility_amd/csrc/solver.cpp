@@ -124,8 +124,8 @@ void NBodySolver::require_positions(const char* msg) const {
 
 void NBodySolver::build_systems(int64_t N, std::vector<int64_t>& off, bool& valid) const {
   off.clear();
-  if (explicit_systems_ && !sys_off_host_.empty() && sys_off_host_.back() == N) {
-    off = sys_off_host_;
+  if (explicit_systems_ && (N > 0 || explicit_off_.back() == 0)) {
+    off = explicit_off_;
     valid = true;
     return;
   }
@@ -145,7 +145,7 @@ void NBodySolver::setSystems(const int64_t* offsets, int nsys, const int* kinds)
   if (offsets[0] != 0) throw Error("[libmobility_amd] system offsets must start at 0");
   for (int s = 0; s < nsys; ++s)
     if (offsets[s + 1] < offsets[s]) throw Error("[libmobility_amd] system offsets must be non-decreasing");
-  sys_off_host_.assign(offsets, offsets + nsys + 1);
+  explicit_off_.assign(offsets, offsets + nsys + 1);
   explicit_kinds_.clear();
   if (kinds) {
     for (int s = 0; s < nsys; ++s)
@@ -153,8 +153,9 @@ void NBodySolver::setSystems(const int64_t* offsets, int nsys, const int* kinds)
     explicit_kinds_.assign(kinds, kinds + nsys);
   }
   explicit_systems_ = true;
-  ++struct_id_;
-  items_tpl_ = -1;
+  // Kinds, records and boxes are those of the current positions: until the next ones
+  // the systems are, too.
+  if (N_ <= 0) sys_off_host_ = explicit_off_;
 }
 
 void NBodySolver::setPositions(const double* pos, int64_t n3, bool dev) {
@@ -262,13 +263,13 @@ void NBodySolver::setPositions(const double* pos, int64_t n3, bool dev) {
   // Work lists depend on N, the system offsets and kinds only: a new
   // configuration of the same systems (every step of a time loop) keeps them.
   const bool same_structure =
-      N == N_ && kinds == sys_kind_host_ && (explicit_systems_ || off == sys_off_host_);
+      N == N_ && kinds == sys_kind_host_ && off == sys_off_host_;
   N_ = N;
   sys_kind_host_ = kinds;
   kinds_dev_valid_ = kinds_d != nullptr;
   any_wall_ = any_wall;
   any_open_ = any_open;
-  if (!explicit_systems_) sys_off_host_ = off;
+  sys_off_host_ = off;
   ++layout_id_;
   if (!same_structure) {
     ++struct_id_;

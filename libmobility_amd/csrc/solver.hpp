@@ -294,6 +294,7 @@ class NBodySolver {
   int64_t N_ = 0;
   std::vector<int64_t> sys_off_host_;
   std::vector<int> sys_kind_host_;  // per system of the current layout
+  std::vector<int64_t> explicit_off_;  // setSystems, for the next positions
   std::vector<int> explicit_kinds_;
   bool explicit_systems_ = false;
   bool any_wall_ = false, any_open_ = true, kinds_dev_valid_ = false;
