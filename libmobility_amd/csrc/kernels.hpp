@@ -68,6 +68,8 @@ struct SymSys;
 // Small systems (wide_kernels.hip): kWideTargets targets per unit of work, a
 // wave (split 1) or a workgroup (split 4) per unit, sources across the lanes.
 constexpr int kWideTargets = 4;
+// Sources of a wave whose terms a lane adds in FP32: 256 per lane, as in k_pair's tiles.
+constexpr int64_t kWideFp32Sources = 256 * 64;
 struct WideItem {
   int32_t sys;
   int32_t tgt;  // first target within the system
@@ -92,6 +94,7 @@ struct WideArgs {
   const int* active;  // per-system flags; units of systems with 0 are skipped (nullptr: all)
   const int* stop;    // as PairArgs::stop
   double t0, rt0, r0;
+  int long_sums;  // FP32, split 1: sums to FP64 every kWideFp32Sources sources
 };
 void launch_pair_wide(const WideArgs& a, hipStream_t s);
 

@@ -825,9 +825,11 @@ void NBodySolver::launch_sym(int blocks, bool fp32, const void* rec, const doubl
 double NBodySolver::mean_system_size() {
   if (mean_size_struct_ != struct_id_ || mean_size_N_ != N_) {
     double s2 = 0.0;
+    largest_size_ = 0;
     for (size_t s = 0; s + 1 < sys_off_host_.size(); ++s) {
-      const double n = (double)(sys_off_host_[s + 1] - sys_off_host_[s]);
-      s2 += n * n;
+      const int64_t ns = sys_off_host_[s + 1] - sys_off_host_[s];
+      s2 += (double)ns * (double)ns;
+      largest_size_ = std::max(largest_size_, ns);
     }
     mean_size_ = N_ > 0 ? s2 / (double)N_ : 0.0;
     mean_size_struct_ = struct_id_;
@@ -903,6 +905,7 @@ WideArgs NBodySolver::wide_args(int blocks, bool fp32, const void* rec) {
   a.fp32 = fp32 ? 1 : 0;
   a.blocks = blocks;
   a.split = wide_.nunits >= kWideWaveUnits && mean_system_size() <= kWideWaveMean ? 1 : 4;
+  if (fp32 && largest_size_ > kWideFp32Sources * a.split) a.split = a.long_sums = 1;
   a.pos = rec;
   a.items = wide_.listed ? wide_.items.as<WideItem>() : nullptr;
   a.sys = wide_.listed ? wide_.sys.as<SymSys>() : nullptr;

@@ -443,6 +443,7 @@ class NBodySolver {
   // size of the system that the average particle is in, of the current structure
   double mean_system_size();
   double mean_size_ = 0.0;
+  int64_t largest_size_ = 0;  // of the same structure
   uint64_t mean_size_struct_ = 0;
   int64_t mean_size_N_ = -1;
   bool use_wide();

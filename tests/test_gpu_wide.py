@@ -113,3 +113,40 @@ def test_infinite_and_nan_forces_stay_with_their_system():
     U, _ = s.Mdot(F)
     assert np.isfinite(U[:70]).all()
     assert not np.isfinite(U[70:140]).any() and np.isnan(U[140:]).all()
+
+
+@pytest.mark.parametrize("wall", [False, True])
+def test_fp32_sums_of_a_large_system_among_small_ones(wall):
+    """A system of 60000 in an ensemble whose mean size selects one wave per four
+    targets: a lane's 938 terms are not one FP32 sum.  The worst case of such a sum
+    is equal terms: one target, and all other particles at one place."""
+    import torch
+    from libmobility_amd import NBody
+    big, small, count = 60000, 64, 39700
+    sizes = [big] + [small] * count
+    N = sum(sizes)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(1)
+    pos = torch.rand((N, 3), generator=g, device="cuda", dtype=torch.float64) * 40.0 + 1.0
+    pos[:big] = torch.tensor([128.0, 0.0, 64.0], dtype=torch.float64)
+    pos[0] = torch.tensor([0.0, 0.0, 64.0], dtype=torch.float64)
+    got = {}
+    for precision in ("fp64", "fp32"):
+        s = NBody("open", "open", "single_wall" if wall else "open")
+        s.setParameters(**({"wallHeight": 0.0} if wall else {}))
+        s.setPairPrecision(precision)
+        s.initialize(viscosity=1 / (6 * np.pi), hydrodynamicRadius=1.0)
+        s.setSystems(sizes)
+        s.setPositions(pos)
+        u = []
+        for f in np.geomspace(1.0, 2.0, 24, endpoint=False):
+            F = torch.zeros((N, 3), dtype=torch.float64, device="cuda")
+            F[1:big, 1] = float(f)
+            u.append(float(s.Mdot(F)[0][0, 1]))
+            assert s.lastPairTiling() == (4, 1)
+        got[precision] = np.array(u)
+    error = np.abs(got["fp32"] / got["fp64"] - 1).max()
+    # 256 equal terms: each addition rounds by half an ulp of the sum so far, at most
+    # 2^-24 (1 + 2 + ... + 256) / 256 of the sum; the terms themselves some 1e-6 (a
+    # dozen roundings of 6e-8, with the wall's differences of open and image terms)
+    assert error <= 129 * 2.0 ** -24 + 1.5e-6
