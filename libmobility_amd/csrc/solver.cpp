@@ -529,6 +529,7 @@ void NBodySolver::ensure_sym_plan(const SymShape& sh, bool ang) {
       plan.nchunks == nch && plan.per == sh.per[0] && plan.ang == (ang ? 1 : 0) && plan.budget == sym_budget_)
     return;
   refuse_capture();
+  if (!plan.host_items.empty()) LM_HIP(hipStreamSynchronize(stream_));
   plan.N = -1;
   const int nsys = (int)sys_off_host_.size() - 1;
   const int64_t bt = 64 * (int64_t)sh.waves * tpl;
@@ -563,7 +564,11 @@ void NBodySolver::ensure_sym_plan(const SymShape& sh, bool ang) {
     }
     return c;
   };
-  std::vector<SymItem> items;
+  struct Group {
+    int weight, s, len, i0, i1;  // ring items of `len` offsets (0: diagonal) of tiles [i0, i1)
+  };
+  std::vector<Group> groups;
+  std::vector<SymItem> items, ring_items;
   size_t nitems = 0;
   plan.passes.clear();
   plan.max_slabs = 0;
@@ -597,34 +602,53 @@ void NBodySolver::ensure_sym_plan(const SymShape& sh, bool ang) {
     }
     nitems += count;
     ps.nitems = (int)count;
-    // An ensemble's items go longest first: a counting sort by weight in eighths
-    // of an open offset, two walks over the items, the first to count.
-    auto walk = [&](auto&& put) {
+    // An ensemble's items go longest first.  A system's items of one weight (eighths of
+    // an open offset) form a group: its ring items of either length, its full diagonal
+    // tiles, the last of them.  The few groups are sorted instead of the items, and
+    // the uploads are not waited for (first product of 96 systems, 19424 items: 759 to
+    // 863 -> 697 to 712 us).
+    if (nsys > 1) {
+      groups.clear();
       for (int s = 0; s < nsys; ++s) {
         const SymSys& S = systems[s];
         const int wgt = S.wall ? 40 : 8;
+        int ws, cs, len[2] = {0, 0};
+        widths(S, ws, cs);
+        for (int c = 0; c < cs; ++c) {
+          const SymItem it = sym_ring_item(S, s, 0, c, cs, oa, ws);
+          const int n = it.o1 - it.o0;
+          len[len[0] != 0 && n != len[0] ? 1 : 0] = n;
+        }
+        for (const int n : len)
+          if (n > 0) groups.push_back({wgt * n, s, n, 0, S.ntiles});
+        if (first && S.ntiles > 0) {
+          const int64_t n = S.n - (int64_t)(S.ntiles - 1) * bt;
+          if (S.ntiles > 1) groups.push_back({wgt / 2, s, 0, 0, S.ntiles - 1});
+          groups.push_back({(int)(wgt * n * n / (2 * bt * bt)), s, 0, S.ntiles - 1, S.ntiles});
+        }
+      }
+      std::stable_sort(groups.begin(), groups.end(),
+                       [](const Group& x, const Group& y) { return x.weight > y.weight; });
+      items.reserve(nitems);
+      for (const Group& g : groups) {
+        const SymSys& S = systems[g.s];
+        if (g.len == 0) {
+          for (int I = g.i0; I < g.i1; ++I) items.push_back(SymItem{g.s, I, 0, 0, ps.nch});
+          continue;
+        }
         int ws, cs;
         widths(S, ws, cs);
-        for (int I = 0; I < S.ntiles; ++I)
-          for (int c = 0; c < cs; ++c) {
-            const SymItem it = sym_ring_item(S, s, I, c, cs, oa, ws);
-            put(wgt * (it.o1 - it.o0), it);
-          }
-        if (first)
-          for (int I = 0; I < S.ntiles; ++I) {
-            const int64_t n = std::min<int64_t>(bt, S.n - (int64_t)I * bt);
-            put((int)(wgt * n * n / (2 * bt * bt)), SymItem{s, I, 0, 0, ps.nch});
+        ring_items.clear();
+        for (int c = 0; c < cs; ++c) {
+          const SymItem it = sym_ring_item(S, g.s, 0, c, cs, oa, ws);
+          if (it.o1 - it.o0 == g.len) ring_items.push_back(it);
+        }
+        for (int I = g.i0; I < g.i1; ++I)
+          for (SymItem it : ring_items) {
+            it.tile = I;
+            items.push_back(it);
           }
       }
-    };
-    if (nsys > 1) {
-      items.resize(nitems);
-      SymItem* out = items.data() + ps.item0;
-      const int top = 40 * std::max(1, width);
-      std::vector<int> bins((size_t)top + 2, 0);
-      walk([&](int w, const SymItem&) { ++bins[top - w + 1]; });
-      for (size_t k = 1; k < bins.size(); ++k) bins[k] += bins[k - 1];
-      walk([&](int w, const SymItem& it) { out[bins[top - w]++] = it; });
     }
     plan.max_slabs = std::max(plan.max_slabs, (size_t)(ps.nch + ps.diag + width));
     plan.passes.push_back(ps);
@@ -641,7 +665,6 @@ void NBodySolver::ensure_sym_plan(const SymShape& sh, bool ang) {
                           hipMemcpyHostToDevice, stream_));
     LM_HIP(hipMemcpyAsync(plan.rows.as<void>(), rows.data(), sizeof(SymRows) * rows.size(),
                           hipMemcpyHostToDevice, stream_));
-    LM_HIP(hipStreamSynchronize(stream_));  // the host vectors go out of scope (items are kept)
   } else {
     // one system: a kernel writes what its formula gives (the upload of some
     // thousand items took 0.13 ms of a first product)
@@ -650,7 +673,9 @@ void NBodySolver::ensure_sym_plan(const SymShape& sh, bool ang) {
                        ps.nch, ps.diag, plan.sys.as<SymSys>(), plan.rows.as<SymRows>(), nrows,
                        stream_);
   }
-  plan.host_items = std::move(items);
+  plan.host_items = std::move(items);  // the copies may still read them
+  plan.host_sys = std::move(systems);
+  plan.host_rows = std::move(rows);
   plan.N = N_;
   plan.structure = struct_id_;
   plan.tpl = tpl;

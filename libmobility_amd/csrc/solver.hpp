@@ -399,6 +399,8 @@ class NBodySolver {
   struct SymPlan {
     DevBuf items, sys, rows, active_items;
     std::vector<SymItem> host_items;  // all passes, in launch order
+    std::vector<SymSys> host_sys;
+    std::vector<SymRows> host_rows;
     int tpl = 0, waves = 0, nchunks = 0, per = 0, hmax = 0, nitems = 0, nrows = 0, ang = -1;
     int64_t N = -1, budget = 0;
     uint64_t structure = 0;

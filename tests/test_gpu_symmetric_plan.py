@@ -106,3 +106,27 @@ def test_partial_sums_of_a_mixed_ensemble_fit_their_memory(slabs, angular):
     for got, ref in zip(*results):
         if ref is not None:
             assert float((got - ref).norm()) <= 1e-12 * float(ref.norm())
+
+
+@pytest.mark.parametrize("tiling", [(0, 0), (1, 0), (1, 3), (2, 0), (2, 5), (0, 7)])
+@pytest.mark.parametrize("slabs", [0, 9])
+@pytest.mark.parametrize("kinds", ["open", "mixed"])
+def test_work_lists_of_ensembles(tiling, slabs, kinds):
+    """Rings whose items have two lengths, shared evenly or with a rest, in one pass
+    and in several: every pair is met once."""
+    from libmobility_amd import NBody
+    sizes = (1500, 64, 0, 1, 2111, 700, 129)
+    walls = [kinds == "mixed" and k % 2 == 0 for k in range(len(sizes))]
+    parts = [_cloud(n, w, 7 + k) for k, (n, w) in enumerate(zip(sizes, walls))]
+    pos, F, _ = (np.concatenate([p[k] for p in parts]) for k in range(3))
+    s = NBody("open", "open", "single_wall")
+    s.setParameters(wallHeight=0.0)
+    s.setPairSymmetric(1, memoryBytes=slabs * 24 * sum(sizes))
+    s.setPairTiling(*tiling)
+    s.initialize(viscosity=ETA, hydrodynamicRadius=A)
+    s.setSystems(sizes, ["single_wall" if w else "open" for w in walls])
+    s.setPositions(pos)
+    U, _ = s.Mdot(F)
+    assert s.lastPairSymmetric()
+    Uo, _ = oracle.mdot(pos, ETA, A, F=F, wall=walls, sys_sizes=sizes)
+    assert np.linalg.norm(U.ravel() - Uo) <= TOL["fp64"] * np.linalg.norm(Uo)
