@@ -636,7 +636,7 @@ __global__ __launch_bounds__(kPairThreads) void k_pair_sym(SymArgs a) {
   const SymSys S = a.sys[it.sys];
   if constexpr (KIND == 2) {
     if (S.wall != 0) {
-      sym_unit<R, true, BLK, TPL, 4>(it, S, a, *reinterpret_cast<Unit*>(s_mem));
+      sym_unit<R, true, BLK, TPL, 4, true>(it, S, a, *reinterpret_cast<Unit*>(s_mem));
       return;
     }
   }

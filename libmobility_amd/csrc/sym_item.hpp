@@ -134,11 +134,12 @@ __device__ inline void put3(double* o, double s, double x, double y, double z) {
 }
 
 // The step loop of one wave: its lanes' targets against block `b0` (+ lane) of
-// the staged sources; DIAG: all ordered pairs, the targets' sums only.
+// the staged sources; DIAG: all ordered pairs, the targets' sums only, which with
+// the same b0 in all lanes may end after the block's `cnt` sources.
 template <class R, bool WALL, int BLK, int TPL, int NW, bool DIAG>
 __device__ inline void sym_steps(const SymStage<R, SymForm<BLK>::nrec, NW>& st, int b0,
                                  const SymParticle<R, WALL, BLK>* me, Vec3<R>* u, Vec3<R>* w,
-                                 Vec3<R>& su, Vec3<R>& sw) {
+                                 Vec3<R>& su, Vec3<R>& sw, int cnt = 64) {
   using Fm = SymForm<BLK>;
   const Vec3<R> zero = {R(0), R(0), R(0)};
   // FP32, several targets per lane: a step's terms of a source are added up before
@@ -149,7 +150,7 @@ __device__ inline void sym_steps(const SymStage<R, SymForm<BLK>::nrec, NW>& st, 
     // FP32 the fences of sym_item (nbody_kernels.hip)
     constexpr bool kFence = std::is_same<R, float>::value;
 #pragma unroll 2
-    for (int k = 0; k < 64; ++k) {
+    for (int k = 0; k < cnt; ++k) {
       R dx[TPL], dy[TPL], dz[TPL], r2[TPL], ir[TPL];
       RpyCoef<R> cf[TPL];
       NearTest<R> near;
@@ -186,7 +187,7 @@ __device__ inline void sym_steps(const SymStage<R, SymForm<BLK>::nrec, NW>& st, 
     }
   } else {
 #pragma unroll 1
-    for (int k = 0; k < 64; ++k) {
+    for (int k = 0; k < cnt; ++k) {
       const Vec3<R> pj = st.get(0, b0 + k);
       Vec3<R> fj = zero, tj = zero;
       if (Fm::needF) fj = st.get(Fm::recF, b0 + k);
@@ -213,8 +214,9 @@ __device__ inline void sym_steps(const SymStage<R, SymForm<BLK>::nrec, NW>& st, 
 }
 
 // Targets of tile it.tile against the partner offsets [it.o0, it.o1), or (DIAG)
-// against themselves.
-template <class R, bool WALL, int BLK, int TPL, int NW, bool DIAG>
+// against themselves (SHORT: source by source, all lanes at the same one, up to the
+// last; a step of the others reads lane + k and takes whole blocks).
+template <class R, bool WALL, int BLK, int TPL, int NW, bool DIAG, bool SHORT = false>
 __device__ inline void sym_unit_item(const SymItem& it, const SymSys& S, const SymArgs& a,
                                      SymLds<R, BLK, NW>& lds) {
   using Fm = SymForm<BLK>;
@@ -268,7 +270,12 @@ __device__ inline void sym_unit_item(const SymItem& it, const SymSys& S, const S
       for (int p = 0; p < NW; ++p) {
         const int blk = NW == 1 ? 0 : (wave + p) & (NW - 1);
         su = sw = zero;
-        sym_steps<R, WALL, BLK, TPL, NW, DIAG>(lds.st, blk * 128 + lane, me, u, w, su, sw);
+        // of a tile that the system does not fill: blocks without sources and waves
+        // without targets give zeros (uniform per wave)
+        if (NW == 1 || (base + 64 * blk < N && tgt0 + 64 * wave < N))
+          sym_steps<R, WALL, BLK, TPL, NW, DIAG>(
+              lds.st, blk * 128 + (SHORT ? 0 : lane), me, u, w, su, sw,
+              SHORT ? (int)min((int64_t)64, N - base - 64 * blk) : 64);
         if constexpr (std::is_same<R, float>::value) {
           // FP32 sums over 64 sources at most
 #pragma unroll
@@ -324,11 +331,11 @@ __device__ inline void sym_unit_item(const SymItem& it, const SymSys& S, const S
   }
 }
 
-template <class R, bool WALL, int BLK, int TPL, int NW>
+template <class R, bool WALL, int BLK, int TPL, int NW, bool SHORT = false>
 __device__ inline void sym_unit(const SymItem& it, const SymSys& S, const SymArgs& a,
                                 SymLds<R, BLK, NW>& lds) {
   if (it.o0 == 0)
-    sym_unit_item<R, WALL, BLK, TPL, NW, true>(it, S, a, lds);
+    sym_unit_item<R, WALL, BLK, TPL, NW, true, SHORT>(it, S, a, lds);
   else
     sym_unit_item<R, WALL, BLK, TPL, NW, false>(it, S, a, lds);
 }

@@ -130,3 +130,41 @@ def test_work_lists_of_ensembles(tiling, slabs, kinds):
     assert s.lastPairSymmetric()
     Uo, _ = oracle.mdot(pos, ETA, A, F=F, wall=walls, sys_sizes=sizes)
     assert np.linalg.norm(U.ravel() - Uo) <= TOL["fp64"] * np.linalg.norm(Uo)
+
+
+@pytest.mark.parametrize("angular", [False, True])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("per_system", [False, True])
+def test_order_keeping_products_of_mixed_ensembles(angular, precision, per_system):
+    """Square roots over open and wall systems around the tiles of 256 and their
+    blocks of 64, applied twice, against the product."""
+    from libmobility_amd import NBody
+    sizes = (1, 63, 64, 65, 100, 0, 128, 129, 255, 256, 257, 330, 513)
+    walls = [k % 2 == 0 for k in range(len(sizes))]
+    parts = [_cloud(n, w, 7 + k) for k, (n, w) in enumerate(zip(sizes, walls))]
+    pos, F, T = (np.concatenate([p[k] for p in parts]) for k in range(3))
+    pos *= 3.0  # dilute: few iterations
+    s = NBody("open", "open", "single_wall")
+    s.setParameters(wallHeight=0.0)
+    s.setPairPrecision(precision)
+    s.setPairSymmetric(1)
+    s.initialize(viscosity=ETA, hydrodynamicRadius=A, includeAngular=angular, tolerance=1e-6)
+    s.setSystems(sizes, ["single_wall" if w else "open" for w in walls])
+    s.setLanczosPerSystem(per_system)
+    s.setPositions(pos)
+
+    def root(x):
+        out = s.sqrtMdotW_with_noise(x)
+        assert s.lastPairSymmetric()
+        return np.concatenate([v.ravel() for v in out if v is not None])
+
+    z = np.concatenate([F.ravel(), T.ravel()]) if angular else F.ravel()
+    got = root(root(z))
+    ref = np.concatenate([v for v in oracle.mdot(pos, ETA, A, F=F, T=T if angular else None,
+                                                 angular=angular, wall=walls, sys_sizes=sizes)
+                          if v is not None])
+    off = np.concatenate([[0], np.cumsum(sizes)])
+    for a, b in zip(off, off[1:]):
+        g, r = (x.reshape(-1, len(pos), 3)[:, a:b] for x in (got, ref))
+        # two roots that end some 1e-6 from theirs; a block left out is far off in its system
+        assert np.linalg.norm(g - r) <= 1e-4 * max(np.linalg.norm(r), 1e-300)
