@@ -250,7 +250,7 @@ __global__ __launch_bounds__(kPairThreads) void k_pair(
 // wave and its sum sits back in lane (source index).  The four waves' sums are
 // added in a fixed order and written once per source to the offset's slab.
 
-template <class R, int TPL>
+template <class R, int TPL, bool FENCE>
 __device__ inline void sym_item(const SymItem& it, const SymArgs& a, typename Rec<R>::T* s_pos,
                                 typename Rec<R>::T* s_f, R* s_red) {
   using R4 = typename Rec<R>::T;
@@ -263,7 +263,9 @@ __device__ inline void sym_item(const SymItem& it, const SymArgs& a, typename Re
   // hardly more than one.  FP64 has no such pairing and keeps groups of 4 pairs.
   //   131072 particles, 4 targets per lane 5.94 -> 5.55 ms, 2 per lane 6.25 ->
   //   5.75 ms; 32768, 2 per lane 449 -> 414 us; 20011, 1 per lane 195 -> 186 us.
-  constexpr bool kFence = std::is_same<R, float>::value;
+  // Not where a CU has one or two workgroups (FENCE false, kFenceItems): little issues
+  // beside a wave then, and it waits for the latencies of one step instead of four.
+  constexpr bool kFence = FENCE && std::is_same<R, float>::value;
   constexpr int SG = kFence || TPL >= 4 ? 1 : 4 / TPL;  // steps per overlap test
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const R4* __restrict__ pos = static_cast<const R4*>(a.pos);
@@ -615,7 +617,7 @@ struct SymKeepLds {
 // One item per workgroup: a diagonal tile (all ordered pairs of tile I, the
 // self pairs included) or a range of partner offsets.  KIND: 0 open, 2 per
 // system (mixed ensembles; their wall systems run in symmetric units).
-template <class R, int KIND, int BLK, int TPL>
+template <class R, int KIND, int BLK, int TPL, bool FENCE>
 __global__ __launch_bounds__(kPairThreads) void k_pair_sym(SymArgs a) {
   using R4 = typename Rec<R>::T;
   using Keep = SymKeepLds<R, BLK>;
@@ -656,7 +658,7 @@ __global__ __launch_bounds__(kPairThreads) void k_pair_sym(SymArgs a) {
     return;
   }
   if constexpr (BLK == kUF)
-    sym_item<R, TPL>(it, a, lds.pos, lds.f, lds.red);
+    sym_item<R, TPL, FENCE>(it, a, lds.pos, lds.f, lds.red);
   else
     sym_item_gen<R, BLK, TPL>(it, a, lds.pos, lds.f, lds.t, lds.red);
 }
@@ -1022,15 +1024,27 @@ void launch_pair(const PairArgs& a, hipStream_t s) {
     launch_pair_kind<double>(a, s);
 }
 
+// Items up to which the open translational kernel runs without fences, one target
+// per lane: at most two workgroups per CU.  Ensembles of open systems, FP32, product
+// in us with / without: 204 items 54.6 / 45.5, 280 items 57.9 / 47.2, 400 items 61.5 /
+// 60.1, 640 and 768 items equal, 1280 items 90.4 / 94.1, 3200 items 151 / 160.
+constexpr int kFenceItems = 512;
+
 template <class R, int KIND, int BLK>
 static void launch_pair_sym_tpl(const SymArgs& a, hipStream_t s) {
   const dim3 grid((unsigned)a.nitems), block(kPairThreads);
+  constexpr bool fence = std::is_same<R, float>::value && BLK == kUF;
   switch (a.tpl) {
-    case 1: hipLaunchKernelGGL((k_pair_sym<R, KIND, BLK, 1>), grid, block, 0, s, a); break;
-    case 2: hipLaunchKernelGGL((k_pair_sym<R, KIND, BLK, 2>), grid, block, 0, s, a); break;
+    case 1:
+      if (fence && a.nitems > kFenceItems)
+        hipLaunchKernelGGL((k_pair_sym<R, KIND, BLK, 1, fence>), grid, block, 0, s, a);
+      else
+        hipLaunchKernelGGL((k_pair_sym<R, KIND, BLK, 1, false>), grid, block, 0, s, a);
+      break;
+    case 2: hipLaunchKernelGGL((k_pair_sym<R, KIND, BLK, 2, fence>), grid, block, 0, s, a); break;
     case 4:
       if constexpr (KIND == 0 && BLK == kUF) {
-        hipLaunchKernelGGL((k_pair_sym<R, KIND, BLK, 4>), grid, block, 0, s, a);
+        hipLaunchKernelGGL((k_pair_sym<R, KIND, BLK, 4, fence>), grid, block, 0, s, a);
         break;
       }
       [[fallthrough]];

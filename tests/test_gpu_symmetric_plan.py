@@ -168,3 +168,27 @@ def test_order_keeping_products_of_mixed_ensembles(angular, precision, per_syste
         g, r = (x.reshape(-1, len(pos), 3)[:, a:b] for x in (got, ref))
         # two roots that end some 1e-6 from theirs; a block left out is far off in its system
         assert np.linalg.norm(g - r) <= 1e-4 * max(np.linalg.norm(r), 1e-300)
+
+
+@pytest.mark.parametrize("sizes", [(300,) * 70, (300,) * 130, (2111,) * 8, (2111,) * 20])
+def test_open_fp32_ensembles_with_few_and_many_items(sizes):
+    """Up to two workgroups per CU the open translational kernel runs without its
+    scheduling fences: 280 and 520 items, some 400 and 1000."""
+    from libmobility_amd import NBody
+    parts = [_cloud(n, False, 7 + k) for k, n in enumerate(sizes)]
+    pos, F = (np.concatenate([p[k] for p in parts]) for k in range(2))
+    results = {}
+    for precision in ("fp64", "fp32"):
+        s = NBody("open", "open", "open")
+        s.setParameters()
+        s.setPairPrecision(precision)
+        s.setPairSymmetric(1)
+        s.initialize(viscosity=ETA, hydrodynamicRadius=A)
+        s.setSystems(sizes)
+        s.setPositions(pos)
+        results[precision], _ = s.Mdot(F)
+        assert s.lastPairSymmetric()
+    Uo, _ = oracle.mdot(pos[:sizes[0]], ETA, A, F=F[:sizes[0]], wall=False)
+    assert np.linalg.norm(results["fp64"][:sizes[0]].ravel() - Uo) <= TOL["fp64"] * np.linalg.norm(Uo)
+    error = np.linalg.norm(results["fp32"] - results["fp64"])
+    assert error <= TOL["fp32"] * np.linalg.norm(results["fp64"])
