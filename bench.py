@@ -217,9 +217,6 @@ def result_line(metric, value, unit, steps, warmup, ms, higher, dtype, config, r
 # C3 tiling of the bench line and its profiles: 4 targets per lane, 32
 # offset chunks
 C3_TILING = (4, 32)
-# C1 tiling (the autotuner's usual pick there), pinned so that profiles of
-# the same command run the same kernels: 1 target per lane, 16 source chunks
-C1_TILING = (1, 16)
 
 # FP32 VALU flops issued per launch, SQ_INSTS_VALU_FLOPS_FP32 x 64 lanes from
 # rocprofv3 --pmc, same keys as MEASURED_TRAFFIC_BYTES.
@@ -238,6 +235,7 @@ MEASURED_TRAFFIC_BYTES = {
     ("c2", 65536, "symmetric", 1, 32): (91020.0 * 2.0 + 493060.0) * 1024.0,
     ("c4", 816182, "symmetric", 1, 16): (124180.0 * 2.0 + 317090.0) * 1024.0,
     ("c1", 1024, "ordered", 1, 16): (173.0 * 2.0 + 384.0) * 1024.0,
+    ("c1", 1024, "wide", 4, 1): (273.0 * 2.0 + 24.0) * 1024.0,
 }
 
 
@@ -621,15 +619,17 @@ def bench_c1(args):
     N = args.N or 1024
     pos, F, Wn = workloads.config_c1(N)
     pos_d, F_d, W_d, U_d = g.put(pos), g.put(F), g.put(Wn), g.zeros(3 * N)
-    h = g.solver(pos_d, "fp64", tiling=args.tiling or C1_TILING)
+    # the library's own rule, so that profiles of the same command run the same
+    # kernels: sources across the lanes for the product, chunks in the recurrence
+    h = g.solver(pos_d, "fp64", tiling=args.tiling, autotune=False)
     ms_mdot = g.time_events(lambda: g.mdot(h, F_d, None, U_d), args.steps, args.warmup)
+    tiling = g.tiling(h)
     U = U_d.cpu().numpy()
     ms_sqrt, its = g.time_lanczos(h, W_d, 3 * N, args.lanczos_calls)
     Uq = g.zeros(3 * N)
     g.sqrt_noise(h, W_d, Uq)
     g.sync()
     sq = Uq.cpu().numpy()
-    tiling = g.tiling(h)
     g.destroy(h)
     pairs = float(N) ** 2
     fpp = flops_per_pair()["open_UF"]
@@ -657,7 +657,8 @@ def bench_c1(args):
                        args.steps, args.warmup, total, False, "f64", config,
                        compute_roofline(pairs * fpp, ms_mdot, PEAK_FP64_TFLOPS,
                                         MEASURED_TRAFFIC_BYTES.get(
-                                            ("c1", N, "ordered", tiling["targets_per_lane"],
+                                            ("c1", N, "ordered" if args.tiling else "wide",
+                                             tiling["targets_per_lane"],
                                              tiling["source_chunks"]))), extra, cpu)
 
 
