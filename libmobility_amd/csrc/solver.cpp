@@ -1622,6 +1622,11 @@ bool NBodySolver::wide_step_route() {
 bool NBodySolver::head_route() const {
   if (kind_code() != 0 || use_persistent() || autotune_ || pair_active_ != nullptr || sym_mode_ == 1)
     return false;
+  // With torques from some 400 particles: below, a workgroup's 256 targets leave the
+  // step in every one of a few workgroups, microseconds per solve with / without: 100
+  // particles FP64 477 / 450, FP32 457 / 428, 200 510 / 485, 300 564 / 549, 400 620 /
+  // 629, 682 685 / 715.
+  if (angular_ && N_ < kHeadTorquesN) return false;
   int tpl, nch;
   rule_tiling(angular_ ? kUF | kUT | kWT | kWF : kUF, tpl, nch);
   return tpl == 1 && resolve_nch(tpl, nch) > 1;

@@ -327,6 +327,7 @@ class NBodySolver {
   // Lanczos step that the next product finishes first (n = 0: none)
   LanczosHead pair_head_{};
   bool head_route() const;
+  static constexpr int64_t kHeadTorquesN = 400;
   DevBuf wide_a_, wide_b_, wide_e1_;  // partial sums and e1 of launch_wide_step
   int64_t wide_e1_n_ = 0;
   bool wide_step_route();

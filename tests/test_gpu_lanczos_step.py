@@ -100,3 +100,10 @@ def test_open_step_lengths_vs_oracle(angular, N, precision, params, tiling):
     ref, it = oracle.LanczosOracle().run(product, W, TOL)
     assert abs(s.lastLanczosIterations() - it) <= 1
     assert np.linalg.norm(got - ref) <= (2 * TOL if precision == "fp64" else 4 * TOL) * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("N", [399, 400])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_open_steps_with_torques_vs_oracle(N, precision):
+    """With torques the product finishes the step before it from 400 particles."""
+    test_open_step_lengths_vs_oracle(True, N, precision, {}, (0, 0))
