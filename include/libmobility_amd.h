@@ -114,8 +114,10 @@ int lm_nbody_set_pair_symmetric_memory(lm_nbody* h, int64_t bytes);
 int lm_nbody_last_pair_symmetric(lm_nbody* h, int* used);
 
 /* Extension: when enabled, the first product for a new (N, systems, kernel,
- * precision, blocks) combination times every tiling candidate on the device
- * and keeps the fastest for later calls. */
+ * precision, blocks) combination times every tiling candidate on the device,
+ * and where the default is the kernel of small systems that one too, and keeps
+ * the fastest for later calls.  Products of plain Lanczos over open systems,
+ * which keep their order of operations, are timed on their own. */
 int lm_nbody_set_autotune(lm_nbody* h, int enable);
 
 /* Extension: tiling used by the last pair-kernel launch.  Small systems run a

@@ -458,6 +458,9 @@ NBodySolver::SymShape NBodySolver::sym_shape(int blocks, bool fp32, int tpl_req,
             (fp32 && kind_code() == 0 && blocks == kUF) || (open_uf && tpl_req == 4);
   if (sh.keep) {
     sh.tpl = tpl_req != 0 ? tpl_req : (open_uf && N_ >= 65536 ? 2 : 1);
+    // FP32 products, us with 1 / 2 / 4: 28000 334 / 340 / 424, 32768 434 / 435 / 584,
+    // 40000 637 / 623 / 757, 65536 1634 / 1511 / 1578, 80000 2488 / 2303 / 2290, 98304
+    // 3922 / 3653 / 3563, 131072 6908 / 6418 / 5986.
     if (!keep_order_ && tpl_req == 0 && open_uf) sh.tpl = N_ >= 98304 ? 4 : (N_ >= 32768 ? 2 : 1);
     if (!open_uf) sh.tpl = std::min(sh.tpl, 2);  // 4 only for one open system
   } else {
@@ -482,7 +485,8 @@ NBodySolver::SymShape NBodySolver::sym_shape(int blocks, bool fp32, int tpl_req,
   // 48), so that there are about 16384 items: 8192 where they are single waves
   // of one system and 4096 with two or four targets per lane, whose target
   // slabs would cost more than the shorter tail gives (131072 particles, four
-  // targets: 5.66 ms with 32 chunks, 5.77 with 64).  A wall pair weighs three
+  // targets: 5.66 ms with 32 chunks, 5.77 with 64).  Rounding to whole offsets
+  // moves that (10007 particles, FP64, one offset per item: 12403).  A wall pair weighs three
   // open ones; in a ragged ensemble (96 systems up to 8192, FP32) items of up
   // to 32 offsets, 0.4 ms for one wave, made it 486 us instead of 455.
   double work = 0.0;

@@ -134,8 +134,9 @@ class NBodySolver {
   // slower at any size (FP32 wall 6x6 at 65536 8641 / 9648: registers).
   static constexpr double kSymWaveN = 16384, kSymTwoN = 32768;
   // Mean system size up to which the ordered evaluation puts sources across
-  // the lanes (wide_kernels.hip has both sides' times; equal from about 8000, and
-  // above only open angular FP32 products get there).
+  // the lanes (wide_kernels.hip has both sides' times).  Only open FP32 products
+  // get above 8192, where k_pair is as fast (6x6) or up to 6 % faster (UF from
+  // 12000: 105 / 109 us, 14000 132 / 140, 16300 167 / 175) with three times the error.
   static constexpr double kWideMaxSize = 16384;
   // Units of work from which each is one wave instead of a workgroup of four
   // (which then only adds the waves' sums and a barrier): 20000 particles in
